@@ -212,7 +212,6 @@ void launch_convert_flat(hipStream_t s, float *out, const double *in, size_t n);
 void launch_begin32(hipStream_t s, float *f32, float *e32, const double *f, const Grid &g);
 void launch_axpbypcz(hipStream_t s, double *out, double a, const double *x, double b, const double *y, double c,
                      const double *z, const Grid &g);
-void launch_relax_block(hipStream_t s, const BottomArgs &a, double omega, int sweeps, int homog);
 
 // Fourth-order finite-volume operator (mgp_fourth.hip), homogeneous Neumann sides.
 // out = rhs - L4 phi (or L4 phi if rhs is null) over the valid cells; nx, ny >= 5.

@@ -18,16 +18,42 @@ namespace mgp {
 // ===========================================================================
 // Ghost fills (arrayutils.f90:871-1492)
 // ===========================================================================
-__device__ void neum_x_ghost(Fld f, const Grid &g, const Geo &geo, const Bc &bc, int homog, int side, int j) {
-    const bool lo = side == XLO;
+// One side's BC.  Picked by comparison, not by an index into the sides' arrays:
+// a run-time index would put the BCs in scratch memory.
+struct SideBc {
+    int type, mode;
+    double val;
+    const double *data;
+};
+__device__ __forceinline__ SideBc x_side(const Bc &b, bool lo) {
+    return SideBc{lo ? b.type[XLO] : b.type[XHI], lo ? b.mode[XLO] : b.mode[XHI], lo ? b.val[XLO] : b.val[XHI],
+                  lo ? b.data[XLO] : b.data[XHI]};
+}
+__device__ __forceinline__ SideBc y_side(const Bc &b, bool lo) {
+    return SideBc{lo ? b.type[YLO] : b.type[YHI], lo ? b.mode[YLO] : b.mode[YHI], lo ? b.val[YLO] : b.val[YHI],
+                  lo ? b.data[YLO] : b.data[YHI]};
+}
+__device__ __forceinline__ double bcval(const SideBc &bc, int k) {
+    return bc.mode == MODE_NONUNIFORM ? bc.data[k] : bc.val;
+}
+
+// Dirichlet order 3 (arrayutils.f90:1160-1177, :1237-1254) or LAH (negate).
+__device__ __forceinline__ double diri_ghost(const SideBc &bc, int homog, double p0, double p1, double p2, int k) {
+    if (bc.mode == MODE_LAH) return -p0;
+    const double sixteenfifth = 16.0 / 5.0, fifth = 1.0 / 5.0;
+    if (homog) return -3.0 * p0 + p1 - fifth * p2;
+    return sixteenfifth * bcval(bc, k) - 3.0 * p0 + p1 - fifth * p2;
+}
+
+__device__ __forceinline__ void neum_x_ghost(Fld f, const Grid &g, const Geo &geo, const SideBc &bc, int homog, bool lo, int j) {
     const int e = lo ? -1 : 1, i = lo ? 0 : g.nx - 1, ny = g.ny;
     const double half = 0.5, threehalves = 1.5;
     const double dx = lo ? -g.dx : g.dx, dy = g.dy;
-    if (bc.mode[side] == MODE_LAH) {
+    if (bc.mode == MODE_LAH) {
         f(i + e, j) = f(i, j);
         return;
     }
-    const int nu = bc.mode[side] == MODE_NONUNIFORM;
+    const int nu = bc.mode == MODE_NONUNIFORM;
     const int P = g.pitch;
     const double Jxy = geo.Jxy[ix(P, i, j)], Jxx = geo.Jxx[ix(P, i, j)];
     // homogeneous: "(-cross)" is evaluated as (-0.0 - cross), identical for every cross
@@ -35,7 +61,7 @@ __device__ void neum_x_ghost(Fld f, const Grid &g, const Geo &geo, const Bc &bc,
     const bool end_hi = j == ny - 1;
     double gv;
     if (homog) gv = -0.0;
-    else gv = bcval(bc, side, nu ? j : 0);
+    else gv = bcval(bc, nu ? j : 0);
     double cross;
     if (end_lo) {
         const double dpn = -(3.0 * f(i, j) - 4.0 * f(i, j + 1) + f(i, j + 2)) * half / dy;
@@ -53,21 +79,20 @@ __device__ void neum_x_ghost(Fld f, const Grid &g, const Geo &geo, const Bc &bc,
     f(i + e, j) = f(i, j) - (gv - cross) * dx / Jxx;
 }
 
-__device__ void neum_y_ghost(Fld f, const Grid &g, const Geo &geo, const Bc &bc, int homog, int side, int i) {
-    const bool lo = side == YLO;
+__device__ __forceinline__ void neum_y_ghost(Fld f, const Grid &g, const Geo &geo, const SideBc &bc, int homog, bool lo, int i) {
     const int e = lo ? -1 : 1, j = lo ? 0 : g.ny - 1, nx = g.nx;
     const double half = 0.5, threehalves = 1.5;
     const double dy = lo ? -g.dy : g.dy, dx = g.dx;
-    if (bc.mode[side] == MODE_LAH) {
+    if (bc.mode == MODE_LAH) {
         f(i, j + e) = f(i, j);
         return;
     }
-    const int nu = bc.mode[side] == MODE_NONUNIFORM;
+    const int nu = bc.mode == MODE_NONUNIFORM;
     const int P = g.pitch;
     const double Jyx = geo.Jyx[ix(P, i, j)], Jyy = geo.Jyy[ix(P, i, j)];
     double gv;
     if (homog) gv = -0.0;
-    else gv = bcval(bc, side, nu ? i : 0);
+    else gv = bcval(bc, nu ? i : 0);
     double cross;
     // the y-side loops cover ilo..ihi in every branch, so only the ihi end
     // keeps its one-sided stencil (arrayutils.f90:1002-1012, 1022-1032, 1042-1052)
@@ -85,10 +110,9 @@ __device__ void neum_y_ghost(Fld f, const Grid &g, const Geo &geo, const Bc &bc,
 
 // x sides iterate j = -1 .. ny (the extrapolating types fill whole ghost
 // columns, corners included); the other types use j = 0 .. ny-1.
-__device__ void fill_x_ghost(Fld f, const Grid &g, const Geo &geo, const Bc &bc, int homog, int do_neum,
-                             int side, int j) {
-    const int t = bc.type[side];
-    const bool lo = side == XLO;
+__device__ __forceinline__ void fill_x_ghost(Fld f, const Grid &g, const Geo &geo, const SideBc &bc, int homog,
+                                             int do_neum, bool lo, int j) {
+    const int t = bc.type;
     const int nx = g.nx;
     const bool edge_row = (j < 0 || j >= g.ny);
     if (t == BC_EXTRAP0 || t == BC_EXTRAP1 || t == BC_EXTRAP2) {
@@ -101,19 +125,18 @@ __device__ void fill_x_ghost(Fld f, const Grid &g, const Geo &geo, const Bc &bc,
     }
     if (edge_row) return;
     if (t == BC_NEUM) {
-        if (do_neum) neum_x_ghost(f, g, geo, bc, homog, side, j);
+        if (do_neum) neum_x_ghost(f, g, geo, bc, homog, lo, j);
     } else if (t == BC_DIRI) {
         const int e = lo ? -1 : 1, i = lo ? 0 : nx - 1;
-        f(i + e, j) = diri_ghost(bc, side, homog, f(i, j), f(i - e, j), f(i - 2 * e, j), j);
+        f(i + e, j) = diri_ghost(bc, homog, f(i, j), f(i - e, j), f(i - 2 * e, j), j);
     } else if (t == BC_PERIODIC) {
         f(lo ? -1 : nx, j) = f(lo ? nx - 1 : 0, j);
     }
 }
 
-__device__ void fill_y_ghost(Fld f, const Grid &g, const Geo &geo, const Bc &bc, int homog, int do_neum,
-                             int side, int i) {
-    const int t = bc.type[side];
-    const bool lo = side == YLO;
+__device__ __forceinline__ void fill_y_ghost(Fld f, const Grid &g, const Geo &geo, const SideBc &bc, int homog,
+                                             int do_neum, bool lo, int i) {
+    const int t = bc.type;
     const int ny = g.ny;
     const bool edge_col = (i < 0 || i >= g.nx);
     if (t == BC_EXTRAP0 || t == BC_EXTRAP1 || t == BC_EXTRAP2) {
@@ -126,16 +149,16 @@ __device__ void fill_y_ghost(Fld f, const Grid &g, const Geo &geo, const Bc &bc,
     }
     if (edge_col) return;
     if (t == BC_NEUM) {
-        if (do_neum) neum_y_ghost(f, g, geo, bc, homog, side, i);
+        if (do_neum) neum_y_ghost(f, g, geo, bc, homog, lo, i);
     } else if (t == BC_DIRI) {
         const int e = lo ? -1 : 1, j = lo ? 0 : ny - 1;
-        f(i, j + e) = diri_ghost(bc, side, homog, f(i, j), f(i, j - e), f(i, j - 2 * e), i);
+        f(i, j + e) = diri_ghost(bc, homog, f(i, j), f(i, j - e), f(i, j - 2 * e), i);
     } else if (t == BC_PERIODIC) {
         f(i, lo ? -1 : ny) = f(i, lo ? ny - 1 : 0);
     }
 }
 
-__device__ void fill_corners(Fld f, const Grid &g, const Bc &bc) {
+__device__ __forceinline__ void fill_corners(Fld f, const Grid &g, const Bc &bc) {
     const int nx = g.nx, ny = g.ny;
     const bool px = bc.type[XLO] == BC_PERIODIC, py = bc.type[YLO] == BC_PERIODIC;
     if (!px && !py) {
@@ -161,21 +184,31 @@ __device__ void fill_corners(Fld f, const Grid &g, const Bc &bc) {
     }
 }
 
-__device__ void block_fill_ghosts(Fld f, const Grid &g, const Geo &geo, const Bc &bc, int homog, int do_neum) {
+// Whether a side's fill writes anything.
+__device__ __forceinline__ bool fills(const Bc &bc, int side, int do_neum) {
+    return bc.type[side] == BC_NEUM ? do_neum != 0 : bc.type[side] >= 0;
+}
+
+__device__ __forceinline__ void block_fill_ghosts(Fld f, const Grid &g, const Geo &geo, const Bc &bc, int homog,
+                                                  int do_neum) {
     const int tid = threadIdx.x, nt = blockDim.x;
     // the two x sides are independent of each other
-    for (int k = tid; k < 2 * (g.ny + 2); k += nt) {
-        const int side = k < g.ny + 2 ? XLO : XHI;
-        const int j = (k % (g.ny + 2)) - 1;
-        fill_x_ghost(f, g, geo, bc, homog, do_neum, side, j);
+    if (fills(bc, XLO, do_neum) || fills(bc, XHI, do_neum)) {
+        for (int k = tid; k < 2 * (g.ny + 2); k += nt) {
+            const bool lo = k < g.ny + 2;
+            fill_x_ghost(f, g, geo, x_side(bc, lo), homog, do_neum, lo, (lo ? k : k - (g.ny + 2)) - 1);
+        }
+        __syncthreads();
     }
-    __syncthreads();
-    for (int k = tid; k < 2 * (g.nx + 2); k += nt) {
-        const int side = k < g.nx + 2 ? YLO : YHI;
-        const int i = (k % (g.nx + 2)) - 1;
-        fill_y_ghost(f, g, geo, bc, homog, do_neum, side, i);
+    if (fills(bc, YLO, do_neum) || fills(bc, YHI, do_neum)) {
+        for (int k = tid; k < 2 * (g.nx + 2); k += nt) {
+            const bool lo = k < g.nx + 2;
+            fill_y_ghost(f, g, geo, y_side(bc, lo), homog, do_neum, lo, (lo ? k : k - (g.nx + 2)) - 1);
+        }
+        // the extrapolating fills write the corners (which fill_corners then
+        // replaces) and the periodic corners read the y ghosts
+        __syncthreads();
     }
-    __syncthreads();
     if (tid == 0) fill_corners(f, g, bc);
     __syncthreads();
 }
@@ -339,27 +372,25 @@ __device__ __forceinline__ void gs_cell(Fld phi, const double *rhs, const double
 
 // Ring phase of the multi-colour sweep, one workgroup: refresh ghosts
 // (do_neum = .false.), ring cells in 4 colours, then the 4 corners.
-__device__ void block_gs_mc_ring(Fld phi, const double *rhs, const double *invd, const Grid &g, const Geo &geo,
-                                 const Bc &bc, int homog, double omega) {
+__device__ __forceinline__ void block_gs_mc_ring(Fld phi, const double *rhs, const double *invd, const Grid &g,
+                                                 const Geo &geo, const Bc &bc, int homog, double omega) {
     const int nx = g.nx, ny = g.ny;
     block_fill_ghosts(phi, g, geo, bc, homog, 0);
     const int nring = 2 * (nx - 2) + 2 * (ny - 2);
-    for (int colour = 0; colour < 4; ++colour) {
-        for (int k = threadIdx.x; k < nring; k += blockDim.x) {
+#pragma unroll 1
+    for (int colour = 0; colour < 5; ++colour) {
+        for (int k = threadIdx.x; k < (colour < 4 ? nring : 4); k += blockDim.x) {
             int i, j;
-            if (k < nx - 2) { i = 1 + k; j = 0; }
+            if (colour == 4) { i = (k & 1) ? nx - 1 : 0; j = (k & 2) ? ny - 1 : 0; }
+            else if (k < nx - 2) { i = 1 + k; j = 0; }
             else if (k < 2 * (nx - 2)) { i = 1 + k - (nx - 2); j = ny - 1; }
             else if (k < 2 * (nx - 2) + (ny - 2)) { i = 0; j = 1 + k - 2 * (nx - 2); }
             else { i = nx - 1; j = 1 + k - 2 * (nx - 2) - (ny - 2); }
-            if (((i & 1) | ((j & 1) << 1)) == colour) gs_cell(phi, rhs, invd, g, geo, bc, homog, omega, i, j);
+            if (colour == 4 || ((i & 1) | ((j & 1) << 1)) == colour)
+                gs_cell(phi, rhs, invd, g, geo, bc, homog, omega, i, j);
         }
         __syncthreads();
     }
-    if (threadIdx.x < 4) {
-        const int i = (threadIdx.x & 1) ? nx - 1 : 0, j = (threadIdx.x & 2) ? ny - 1 : 0;
-        gs_cell(phi, rhs, invd, g, geo, bc, homog, omega, i, j);
-    }
-    __syncthreads();
 }
 
 __global__ void __launch_bounds__(1024) k_gs_mc_ring(Fld phi, const double *rhs, const double *invd, Grid g,
@@ -374,13 +405,15 @@ __global__ void __launch_bounds__(1024) k_gs_mc_ring(Fld phi, const double *rhs,
 __global__ void __launch_bounds__(256) k_fill_x_ghosts(Fld f, Grid g, Geo geo, Bc bc, int homog, int do_neum) {
     const int k = blockIdx.x * 256 + threadIdx.x;
     if (k >= 2 * (g.ny + 2)) return;
-    fill_x_ghost(f, g, geo, bc, homog, do_neum, k < g.ny + 2 ? XLO : XHI, (k % (g.ny + 2)) - 1);
+    const bool lo = k < g.ny + 2;
+    fill_x_ghost(f, g, geo, x_side(bc, lo), homog, do_neum, lo, (lo ? k : k - (g.ny + 2)) - 1);
 }
 
 __global__ void __launch_bounds__(256) k_fill_y_ghosts(Fld f, Grid g, Geo geo, Bc bc, int homog, int do_neum) {
     const int k = blockIdx.x * 256 + threadIdx.x;
     if (k >= 2 * (g.nx + 2)) return;
-    fill_y_ghost(f, g, geo, bc, homog, do_neum, k < g.nx + 2 ? YLO : YHI, (k % (g.nx + 2)) - 1);
+    const bool lo = k < g.nx + 2;
+    fill_y_ghost(f, g, geo, y_side(bc, lo), homog, do_neum, lo, (lo ? k : k - (g.nx + 2)) - 1);
 }
 
 __global__ void k_fill_corner_ghosts(Fld f, Grid g, Bc bc) {
@@ -412,7 +445,7 @@ __global__ void k_gs_mc_corner_cells(Fld phi, const double *rhs, const double *i
 // every value a cell reads from an earlier row (reach up to (i+2, j-1)) lies
 // on an earlier front and every later-row or later-column read on a later
 // one.  One workgroup; ghosts refreshed once per sweep as in the reference.
-__device__ void block_gs_lex(Fld phi, const double *rhs, const double *invd, const Grid &g, const Geo &geo,
+__device__ __forceinline__ void block_gs_lex(Fld phi, const double *rhs, const double *invd, const Grid &g, const Geo &geo,
                              const Bc &bc, int homog, double omega, int sweeps) {
     const int nx = g.nx, ny = g.ny;
     for (int s = 0; s < sweeps; ++s) {
@@ -459,7 +492,7 @@ __global__ void __launch_bounds__(256) k_dc_rb(Fld phi, const double *modrhs, co
 
 // Lexicographic DC sweeps (MGPoisson2D_DD.f90:288-306) by wavefronts t = i + j,
 // one workgroup, ghosts refreshed per sweep (do_neum = .true.).
-__device__ void block_dc_lex(Fld phi, const double *modrhs, const double *invd, const Grid &g, const Geo &geo,
+__device__ __forceinline__ void block_dc_lex(Fld phi, const double *modrhs, const double *invd, const Grid &g, const Geo &geo,
                              const Bc &bc, int homog, double omega, int sweeps) {
     const int nx = g.nx, ny = g.ny;
     for (int s = 0; s < sweeps; ++s) {
@@ -718,20 +751,65 @@ __global__ void __launch_bounds__(256) k_reduce_final(double *out, const double 
     if (threadIdx.x == 0) *out = v;
 }
 
-// Sequential J-weighted sums in the reference's loop order (one thread):
-// out[0] = sum dvol*fine, out[1] = sum dvol, dvol = dxprod*J.
-__global__ void k_seq_mean(double *out, const double *fine, const double *J, Grid g, double dxprod) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    double sum = 0.0, vol = 0.0;
-    for (int j = 0; j < g.ny; ++j)
-        for (int i = 0; i < g.nx; ++i) {
-            const size_t c = ix(g.pitch, i, j);
-            const double dvol = dxprod * J[c];
-            sum = sum + dvol * fine[c];
-            vol = vol + dvol;
+// Sequential J-weighted sums in the reference's loop order (rows outer,
+// columns inner): out[0] = sum dvol*fine, out[1] = sum dvol, dvol = dxprod*J.
+// Bound by the chain of dependent additions, one per cell, that the order
+// prescribes.  The last two waves stage the terms of the next tile in LDS
+// while lane 0 of the first wave adds the current tile's dvol*fine and lane 0
+// of the second its dvol, so the chain never waits for global memory (one
+// thread loading its own operands took 70 ns a cell).
+constexpr int SM_TILE = 1024, SM_STAGE = 128;  // cells per tile, staging threads
+
+__device__ __forceinline__ double seq_add(double acc, const double *t) {
+    double x[16], y[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) x[q] = t[q];
+    for (int k = 16; k < SM_TILE; k += 32) {
+#pragma unroll
+        for (int q = 0; q < 16; ++q) y[q] = t[k + q];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) acc = acc + x[q];
+        if (k + 16 < SM_TILE) {
+#pragma unroll
+            for (int q = 0; q < 16; ++q) x[q] = t[k + 16 + q];
         }
-    out[0] = sum;
-    out[1] = vol;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) acc = acc + y[q];
+    }
+    return acc;
+}
+
+__global__ void __launch_bounds__(256) k_seq_mean(double *out, const double *fine, const double *J, Grid g, double dxprod) {
+    __shared__ __attribute__((aligned(16))) double term[2][2][SM_TILE];  // [buffer][dvol*fine | dvol]
+    const int n = g.nx * g.ny, ntiles = (n + SM_TILE - 1) / SM_TILE, tid = threadIdx.x;
+    // cells past the end are -0.0: adding it changes no sum
+    auto stage = [&](int t, int first, int threads) {
+        double *wf = term[t & 1][0], *w = term[t & 1][1];
+        for (int q = tid - first; q < SM_TILE; q += threads) {
+            const int k = t * SM_TILE + q;
+            double dvol = -0.0, v = -0.0;
+            if (k < n) {
+                const int j = k / g.nx;
+                const size_t c = ix(g.pitch, k - j * g.nx, j);
+                dvol = dxprod * J[c];
+                v = dvol * fine[c];
+            }
+            w[q] = dvol;
+            wf[q] = v;
+        }
+    };
+    stage(0, 0, 256);
+    __syncthreads();
+    double acc = 0.0;
+    for (int t = 0; t < ntiles; ++t) {
+        if (tid >= 256 - SM_STAGE) {
+            if (t + 1 < ntiles) stage(t + 1, 256 - SM_STAGE, SM_STAGE);
+        } else if ((tid & 63) == 0) {
+            acc = seq_add(acc, term[t & 1][tid >> 6]);
+        }
+        __syncthreads();
+    }
+    if (tid < 128 && (tid & 63) == 0) out[tid >> 6] = acc;
 }
 
 // fine = fine - sums[0]/sums[1] over the cells and the ghost ring.
@@ -749,113 +827,151 @@ __global__ void __launch_bounds__(256) k_sub_mean(double *fine, const double *su
 // reduced in the reference's sequential order by thread 0, so the bottom
 // trajectory (restart and convergence decisions included) matches.
 // ===========================================================================
-using Bottom = BottomArgs;  // work arrays use the padded layout
+// The fields a workgroup works on: those of the arguments, or their copies in
+// LDS.  The BCs stay in the kernel's arguments (their sides are indexed at run
+// time, which in a copy would mean scratch memory).
+struct Bottom {
+    Grid g;
+    Geo geo;
+    const Bc &bc;
+    double *phi, *rhs, *invd;
+    double *e, *pt, *st, *r, *rt, *p, *t, *v, *mod;
+    double *scal;
+    int max_iters, max_restarts, homog;
+    double tol;
+};
 
-__device__ double seq_dot(const Bottom &B, const double *a, const double *b) {
-    // inner_prod (arrayutils.f90:637-661): per-row dot, scaled, accumulated
-    __shared__ double res;
-    if (threadIdx.x == 0) {
-        const double vol = B.g.dx * B.g.dy;
-        double ip = 0.0;
-        for (int j = 0; j < B.g.ny; ++j) {
+// Scratch of the ordered sums.
+constexpr int SEQ_BUF = 1024;
+
+// inner_prod (arrayutils.f90:637-661): per-row dot products, scaled and
+// accumulated row by row.  A row's dot is a chain of its own, so each thread
+// sums whole rows and thread 0 then adds the rows' results in order: the
+// additions and their order are the reference's.
+__device__ __forceinline__ double seq_dot(const Bottom &B, const double *a, const double *b, double *buf) {
+    const double vol = B.g.dx * B.g.dy;
+    double ip = 0.0;
+    for (int j0 = 0; j0 < B.g.ny; j0 += SEQ_BUF) {
+        const int rows = B.g.ny - j0 < SEQ_BUF ? B.g.ny - j0 : SEQ_BUF;
+        for (int q = threadIdx.x; q < rows; q += blockDim.x) {
+            const double *ra = a + ix(B.g.pitch, 0, j0 + q), *rb = b + ix(B.g.pitch, 0, j0 + q);
             double d = 0.0;
-            for (int i = 0; i < B.g.nx; ++i) d = d + a[ix(B.g.pitch, i, j)] * b[ix(B.g.pitch, i, j)];
-            ip = ip + vol * d;
+#pragma unroll 4
+            for (int i = 0; i < B.g.nx; ++i) d = d + ra[i] * rb[i];
+            buf[q] = vol * d;
         }
-        res = ip;
+        __syncthreads();
+        // every thread forms the same sum: no broadcast
+#pragma unroll 8
+        for (int q = 0; q < rows; ++q) ip = ip + buf[q];
+        __syncthreads();
     }
-    __syncthreads();
-    const double v = res;
-    __syncthreads();
-    return v;
+    return ip;
 }
 
-__device__ double seq_norm(const Bottom &B, const double *a, int p) {
-    __shared__ double res;
-    if (threadIdx.x == 0) {
-        const double vs = B.g.dx * B.g.dy;
-        double pn = 0.0;
-        for (int j = 0; j < B.g.ny; ++j)
-            for (int i = 0; i < B.g.nx; ++i) {
-                const double x = a[ix(B.g.pitch, i, j)];
-                if (p == 0) pn = fmax(pn, fabs(x));
-                else pn = pn + vs * (x * x);
-            }
-        res = p == 0 ? pn : sqrt(pn);
+// pnorm (arrayutils.f90:753-790): p = 0 the maximum, in any order; p = 2 the
+// terms dx dy x^2 added cell by cell in the reference's order, staged in LDS
+// by the whole workgroup.
+template <int p>
+__device__ __forceinline__ double seq_norm(const Bottom &B, const double *a, double *buf) {
+    const double vs = B.g.dx * B.g.dy;
+    const int n = B.g.nx * B.g.ny;
+    double pn = 0.0;
+    if (p == 0) {
+        for (int k = threadIdx.x; k < n; k += blockDim.x) {
+            const int j = k / B.g.nx;
+            pn = fmax(pn, fabs(a[ix(B.g.pitch, k - j * B.g.nx, j)]));
+        }
+        buf[threadIdx.x] = pn;
+        __syncthreads();
+        const int m = n < (int)blockDim.x ? n : (int)blockDim.x;
+        pn = 0.0;
+#pragma unroll 8
+        for (int q = 0; q < m; ++q) pn = fmax(pn, buf[q]);
+        __syncthreads();
+        return pn;
     }
-    __syncthreads();
-    const double v = res;
-    __syncthreads();
-    return v;
+    for (int k0 = 0; k0 < n; k0 += SEQ_BUF) {
+        const int m = n - k0 < SEQ_BUF ? n - k0 : SEQ_BUF;
+        for (int q = threadIdx.x; q < m; q += blockDim.x) {
+            const int k = k0 + q, j = k / B.g.nx;
+            const double x = a[ix(B.g.pitch, k - j * B.g.nx, j)];
+            buf[q] = vs * (x * x);
+        }
+        __syncthreads();
+#pragma unroll 8
+        for (int q = 0; q < m; ++q) pn = pn + buf[q];
+        __syncthreads();
+    }
+    return sqrt(pn);
 }
 
+// fn(i, j, offset) for every cell (and ghost) of the level, then a barrier.
+// The functions are always inlined: a call would pass what they refer to
+// through scratch memory.
+#define CELL_FN __attribute__((always_inline))
 template <class F>
 __device__ __forceinline__ void block_cells(const Grid &g, int ghosted, F fn) {
     const int o = ghosted ? 1 : 0;
     const int w = g.nx + 2 * o, h = g.ny + 2 * o;
-    for (int k = threadIdx.x; k < w * h; k += blockDim.x) fn(k % w - o, k / w - o, ix(g.pitch, k % w - o, k / w - o));
+    for (int k = threadIdx.x; k < w * h; k += blockDim.x) {
+        const int j = k / w, i = k - j * w;
+        fn(i - o, j - o, ix(g.pitch, i - o, j - o));
+    }
     __syncthreads();
 }
 
-__device__ void block_residual(const Bottom &B, int homog, const double *rhs, double *phi, double *res) {
+// out = L phi, or rhs - L phi with rhs given.
+template <bool DC>
+__device__ __forceinline__ void block_operator(const Bottom &B, int homog, const double *rhs, double *phi, double *out) {
     Fld f{phi, B.g.pitch};
-    if (B.dc) {
-        block_fill_ghosts(f, B.g, B.geo, B.bc, homog, 1);
-        block_cells(B.g, 0, [&](int i, int j, size_t c) {
+    block_fill_ghosts(f, B.g, B.geo, B.bc, homog, DC ? 1 : 0);
+    block_cells(B.g, 0, [&](int i, int j, size_t c) CELL_FN {
+        double v;
+        if (DC) {
             double ax, ay;
             dc_five(CFld{phi, B.g.pitch}, B.g, B.geo, i, j, ax, ay);
-            res[c] = rhs[c] - (dc_cross(CFld{phi, B.g.pitch}, B.g, B.geo, i, j) + ax + ay);
-        });
-    } else {
-        block_fill_ghosts(f, B.g, B.geo, B.bc, homog, 0);
-        block_cells(B.g, 0, [&](int i, int j, size_t c) {
-            res[c] = rhs[c] - cell_lap(CFld{phi, B.g.pitch}, B.g, B.geo, B.bc, homog, i, j);
-        });
-    }
-}
-
-__device__ void block_laplacian(const Bottom &B, double *phi, double *out) {
-    Fld f{phi, B.g.pitch};
-    if (B.dc) {
-        block_fill_ghosts(f, B.g, B.geo, B.bc, 1, 1);
-        block_cells(B.g, 0, [&](int i, int j, size_t c) {
-            double ax, ay;
-            dc_five(CFld{phi, B.g.pitch}, B.g, B.geo, i, j, ax, ay);
-            out[c] = dc_cross(CFld{phi, B.g.pitch}, B.g, B.geo, i, j) + ax + ay;
-        });
-    } else {
-        block_fill_ghosts(f, B.g, B.geo, B.bc, 1, 0);
-        block_cells(B.g, 0, [&](int i, int j, size_t c) {
-            out[c] = cell_lap(CFld{phi, B.g.pitch}, B.g, B.geo, B.bc, 1, i, j);
-        });
-    }
+            v = dc_cross(CFld{phi, B.g.pitch}, B.g, B.geo, i, j) + ax + ay;
+        } else {
+            v = cell_lap(CFld{phi, B.g.pitch}, B.g, B.geo, B.bc, homog, i, j);
+        }
+        out[c] = rhs ? rhs[c] - v : v;
+    });
 }
 
 // One relax_gs call (tol < 0) on the bottom level, by one workgroup.
-__device__ void block_relax(const Bottom &B, int homog, double omega, int sweeps, const double *rhs, double *phi) {
+template <bool DC, int ORDER>
+__device__ __forceinline__ void block_relax(const Bottom &B, int homog, double omega, int sweeps, const double *rhs,
+                                            double *phi) {
     if (sweeps == 0) return;
     Fld f{phi, B.g.pitch};
-    if (B.dc) {
-        block_cells(B.g, 0, [&](int i, int j, size_t c) {
+    if (DC) {
+        block_cells(B.g, 0, [&](int i, int j, size_t c) CELL_FN {
             B.mod[c] = rhs[c] - dc_lagged_cross(CFld{phi, B.g.pitch}, B.g, B.geo, i, j);
         });
-        if (B.order == 1) {  // red-black
+        if (ORDER == MGP_ORDER_RB) {
+#pragma unroll 1
             for (int s = 0; s < sweeps; ++s) {
                 block_fill_ghosts(f, B.g, B.geo, B.bc, homog, 1);
+#pragma unroll 1
                 for (int colour = 0; colour < 2; ++colour)
-                    block_cells(B.g, 0, [&](int i, int j, size_t) {
+                    block_cells(B.g, 0, [&](int i, int j, size_t) CELL_FN {
                         if (((i + j + colour) & 1) == 0) dc_cell(f, B.mod, B.invd, B.g, B.geo, omega, i, j);
                     });
             }
         } else {
             block_dc_lex(f, B.mod, B.invd, B.g, B.geo, B.bc, homog, omega, sweeps);
         }
-    } else if (B.order == 2) {  // multi-colour
+    } else if (ORDER == MGP_ORDER_MC) {
+#pragma unroll 1
         for (int s = 0; s < sweeps; ++s) {
+#pragma unroll 1
             for (int colour = 0; colour < 4; ++colour)
-                block_cells(B.g, 0, [&](int i, int j, size_t) {
-                    if (i > 0 && i < B.g.nx - 1 && j > 0 && j < B.g.ny - 1 && ((i & 1) | ((j & 1) << 1)) == colour)
-                        gs_cell(f, rhs, B.invd, B.g, B.geo, B.bc, homog, omega, i, j);
+                block_cells(B.g, 0, [&](int i, int j, size_t c) CELL_FN {
+                    if (i > 0 && i < B.g.nx - 1 && j > 0 && j < B.g.ny - 1 && ((i & 1) | ((j & 1) << 1)) == colour) {
+                        const double lphi = cell_lap_interior(CFld{phi, B.g.pitch}, B.g, B.geo, i, j);
+                        phi[c] = gs_update(phi[c], rhs[c], lphi, B.invd[c], omega);
+                    }
                 });
             block_gs_mc_ring(f, rhs, B.invd, B.g, B.geo, B.bc, homog, omega);
         }
@@ -864,62 +980,78 @@ __device__ void block_relax(const Bottom &B, int homog, double omega, int sweeps
     }
 }
 
-__global__ void __launch_bounds__(256) k_bicgstab2(Bottom B) {
+// The two preconditioned halves of an iteration, and the two places that
+// form the residual, are each one piece of code run twice: the kernel has to
+// stay within the instruction cache (inlined at every use it was 117 KB).
+template <bool DC, int ORDER>
+__device__ __forceinline__ void bicgstab2(const Bottom &B, double *buf) {
     const double reps = 1.0e-12, hang = 1.0e-7, small = 1.0e-30;
-    const int norm_type = B.dc ? 0 : 2;
-    const double relax_omega = B.dc ? 4.0 / 5.0 : 1.0 - 1.0 / 3.0;
+    const double relax_omega = DC ? 4.0 / 5.0 : 1.0 - 1.0 / 3.0;
     const int relax_iters = 2;
     const Grid &g = B.g;
     if (B.max_iters == 0) return;
     // e, p_tilde, s_tilde start at zero, ghosts included
-    block_cells(g, 1, [&](int, int, size_t c) { B.e[c] = 0.0; B.pt[c] = 0.0; B.st[c] = 0.0; });
+    block_cells(g, 1, [&](int, int, size_t c) CELL_FN { B.e[c] = 0.0; B.pt[c] = 0.0; B.st[c] = 0.0; });
     int recount = 0, it = 0, restarts = 0, init = 1;
-    block_residual(B, B.homog, B.rhs, B.phi, B.r);
-    block_cells(g, 0, [&](int, int, size_t c) { B.rt[c] = B.r[c]; });
-    double norm0 = seq_norm(B, B.r, norm_type);
-    const double initial_norm = norm0, initial_rnorm = norm0;
-    double norm1 = norm0;
+    bool start = true, fresh = true;  // a residual from phi is due
+    double norm0 = 0, initial_norm = 0, initial_rnorm = 0, norm1 = 0;
     double rho1 = 0, rho2 = 0, alpha0 = 0, alpha1 = 0, omega0 = 0, omega1 = 0, beta1 = 0;
-    while (it < B.max_iters && norm0 > B.tol * norm1 && norm1 > 0.0) {
+#pragma unroll 1
+    while (true) {
+        if (fresh) {
+            block_operator<DC>(B, B.homog, B.rhs, B.phi, B.r);
+            norm0 = seq_norm<DC ? 0 : 2>(B, B.r, buf);
+            block_cells(g, 0, [&](int, int, size_t c) CELL_FN { B.rt[c] = B.r[c]; });
+            if (start) {
+                initial_norm = initial_rnorm = norm1 = norm0;
+                start = false;
+            } else {
+                block_cells(g, 1, [&](int, int, size_t c) CELL_FN { B.e[c] = 0.0; });
+            }
+            fresh = false;
+        }
+        if (!(it < B.max_iters && norm0 > B.tol * norm1 && norm1 > 0.0)) break;
         ++it;
         norm1 = norm0;
         alpha1 = alpha0;
         beta1 = 0.0;
         omega1 = omega0;
         rho2 = rho1;
-        rho1 = seq_dot(B, B.rt, B.r);
+        rho1 = seq_dot(B, B.rt, B.r, buf);
         if (rho1 == 0.0) break;
         if (init) {
-            block_cells(g, 0, [&](int, int, size_t c) { B.p[c] = B.r[c]; });
+            block_cells(g, 0, [&](int, int, size_t c) CELL_FN { B.p[c] = B.r[c]; });
             init = 0;
         } else {
             beta1 = (rho1 / rho2) * (alpha1 / omega1);
             const double b1 = beta1, o1 = omega1;
-            block_cells(g, 0, [&](int, int, size_t c) { B.p[c] = b1 * (B.p[c] - o1 * B.v[c]) + B.r[c]; });
+            block_cells(g, 0, [&](int, int, size_t c) CELL_FN { B.p[c] = b1 * (B.p[c] - o1 * B.v[c]) + B.r[c]; });
         }
-        block_cells(g, 0, [&](int, int, size_t c) { B.pt[c] = B.p[c] * B.invd[c]; });
-        block_relax(B, 1, relax_omega, relax_iters, B.p, B.pt);
-        block_laplacian(B, B.pt, B.v);
-        const double m = seq_dot(B, B.rt, B.v);
-        alpha0 = rho1 / m;
-        if (fabs(m) > small * fabs(rho1)) {
-            const double a0 = alpha0;
-            block_cells(g, 0, [&](int, int, size_t c) { B.r[c] = B.r[c] - a0 * B.v[c]; });
-            norm0 = seq_norm(B, B.r, norm_type);
-            block_cells(g, 1, [&](int, int, size_t c) { B.e[c] = B.e[c] + a0 * B.pt[c]; });
-        } else {
-            block_cells(g, 0, [&](int, int, size_t c) { B.r[c] = 0.0; });
-            norm0 = 0.0;
-        }
-        if (norm0 > B.tol * initial_norm && norm0 > reps * initial_rnorm) {
-            block_cells(g, 0, [&](int, int, size_t c) { B.st[c] = B.r[c] * B.invd[c]; });
-            block_relax(B, 1, relax_omega, relax_iters, B.r, B.st);
-            block_laplacian(B, B.st, B.t);
-            omega0 = seq_dot(B, B.t, B.r) / seq_dot(B, B.t, B.t);
-            const double o0 = omega0;
-            block_cells(g, 1, [&](int, int, size_t c) { B.e[c] = B.e[c] + o0 * B.st[c]; });
-            block_cells(g, 0, [&](int, int, size_t c) { B.r[c] = B.r[c] - o0 * B.t[c]; });
-            norm0 = seq_norm(B, B.r, norm_type);
+#pragma unroll 1
+        for (int half = 0; half < 2; ++half) {
+            const double *src = half ? B.r : B.p;
+            double *x = half ? B.st : B.pt, *y = half ? B.t : B.v;
+            block_cells(g, 0, [&](int, int, size_t c) CELL_FN { x[c] = src[c] * B.invd[c]; });
+            block_relax<DC, ORDER>(B, 1, relax_omega, relax_iters, src, x);
+            block_operator<DC>(B, 1, nullptr, x, y);
+            double step;
+            if (half == 0) {
+                const double m = seq_dot(B, B.rt, B.v, buf);
+                alpha0 = rho1 / m;
+                if (!(fabs(m) > small * fabs(rho1))) {
+                    block_cells(g, 0, [&](int, int, size_t c) CELL_FN { B.r[c] = 0.0; });
+                    norm0 = 0.0;
+                    break;
+                }
+                step = alpha0;
+            } else {
+                omega0 = seq_dot(B, B.t, B.r, buf) / seq_dot(B, B.t, B.t, buf);
+                step = omega0;
+            }
+            block_cells(g, 1, [&](int, int, size_t c) CELL_FN { B.e[c] = B.e[c] + step * x[c]; });
+            block_cells(g, 0, [&](int, int, size_t c) CELL_FN { B.r[c] = B.r[c] - step * y[c]; });
+            norm0 = seq_norm<DC ? 0 : 2>(B, B.r, buf);
+            if (half == 0 && !(norm0 > B.tol * initial_norm && norm0 > reps * initial_rnorm)) break;
         }
         if (norm0 <= B.tol * initial_norm || norm0 <= reps * initial_rnorm) break;
         if (omega0 == 0.0 || norm0 > (1.0 - hang) * norm1) {
@@ -927,33 +1059,69 @@ __global__ void __launch_bounds__(256) k_bicgstab2(Bottom B) {
                 recount = 1;
             } else {
                 recount = 0;
-                block_cells(g, 1, [&](int, int, size_t c) { B.phi[c] = B.phi[c] + B.e[c]; });
+                block_cells(g, 1, [&](int, int, size_t c) CELL_FN { B.phi[c] = B.phi[c] + B.e[c]; });
                 // the reference exits here and adds e once more after the loop
                 if (restarts == B.max_restarts) break;
-                block_residual(B, B.homog, B.rhs, B.phi, B.r);
-                norm0 = seq_norm(B, B.r, norm_type);
                 rho1 = rho2 = 0.0;
                 alpha0 = 0.0;
                 omega0 = 0.0;
-                block_cells(g, 0, [&](int, int, size_t c) { B.rt[c] = B.r[c]; });
-                block_cells(g, 1, [&](int, int, size_t c) { B.e[c] = 0.0; });
                 ++restarts;
                 init = 1;
+                fresh = true;
             }
         }
     }
     (void)beta1;
-    block_cells(g, 1, [&](int, int, size_t c) { B.phi[c] = B.phi[c] + B.e[c]; });
+    block_cells(g, 1, [&](int, int, size_t c) CELL_FN { B.phi[c] = B.phi[c] + B.e[c]; });
     if (threadIdx.x == 0 && B.scal) {
         B.scal[0] = (double)it;
         B.scal[1] = norm0;
     }
 }
 
-// Whole relax_gs call on a small level in one workgroup (coarse levels,
-// parity mode): the same block functions the bottom solver uses.
-__global__ void __launch_bounds__(256) k_relax_block(Bottom B, double omega, int sweeps, int homog) {
-    block_relax(B, homog, omega, sweeps, B.rhs, B.phi);
+// Any size: the fields stay in global memory.
+template <bool DC, int ORDER>
+__global__ void __launch_bounds__(256) k_bicgstab2(BottomArgs A) {
+    __shared__ double buf[SEQ_BUF];
+    const Bottom B{A.g, A.geo, A.bc, A.phi, A.rhs, A.invd, A.e, A.pt, A.st, A.r, A.rt, A.p, A.t, A.v, A.mod, A.scal, A.max_iters, A.max_restarts, A.homog, A.tol};
+    bicgstab2<DC, ORDER>(B, buf);
+}
+
+// Bottom levels whose 16 fields fit in LDS.  An iteration is some 70 phases
+// with a barrier after each, so the time is the phases' latency: from LDS a
+// phase waits for no global memory, and the bottoms of power-of-two grids
+// (4 x 4) take one wave, whose barriers cost nothing.
+enum { BL_PHI = 0, BL_RHS, BL_INVD, BL_JXX, BL_JXY, BL_JYX, BL_JYY, BL_IN, BL_COUNT = BL_IN + 9 };
+__host__ __device__ inline int bottom_lds_elems(const Grid &g) { return OFFX + BL_COUNT * (g.nx + 2) * (g.ny + 2); }
+
+template <bool DC, int ORDER, int NT>
+__global__ void __launch_bounds__(NT) k_bicgstab2_lds(BottomArgs A) {
+    extern __shared__ __attribute__((aligned(16))) double bottom_lds[];
+    __shared__ double buf[SEQ_BUF];
+    if (A.max_iters == 0) return;
+    const int w = A.g.nx + 2, sz = w * (A.g.ny + 2);
+    // the level layout with a pitch of nx + 2: cell (-1, -1) first (OFFX
+    // elements are kept free in front, so no pointer lies before the array)
+    auto at = [&](int f) { return bottom_lds + OFFX + f * sz + 1 - OFFX; };
+    const double *const in[BL_IN] = {A.phi, A.rhs, A.invd, A.geo.Jxx, A.geo.Jxy, A.geo.Jyx, A.geo.Jyy};
+    for (int k = threadIdx.x; k < sz; k += NT) {
+        const int j = k / w - 1, i = k - (j + 1) * w - 1;
+        const size_t c = ix(A.g.pitch, i, j);
+#pragma unroll
+        for (int f = 0; f < BL_IN; ++f) bottom_lds[OFFX + f * sz + k] = in[f][c];
+#pragma unroll
+        for (int f = BL_IN; f < BL_COUNT; ++f) bottom_lds[OFFX + f * sz + k] = 0.0;
+    }
+    __syncthreads();
+    const Bottom B{Grid{A.g.nx, A.g.ny, w, A.g.dx, A.g.dy}, Geo{nullptr, at(BL_JXX), at(BL_JXY), at(BL_JYX), at(BL_JYY)},
+                   A.bc, at(BL_PHI), at(BL_RHS), at(BL_INVD), at(BL_IN), at(BL_IN + 1), at(BL_IN + 2), at(BL_IN + 3),
+                   at(BL_IN + 4), at(BL_IN + 5), at(BL_IN + 6), at(BL_IN + 7), at(BL_IN + 8), A.scal, A.max_iters,
+                   A.max_restarts, A.homog, A.tol};
+    bicgstab2<DC, ORDER>(B, buf);
+    for (int k = threadIdx.x; k < sz; k += NT) {
+        const int j = k / w - 1, i = k - (j + 1) * w - 1;
+        A.phi[ix(A.g.pitch, i, j)] = bottom_lds[OFFX + BL_PHI * sz + k];
+    }
 }
 
 }  // namespace mgp
@@ -1203,14 +1371,25 @@ void launch_bicg_update(hipStream_t s, double *out, const double *x, const doubl
     k_bicg_update<<<tiles(g.nx, g.ny), 256, 0, s>>>(out, x, y, sc, g, op);
 }
 void launch_seq_mean(hipStream_t s, double *out, const double *fine, const double *J, const Grid &g, double dxprod) {
-    k_seq_mean<<<1, 64, 0, s>>>(out, fine, J, g, dxprod);
+    k_seq_mean<<<1, 256, 0, s>>>(out, fine, J, g, dxprod);
 }
 void launch_sub_mean(hipStream_t s, double *fine, const double *sums, const Grid &g) {
     k_sub_mean<<<tiles(g.nx + 2, g.ny + 2), 256, 0, s>>>(fine, sums, g);
 }
-void launch_bicgstab2(hipStream_t s, const BottomArgs &a) { k_bicgstab2<<<1, 256, 0, s>>>(a); }
-void launch_relax_block(hipStream_t s, const BottomArgs &a, double omega, int sweeps, int homog) {
-    k_relax_block<<<1, 256, 0, s>>>(a, omega, sweeps, homog);
+template <bool DC, int ORDER>
+static void launch_bottom(hipStream_t s, const BottomArgs &a) {
+    // LDS while the fields fit beside the sums' scratch (29 x 29 cells and
+    // the like); one wave while it holds the cells in one pass
+    const size_t lds = (size_t)bottom_lds_elems(a.g) * sizeof(double);
+    if (lds > 128 * 1024) k_bicgstab2<DC, ORDER><<<1, 256, 0, s>>>(a);
+    else if (a.g.nx * a.g.ny <= 64) k_bicgstab2_lds<DC, ORDER, 64><<<1, 64, lds, s>>>(a);
+    else k_bicgstab2_lds<DC, ORDER, 256><<<1, 256, lds, s>>>(a);
+}
+void launch_bicgstab2(hipStream_t s, const BottomArgs &a) {
+    if (a.dc && a.order == MGP_ORDER_RB) launch_bottom<true, MGP_ORDER_RB>(s, a);
+    else if (a.dc) launch_bottom<true, MGP_ORDER_LEX>(s, a);
+    else if (a.order == MGP_ORDER_MC) launch_bottom<false, MGP_ORDER_MC>(s, a);
+    else launch_bottom<false, MGP_ORDER_LEX>(s, a);
 }
 
 }  // namespace mgp

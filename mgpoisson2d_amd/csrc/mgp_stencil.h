@@ -7,9 +7,6 @@
 //                  in compute_invdiags :16-388)
 //  * dc_*          DeferredPoisson2D's low-order operator and lagged cross
 //                  terms (MGPoisson2D_DD.f90:45-119, :227-250)
-//  * fill_*        arrayutils.f90 fill_ghosts (:1277-1492) and its side
-//                  helpers (:871-1272); Dirichlet ghosts are order 3
-//                  (:1284-1287)
 //
 // Operand order follows the reference expression by expression; all HIP code
 // is compiled with -ffp-contract=off, so results equal the reference's bit
@@ -304,35 +301,5 @@ __device__ __forceinline__ void dc_five(const CFld &f, const Grid &g, const Geo 
     dc_five_vals(q[0], q[1], q[-1], q[P], q[-P], geo.Jxx[c + 1], geo.Jxx[c], geo.Jyy[c + P], geo.Jyy[c], idx, idy,
                  ax, ay);
 }
-
-// ---------------------------------------------------------------------------
-// Ghost fills, one boundary cell at a time.  A kernel runs the x sides, then
-// (after a barrier) the y sides, then the corners, as fill_ghosts does.
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ double bcval(const Bc &bc, int side, int k) {
-    return bc.mode[side] == MODE_NONUNIFORM ? bc.data[side][k] : bc.val[side];
-}
-
-// Dirichlet order 3 (arrayutils.f90:1160-1177, :1237-1254) or LAH (negate).
-__device__ __forceinline__ double diri_ghost(const Bc &bc, int side, int homog, double p0, double p1,
-                                             double p2, int k) {
-    if (bc.mode[side] == MODE_LAH) return -p0;
-    const double sixteenfifth = 16.0 / 5.0, fifth = 1.0 / 5.0;
-    if (homog) return -3.0 * p0 + p1 - fifth * p2;
-    return sixteenfifth * bcval(bc, side, k) - 3.0 * p0 + p1 - fifth * p2;
-}
-
-// x-side ghost (side XLO/XHI) at row j: fill_ghosts_neum/diri/periodic.
-__device__ void fill_x_ghost(Fld f, const Grid &g, const Geo &geo, const Bc &bc, int homog,
-                             int do_neum, int side, int j);
-// y-side ghost (side YLO/YHI) at column i.
-__device__ void fill_y_ghost(Fld f, const Grid &g, const Geo &geo, const Bc &bc, int homog,
-                             int do_neum, int side, int i);
-// Corners after the four sides (arrayutils.f90:1459-1490); one thread.
-__device__ void fill_corners(Fld f, const Grid &g, const Bc &bc);
-
-// Whole fill by one workgroup (any blockDim), with barriers between phases.
-__device__ void block_fill_ghosts(Fld f, const Grid &g, const Geo &geo, const Bc &bc, int homog,
-                                  int do_neum);
 
 }  // namespace mgp
