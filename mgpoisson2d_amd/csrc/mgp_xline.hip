@@ -12,14 +12,16 @@
 // extrapolations and the Dirichlet ghost rule, use an explicit coefficient
 // table probed once per level with unit impulses (k_ring_coef).
 //
-// One workgroup (256 threads) per row:
+// One workgroup (64 to 512 threads) per row:
 //  1. coalesced pass: each thread evaluates d = f - L e and the row
-//     coefficients for cells i = tid + 256 u (all loads issued up front);
+//     coefficients for cells i = tid + NT u (groups of loads issued up front);
 //  2. the values go through LDS into contiguous chunks of C or C+1 cells
 //     per thread (padded stride C+1: no bank conflicts);
-//  3. partition method in registers: each chunk is eliminated towards its
-//     two ends, leaving a tridiagonal system of 2 nt unknowns;
-//  4. parallel cyclic reduction of that system in LDS (log2(2 nt) steps);
+//  3. partition method in registers: each chunk is eliminated to one row in
+//     the chunks' last unknowns;
+//  4. that system is solved by the first wave: one row per lane (after an
+//     elimination of NT / 64 chunks per lane) by parallel cyclic reduction
+//     with cross-lane shuffles;
 //  5. back substitution in registers, transpose back, coalesced e update.
 // Rows are mapped to workgroups so that the rows an XCD processes are
 // contiguous (workgroups are dealt to the 8 XCDs round robin): neighbouring
@@ -246,7 +248,7 @@ struct Buf {
 
 template <int C, int NT, bool SEG = false, int RG = 1, typename T, typename GM>
 __device__ __forceinline__ void row_pass(const RowCtx<T> &X, const T *e_, const T *f_, const T *K_, const Grid &g,
-                                         const GM &geo_, int j, T *Ld, T *La, T *Lb, T *Lc) {
+                                         const GM &geo_, int j, T *Ld, T *La, T *Lb, T *Lc, T (&ev)[C + 1]) {
     constexpr int U = C + 1;
     gconst<T> *e = gptr(e_), *f = gptr(f_), *K = gptr(K_);
     // SEG: the cells solved may be a segment of the row (xline_rows); whole
@@ -315,6 +317,7 @@ __device__ __forceinline__ void row_pass(const RowCtx<T> &X, const T *e_, const 
                 const T xfw = v.Jxx_w * (v.p - v.pw) * X.idx + v.Jxy_w * fourth * (v.pn - v.ps + v.enw - v.esw) * X.idy;
                 const T yfn = v.Jyy_n * (v.pn - v.p) * X.idy + v.Jyx_n * fourth * (v.ene - v.enw + v.pe - v.pw) * X.idx;
                 const T yfs = v.Jyy_s * (v.p - v.ps) * X.idy + v.Jyx_s * fourth * (v.pe - v.pw + v.ese - v.esw) * X.idx;
+                ev[u] = v.p;
                 const int o = iraw < nx ? chunk_pos<C>(il, X.rem) : dump;
                 Ld[o] = v.fv - ((xfe - xfw) * X.idx + (yfn - yfs) * X.idy);
                 La[o] = cut_w && il == 0 ? T(0) : v.Jxx_w * X.idx2 - (v.Jyx_n - v.Jyx_s) * X.ixy4;
@@ -338,6 +341,7 @@ __device__ __forceinline__ void row_pass(const RowCtx<T> &X, const T *e_, const 
             const int iraw = tid + NT * u;
             const int il = iraw < nx ? iraw : nx - 1;
             const int i = i0 + il;
+            ev[u] = e[ix(P, i, j)];
             const T fv = f[ix(P, i, j)];
             const T lap = ring_lap(e, K, X.nring, g, i, j);
             T a, b, c;
@@ -351,170 +355,165 @@ __device__ __forceinline__ void row_pass(const RowCtx<T> &X, const T *e_, const 
     }
 }
 
-// Coalesced update e(:, j) += x, x in the chunk layout (e re-read).
+// Coalesced update e(:, j) += x, x in the chunk layout.  The row pass's values
+// ev serve where registers hold them across the solve (one memory round trip
+// less); the 17-cell chunks and the segmented kernels would spill them.
+template <int C, bool SEG>
+constexpr bool keep_values() {
+    return C < 16 && !SEG;
+}
+
 template <int C, int NT, bool SEG = false, typename T>
-__device__ __forceinline__ void row_update_add(const RowCtx<T> &X, T *e, int j, const T *Lx) {
+__device__ __forceinline__ void row_update_add(const RowCtx<T> &X, T *e_, int j, const T *Lx, const T (&ev)[C + 1]) {
+    __attribute__((address_space(1))) T *e = (__attribute__((address_space(1))) T *)e_;
 #pragma unroll
     for (int u = 0; u < C + 1; ++u) {
         const int i = threadIdx.x + NT * u;
-        if (i < X.nx) e[ix(X.P, (SEG ? X.i0 : 0) + i, j)] += Lx[chunk_pos<C>(i, X.rem)];
+        if (i >= X.nx) continue;
+        const size_t c = ix(X.P, (SEG ? X.i0 : 0) + i, j);
+        e[c] = (keep_values<C, SEG>() ? ev[u] : e[c]) + Lx[chunk_pos<C>(i, X.rem)];
     }
 }
 
-// ---------------------------------------------------------------------------
-// Interface solve of the row system, one wave.  The 2 NT interface rows (2
-// per thread of the workgroup; NT = 256: 512, L = 8 per lane; NT = 64: 128,
-// L = 2) sit in LDS lane-major: row q at iface_pos(q) = (q % L) * 64 + q / L,
-// so lane l reads its rows L l .. L l + L-1 without bank conflicts.  Lane l
-//  1. eliminates its L rows to 2 (the partition step of the chunks): its
-//     first row in terms of x(Ll-1), x(Ll), x(Ll+L-1), its last in terms of
-//     x(Ll), x(Ll+L-1), x(Ll+L);
-//  2. takes part in parallel cyclic reduction of those 128 rows (7 steps,
-//     neighbours exchanged with cross-lane shuffles, no barrier);
-//  3. evaluates its L-2 inner unknowns from the first and last ones (their
-//     linear forms were set up in step 1) and writes x(Ll .. Ll+L-1) to X in
-//     natural order.
-// ---------------------------------------------------------------------------
-template <int NT>
-constexpr int iface_rows() {
-    return 2 * NT;  // interface rows, padded
-}
-
-// Quotients of the line solves: v_rcp_f64 refined by one Newton step (error
-// of order eps^2 relative, three dependent instructions instead of the
-// correctly rounded division sequence).  The line solves are part of the
-// preconditioner, so they need accuracy, not bit-exact rounding.
+// Reciprocals of the line solves: v_rcp_f64 (measured error up to 4.4e-8)
+// refined by two Newton steps, which leaves 1.1e-16, an ulp (2e-15 after
+// one).  Each is used for several products, so an error in it would act as
+// a perturbation of the row's diagonal, times the row system's condition.
 __device__ __forceinline__ double rcp(double x) {
-    const double r = __builtin_amdgcn_rcp(x);
+    double r = __builtin_amdgcn_rcp(x);
+    r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
     return __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
 }
 // FP32: v_rcp_f32 alone (about 1 ulp).
 __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
-template <typename T>
-__device__ __forceinline__ T quot(T a, T b) {
-    return a * rcp(b);
-}
-
-template <int NT>
-__device__ __forceinline__ int iface_pos(int q) {
-    constexpr int L = NT / 32;
-    return (q % L) * 64 + q / L;
-}
 
 template <typename T>
 struct Row4 {
     T a, b, c, d;
 };
 
-template <typename T>
-__device__ __forceinline__ Row4<T> shfl_up4(const Row4<T> &r, int s) {
-    return Row4<T>{__shfl_up(r.a, s), __shfl_up(r.b, s), __shfl_up(r.c, s), __shfl_up(r.d, s)};
-}
-template <typename T>
-__device__ __forceinline__ Row4<T> shfl_down4(const Row4<T> &r, int s) {
-    return Row4<T>{__shfl_down(r.a, s), __shfl_down(r.b, s), __shfl_down(r.c, s), __shfl_down(r.d, s)};
+// ---------------------------------------------------------------------------
+// The row system is solved by partition.  A chunk of consecutive rows is
+// eliminated to one row in the last unknowns of the chunks (its own, the
+// previous and the next chunk's): a forward sweep leaves the chunk's last row
+// in terms of the previous chunk's last unknown, its own and the next chunk's
+// first, and the back substitution gives every other unknown of the chunk,
+// the first included, as a linear form G + H x_prev + M x_last.  Each row
+// costs one reciprocal.  What bounds a row is this serial chain and the row
+// pass before it; keeping both ends of each chunk as unknowns took two sweeps,
+// three reciprocals a row and a system of twice the size (single FP64 solves:
+// 64^2 13.54 -> 10.56 ms, 512^2 52.4 -> 43.4, 2048^2 134.7 -> 116.0).
+// ---------------------------------------------------------------------------
+// Rows a x(k-1) + b x(k) + c x(k+1) = d, k = 0 .. len-1 (len = N or N-1 >= 2).
+// On return (a, b, c, d) at row len-1 are the last row's coefficients of
+// x_prev, x_last and the next chunk's first unknown, and its right-hand side;
+// at the rows before, (d, a, c) hold the forms (G, H, M).
+template <int N, bool SHORT, typename T>
+__device__ __forceinline__ void eliminate(T (&a)[N], T (&b)[N], T (&c)[N], T (&d)[N], int len, Row4<T> &last) {
+    T ib[N];
+    ib[0] = rcp(b[0]);
+#pragma unroll
+    for (int k = 1; k < N; ++k)
+        if (!SHORT || k < N - 1 || len == N) {
+            const T r = a[k] * ib[k - 1];
+            a[k] = -r * a[k - 1];
+            b[k] = b[k] - r * c[k - 1];
+            d[k] = d[k] - r * d[k - 1];
+            ib[k] = rcp(b[k]);
+        }
+    const bool full = !SHORT || len == N;
+    last = Row4<T>{full ? a[N - 1] : a[N - 2], full ? b[N - 1] : b[N - 2], full ? c[N - 1] : c[N - 2],
+                   full ? d[N - 1] : d[N - 2]};
+    T G = 0, H = 0, M = 1;
+#pragma unroll
+    for (int k = N - 2; k >= 0; --k)
+        if (!SHORT || k < N - 2 || len == N) {
+            G = (d[k] - c[k] * G) * ib[k];
+            H = (-a[k] - c[k] * H) * ib[k];
+            M = (-c[k] * M) * ib[k];
+            d[k] = G;
+            a[k] = H;
+            c[k] = M;
+        }
 }
 
-// One PCR update of row r from its neighbours m (q - st) and p (q + st);
-// a missing neighbour contributes nothing.
+// The last row with the next chunk's first unknown g + h x_last + m x_next put in.
 template <typename T>
-__device__ __forceinline__ Row4<T> pcr_update(const Row4<T> &r, const Row4<T> &m, bool has_m, const Row4<T> &p,
-                                              bool has_p) {
-    const T k1 = has_m ? quot(r.a, m.b) : T(0), k2 = has_p ? quot(r.c, p.b) : T(0);
-    Row4<T> o;
-    o.a = has_m ? -m.a * k1 : T(0);
-    o.c = has_p ? -p.c * k2 : T(0);
-    o.b = r.b - (has_m ? m.c * k1 : T(0)) - (has_p ? p.a * k2 : T(0));
-    o.d = r.d - (has_m ? m.d * k1 : T(0)) - (has_p ? p.d * k2 : T(0));
-    return o;
+__device__ __forceinline__ Row4<T> join(const Row4<T> &r, T g, T h, T m) {
+    return Row4<T>{r.a, r.b + r.c * h, r.c * m, r.d - r.c * g};
+}
+
+// Solves the 64-row tridiagonal system of one row per lane by parallel cyclic
+// reduction on rows scaled to a unit diagonal (one reciprocal and six
+// shuffles a step); n: rows that are not identity rows.  A lane whose
+// neighbour is missing has a (or c) = 0, so what it is handed does not count.
+template <typename T>
+__device__ __forceinline__ T wave_pcr(const Row4<T> &r, int n) {
+    const T i0 = rcp(r.b);
+    T a = r.a * i0, c = r.c * i0, d = r.d * i0;
+    for (int st = 1; st < n; st *= 2) {
+        const T am = __shfl_up(a, st), cm = __shfl_up(c, st), dm = __shfl_up(d, st);
+        const T ap = __shfl_down(a, st), cp = __shfl_down(c, st), dp = __shfl_down(d, st);
+        const T q = rcp(T(1) - a * cm - c * ap);
+        d = (d - a * dm - c * dp) * q;
+        a = -a * am * q;
+        c = -c * cp * q;
+    }
+    return d;
+}
+
+// Interface solve of a row of more than one wave (NT chunks, one per thread),
+// by the first wave: lane l takes the L = NT / 64 chunks L l .. L l + L - 1,
+// eliminates their rows to one, and the 64 lane rows go through wave_pcr.
+// I: 7 arrays of NT values in LDS (the chunk's last row a, b, c, d and the form
+// G, H, M of its first unknown), chunk t at (t % L) * 64 + t / L, so that a
+// lane's reads are free of bank conflicts; X receives the chunks' last
+// unknowns in order.
+template <int NT>
+__device__ __forceinline__ int iface_pos(int t) {
+    constexpr int L = NT / 64;
+    return (t % L) * 64 + t / L;
 }
 
 template <int NT, typename T>
-__device__ __forceinline__ void interface_solve(T *IA, T *IB, const T *IC, T *ID, T *IX, int l) {
-    constexpr int L = NT / 32;
-    T a[L], b[L], c[L], d[L];
+__device__ __forceinline__ void interface_solve(const T *I, T *X, int nt, int l) {
+    constexpr int L = NT / 64;
+    T a[L], b[L], c[L], d[L], g[L], h[L], m[L];
 #pragma unroll
     for (int k = 0; k < L; ++k) {
         const int q = k * 64 + l;
-        a[k] = IA[q];
-        b[k] = IB[q];
-        c[k] = IC[q];
-        d[k] = ID[q];
+        a[k] = I[q];
+        b[k] = I[NT + q];
+        c[k] = I[2 * NT + q];
+        d[k] = I[3 * NT + q];
+        g[k] = I[4 * NT + q];
+        h[k] = I[5 * NT + q];
+        m[k] = I[6 * NT + q];
     }
-    // 1. partition: first row (backward sweep), last row (forward sweep)
-    T bu = b[L - 2], cu = c[L - 2], du = d[L - 2];
+    const T gn = __shfl_down(g[0], 1), hn = __shfl_down(h[0], 1), mn = __shfl_down(m[0], 1);
 #pragma unroll
-    for (int k = L - 3; k >= 0; --k) {
-        const T r = quot(c[k], bu);
-        bu = b[k] - r * a[k + 1];
-        cu = -r * cu;
-        du = d[k] - r * du;
+    for (int k = 0; k < L; ++k) {
+        const bool end = k == L - 1;
+        const Row4<T> r = join(Row4<T>{a[k], b[k], c[k], d[k]}, end ? gn : g[(k + 1) % L], end ? hn : h[(k + 1) % L],
+                               end ? mn : m[(k + 1) % L]);
+        b[k] = r.b;
+        c[k] = r.c;
+        d[k] = r.d;
     }
-    Row4<T> f{a[0], bu, cu, du};
+    Row4<T> last;
+    eliminate<L, false>(a, b, c, d, L, last);
+    const T gs = __shfl_down(d[0], 1), hs = __shfl_down(a[0], 1), ms = __shfl_down(c[0], 1);
+    const T xe = wave_pcr(join(last, gs, hs, ms), (nt + L - 1) / L);
+    const T xp = __shfl_up(xe, 1);
 #pragma unroll
-    for (int k = 2; k < L; ++k) {
-        const T r = quot(a[k], b[k - 1]);
-        a[k] = -r * a[k - 1];
-        b[k] = b[k] - r * c[k - 1];
-        d[k] = d[k] - r * d[k - 1];
-    }
-    Row4<T> g{a[L - 1], b[L - 1], c[L - 1], d[L - 1]};
-    // inner unknowns as x_k = G_k + H_k x_first + M_k x_last, kept in this
-    // lane's own LDS slots (IA, IB, ID) for step 3, so that the PCR runs with
-    // only the two lane rows in registers and step 3 has no dependent chain
-    {
-        T G = 0, H = 0, M = 1;
-#pragma unroll
-        for (int k = L - 2; k >= 1; --k) {
-            const T ib = rcp(b[k]);
-            G = (d[k] - c[k] * G) * ib;
-            H = (-a[k] - c[k] * H) * ib;
-            M = (-c[k] * M) * ib;
-            const int q = k * 64 + l;
-            IA[q] = G;
-            IB[q] = H;
-            ID[q] = M;
-        }
-    }
-    asm volatile("" ::: "memory");
-    // 2. PCR over the 128 lane rows, Q = 2l (first) and 2l+1 (last)
-#pragma unroll
-    for (int st = 1; st < 128; st *= 2) {
-        Row4<T> fm, fp, gm, gp;
-        if (st == 1) {
-            fm = shfl_up4(g, 1);   // Q-1 of the first row: the previous lane's last
-            fp = g;                // Q+1: this lane's last
-            gm = f;                // Q-1 of the last row: this lane's first
-            gp = shfl_down4(f, 1); // Q+1: the next lane's first
-        } else {
-            const int sl = st / 2;
-            fm = shfl_up4(f, sl);
-            fp = shfl_down4(f, sl);
-            gm = shfl_up4(g, sl);
-            gp = shfl_down4(g, sl);
-        }
-        const int Qf = 2 * l, Qg = 2 * l + 1;
-        const Row4<T> nf = pcr_update(f, fm, Qf - st >= 0, fp, Qf + st < 128);
-        const Row4<T> ng = pcr_update(g, gm, Qg - st >= 0, gp, Qg + st < 128);
-        f = nf;
-        g = ng;
-    }
-    const T xs = quot(f.d, f.b), xe = quot(g.d, g.b);
-    // 3. back substitution of the inner unknowns
-    asm volatile("" ::: "memory");
-    IX[L * l] = xs;
-    IX[L * l + L - 1] = xe;
-#pragma unroll
-    for (int k = 1; k <= L - 2; ++k) {
-        const int q = k * 64 + l;
-        IX[L * l + k] = IA[q] + IB[q] * xs + ID[q] * xe;
-    }
+    for (int k = 0; k < L - 1; ++k) X[L * l + k] = d[k] + a[k] * xp + c[k] * xe;
+    X[L * l + L - 1] = xe;
 }
 
 // ---------------------------------------------------------------------------
-// On-the-fly solve of one row (fine levels, bandwidth-bound): coefficients
-// from the metrics, elimination, PCR and back substitution per call.
-// LDS: 4 nt (C+1) doubles.
+// On-the-fly solve of one row: coefficients from the metrics, elimination,
+// interface solve and back substitution per call.
+// LDS: 4 nt (C+1) elements, or nt (C+1) + 8 NT (rows of more than one wave).
 // ---------------------------------------------------------------------------
 template <int C, int NT, bool SEG = false, int RG = 1, typename T, typename GM>
 __device__ void xline_row(const RowCtx<T> &X, T *__restrict__ e, const T *__restrict__ f, const T *__restrict__ K,
@@ -523,7 +522,8 @@ __device__ void xline_row(const RowCtx<T> &X, T *__restrict__ e, const T *__rest
     const int tid = threadIdx.x, nt = X.nt;
     const int NT1 = nt * CP;
     T *Ld = lds, *Lb = lds + NT1, *La = lds + 2 * NT1, *Lc = lds + 3 * NT1;
-    row_pass<C, NT, SEG, RG>(X, e, f, K, g, geo, j, Ld, La, Lb, Lc);
+    T ev[CP];
+    row_pass<C, NT, SEG, RG>(X, e, f, K, g, geo, j, Ld, La, Lb, Lc, ev);
     __syncthreads();
 
     // each thread takes its chunk into registers
@@ -539,91 +539,48 @@ __device__ void xline_row(const RowCtx<T> &X, T *__restrict__ e, const T *__rest
         }
     __syncthreads();
 
-    // partition elimination in registers
-    // start row:  a_0 x_{prev end} + bu x_s + cu x_e = du
-    // end row:    a'_L x_s + b'_L x_e + c_L x_{next start} = d'_L
-    T ea = 0, eb = 1, ec = 0, ed = 0, oa = 0, ob = 1, oc = 0, od = 0;
-    T sg[CP], sh[CP], sm[CP];
+    // chunks past the row's end are identity rows
+    Row4<T> last{0, 1, 0, 0};
+    T g0 = 0, h0 = 0, m0 = 0;
     if (tid < nt) {
-        const bool longc = len == CP;
-        T bu = longc ? cb[C - 1] : cb[C - 2];
-        T cu = longc ? cc[C - 1] : cc[C - 2];
-        T du = longc ? cd[C - 1] : cd[C - 2];
-#pragma unroll
-        for (int k = C - 2; k >= 0; --k)
-            if (k <= len - 3) {
-                const T r = quot(cc[k], bu);
-                bu = cb[k] - r * ca[k + 1];
-                cu = -r * cu;
-                du = cd[k] - r * du;
-            }
-        ea = ca[0];
-        eb = bu;
-        ec = cu;
-        ed = du;
-#pragma unroll
-        for (int k = 2; k <= C; ++k)
-            if (k <= len - 1) {
-                const T r = quot(ca[k], cb[k - 1]);
-                ca[k] = -r * ca[k - 1];
-                cb[k] = cb[k] - r * cc[k - 1];
-                cd[k] = cd[k] - r * cd[k - 1];
-            }
-        oa = longc ? ca[C] : ca[C - 1];
-        ob = longc ? cb[C] : cb[C - 1];
-        oc = longc ? cc[C] : cc[C - 1];
-        od = longc ? cd[C] : cd[C - 1];
-        // inner unknowns as x_k = sg_k + sh_k x_s + sm_k x_e (the back
-        // substitution unrolled once here, off the critical path of the
-        // interface solve): ca/cb/cc/cd are dead after this
-        T G = 0, H = 0, M = 1;
-#pragma unroll
-        for (int k = C - 1; k >= 1; --k)
-            if (k <= len - 2) {
-                const T ib = rcp(cb[k]);
-                G = (cd[k] - cc[k] * G) * ib;
-                H = (-ca[k] - cc[k] * H) * ib;
-                M = (-cc[k] * M) * ib;
-                sg[k] = G;
-                sh[k] = H;
-                sm[k] = M;
-            }
+        eliminate<CP, true>(ca, cb, cc, cd, len, last);
+        g0 = cd[0];
+        h0 = ca[0];
+        m0 = cc[0];
     }
-
-    // Interface system: the 2 nt chunk-end unknowns (start of chunk t at
-    // q = 2t, end at q = 2t+1; tridiagonal in that order), padded to 512 rows
-    // with identity rows by the threads past nt.  Staged once through LDS,
-    // solved by wave 0 (interface_solve), read back once: two barriers.
-    constexpr int IFACE = iface_rows<NT>();
-    T *IA = lds + NT1, *IB = IA + IFACE, *IC = IB + IFACE, *ID = IC + IFACE, *IX = ID + IFACE;
-    {
-        const int q0 = iface_pos<NT>(2 * tid), q1 = iface_pos<NT>(2 * tid + 1);
-        IA[q0] = ea;
-        IB[q0] = eb;
-        IC[q0] = ec;
-        ID[q0] = ed;
-        IA[q1] = oa;
-        IB[q1] = ob;
-        IC[q1] = oc;
-        ID[q1] = od;
+    T xe, xp;
+    if (NT == 64) {
+        const T gn = __shfl_down(g0, 1), hn = __shfl_down(h0, 1), mn = __shfl_down(m0, 1);
+        xe = wave_pcr(join(last, gn, hn, mn), nt);
+        xp = __shfl_up(xe, 1);
+    } else {
+        // staged once through LDS, solved by wave 0, read back once: two barriers
+        T *I = lds + NT1, *IX = I + 7 * NT;
+        const int q = iface_pos<NT>(tid);
+        I[q] = last.a;
+        I[NT + q] = last.b;
+        I[2 * NT + q] = last.c;
+        I[3 * NT + q] = last.d;
+        I[4 * NT + q] = g0;
+        I[5 * NT + q] = h0;
+        I[6 * NT + q] = m0;
+        __syncthreads();
+        if (tid < 64) interface_solve<NT>(I, IX, nt, tid);
+        __syncthreads();
+        xe = IX[tid];
+        xp = tid ? IX[tid - 1] : T(0);
     }
-    __syncthreads();
-    if (tid < 64) interface_solve<NT>(IA, IB, IC, ID, IX, tid);
-    __syncthreads();
-    const T x_start = IX[2 * tid], x_end = IX[2 * tid + 1];
 
     // back substitution, then the coalesced update
     if (tid < nt) {
-        const T xs = x_start, xe = x_end;
         const bool longc = len == CP;
 #pragma unroll
-        for (int k = 1; k <= C - 1; ++k)
-            if (k <= len - 2) lds[tid * CP + k] = sg[k] + sh[k] * xs + sm[k] * xe;
-        lds[tid * CP] = xs;
+        for (int k = 0; k <= C - 1; ++k)
+            if (k <= len - 2) lds[tid * CP + k] = cd[k] + ca[k] * xp + cc[k] * xe;
         lds[tid * CP + (longc ? C : C - 1)] = xe;
     }
     __syncthreads();
-    row_update_add<C, NT, SEG>(X, e, j, lds);
+    row_update_add<C, NT, SEG>(X, e, j, lds, ev);
 }
 
 // Rows j = row0 + slot*rowstep; the workgroup of slot 0 then also relaxes
@@ -908,8 +865,8 @@ size_t xline_lds_bytes(int nx, size_t elem) { return xline_lds_bytes_for(nx, xli
 size_t xline_lds_bytes_for(int nx, int C, size_t elem, int threads) {
     if (C == 0) return (size_t)-1;
     const size_t nt = (size_t)(nx / C);
-    // chunk staging (4 arrays), or one chunk array plus the interface rows
-    const size_t tr = 4 * nt * (C + 1), iface = nt * (C + 1) + 5 * 2 * (size_t)threads;
+    // chunk staging (4 arrays), or one chunk array plus the interface rows and unknowns
+    const size_t tr = 4 * nt * (C + 1), iface = nt * (C + 1) + (threads > 64 ? 8 * (size_t)threads : 0);
     return (tr > iface ? tr : iface) * elem;
 }
 
