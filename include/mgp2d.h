@@ -98,8 +98,8 @@ int mgp_compute_invdiags(const mgp_geo *geo, const mgp_bc *bc, int homog, double
  * ordering MGP_ORDER_LEX (reference order) or MGP_ORDER_MC. */
 int mgp_relax_gs(const mgp_geo *geo, const mgp_bc *bc, int homog, const double *invd, double omega,
                  int maxiters, const double *rhs, double *phi, int ordering);
-/* x-line zebra relaxation, the smoother of MGP_METHOD_KRYLOV_MG (no counterpart in the
- * reference): each sweep solves, row by row, T_j delta = rhs - L phi and adds delta, where L is
+/* x-line zebra relaxation (no counterpart in the reference; the smoother of MGP_METHOD_KRYLOV_MG is
+ * the same with rows 0 and ny-1 relaxed with the other rows of their parity): each sweep solves, row by row, T_j delta = rhs - L phi and adds delta, where L is
  * the reference operator with homogeneous BCs and T_j its tridiagonal part along row j; even
  * interior rows, then odd ones, then rows 0 and ny-1.  Dirichlet/Neumann sides, nx, ny >= 4;
  * phi's ghost cells are neither read nor written.  Rows over 4111 cells are cut into 2, 4, ..

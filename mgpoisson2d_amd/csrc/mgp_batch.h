@@ -26,6 +26,7 @@ struct BLev {
     double *e[2];
     double *f[2];
     const double *K;    // ring stencil table
+    double *far;        // far rows of the line relaxation: lo, hi (XlFar)
     double slo, shi;    // ghost signs of the y sides in the prolongation
     int prob, nt;       // problem index; x-line chunks (nx / C)
     int off;            // the fine row of the next coarser level's row 0 (semicoarsen_step)
@@ -35,7 +36,7 @@ struct BLev {
     // applications of an iteration run one after the other)
     GeoF geo32;
     const float *K32;
-    float *e32, *f32;
+    float *e32, *f32, *far32;
 };
 
 // Krylov vectors of one problem (finest level, level layout).
@@ -52,10 +53,10 @@ struct BProb {
     int lev0;          // index of the finest level in the level table
 };
 
-// Row task: row `row` of level `lev`, then row `extra` (< 0: none) by the
-// same workgroup (the boundary-row fold of the single-problem sweep).
+// Row task: relax row `row` of level `lev`, or (save) copy it into the level's
+// far rows (side 0: lo, 1: hi).
 struct XlTask {
-    int lev, row, extra, pad;
+    int lev, row, side, save;
 };
 
 // Cell tile: cells (64 tx .. 64 tx + 63, BT_ROWS ty .. BT_ROWS ty + 15) of

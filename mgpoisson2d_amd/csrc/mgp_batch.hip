@@ -165,7 +165,8 @@ __global__ void k_b_scalars(const BProb *P, const int *mask, int n, int op) {
 //  0: p = r + beta (p - omega v)   1: s = r - alpha v   2: phi += alpha phat
 //  3: phi += omega shat            4: r = s - omega t
 // With L (FP32 cycles), ops 0 and 1 also start the cycle that preconditions
-// the vector they produce: the finest level's f32 = (float) p or s, e32 = 0.
+// the vector they produce: the finest level's f32 = (float) p or s, e32 = 0
+// (and its far rows).
 __global__ void __launch_bounds__(256) k_b_update(const BTile *tiles, const BProb *P, const int *mask, int op,
                                                   const BLev *L) {
     const BTile t = tiles[blockIdx.x];
@@ -176,6 +177,7 @@ __global__ void __launch_bounds__(256) k_b_update(const BTile *tiles, const BPro
     double *const *v = p->v;
     const double alpha = sc[SC_ALPHA], beta = sc[SC_BETA], omega = sc[SC_OMEGA];
     float *f32 = L ? L[p->lev0].f32 : nullptr, *e32 = L ? L[p->lev0].e32 : nullptr;
+    float *far = L ? L[p->lev0].far32 : nullptr;
     tile_cells(t, g, [&](int i, int j) {
         const size_t c = ix(g.pitch, i, j);
         double out;
@@ -189,6 +191,7 @@ __global__ void __launch_bounds__(256) k_b_update(const BTile *tiles, const BPro
         if (f32 && op <= 1) {
             f32[c] = (float)out;
             e32[c] = 0.0f;
+            if (j < 2) far[j * g.pitch + OFFX + i] = 0.0f;
         }
     });
 }
@@ -204,6 +207,20 @@ __global__ void __launch_bounds__(256) k_b_copy(const BTile *tiles, const BProb 
     tile_cells(t, g, [&](int i, int j) {
         const size_t c = ix(g.pitch, i, j);
         d[c] = sv ? sv[c] : 0.0;
+    });
+}
+
+// Start of an FP64 cycle: v[PHAT or SHAT] = 0, and the finest level's far rows.
+__global__ void __launch_bounds__(256) k_b_begin(const BTile *tiles, const BProb *P, const BLev *L, const int *mask,
+                                                 int sel) {
+    const BTile t = tiles[blockIdx.x];
+    if (!mask[t.item]) return;
+    const BProb *p = P + t.item;
+    const Grid g = p->g;
+    double *e = p->v[sel ? BV_SHAT : BV_PHAT], *far = L[p->lev0].far;
+    tile_cells(t, g, [&](int i, int j) {
+        e[ix(g.pitch, i, j)] = 0.0;
+        if (j < 2) far[j * g.pitch + OFFX + i] = 0.0;
     });
 }
 
@@ -273,6 +290,7 @@ size_t BatchKMG::problem_bytes(const Problem &q, const mgp_solver_opts &o) {
         const size_t nl = level_elems(q.nx, ny);
         b += 5 * round256(nl * sizeof(double));
         if (lev) b += 2 * round256(nl * sizeof(double));
+        b += round256((size_t)2 * level_pitch(q.nx) * (mx ? sizeof(float) : sizeof(double)));
         const Grid gl = make_grid(q.nx, ny, q.dx, q.dy);
         b += round256((size_t)ring_table_elems(gl) * sizeof(double));
         if (mx) {
@@ -328,7 +346,7 @@ BatchKMG::BatchKMG(hipStream_t s_, const std::vector<Problem> &probs, const mgp_
     };
     struct Off {
         size_t v[BV_COUNT], partial;
-        std::vector<size_t> J, Jxx, Jxy, Jyx, Jyy, e, r, K;
+        std::vector<size_t> J, Jxx, Jxy, Jyx, Jyy, e, r, K, far;
         std::vector<size_t> f32m[4], K32, e32, r32;  // FP32 copies (mixed precision)
     };
     std::vector<Off> off(n);
@@ -349,6 +367,7 @@ BatchKMG::BatchKMG(hipStream_t s_, const std::vector<Problem> &probs, const mgp_
             O.Jyy.push_back(take(nl));
             O.e.push_back(lev ? take(nl) : 0);
             O.r.push_back(lev ? take(nl) : 0);
+            O.far.push_back(take((size_t)2 * level_pitch(q.nx), mixed ? sizeof(float) : sizeof(double)));
             const Grid gl = make_grid(q.nx, ny, q.dx, q.dy);
             O.K.push_back(take((size_t)ring_table_elems(gl)));
             if (mixed) {
@@ -432,7 +451,8 @@ BatchKMG::BatchKMG(hipStream_t s_, const std::vector<Problem> &probs, const mgp_
             l.K = at(O.K[d]);
             l.geo32 = GeoF{nullptr, nullptr, nullptr, nullptr, nullptr};
             l.K32 = nullptr;
-            l.e32 = l.f32 = nullptr;
+            l.e32 = l.f32 = l.far32 = nullptr;
+            l.far = mixed ? nullptr : at(O.far[d]);
             if (mixed) {
                 // FP32 copies of the whole padded arrays (formed in FP64, rounded once)
                 const size_t nl = level_elems(q.nx, ny);
@@ -443,6 +463,7 @@ BatchKMG::BatchKMG(hipStream_t s_, const std::vector<Problem> &probs, const mgp_
                 l.K32 = atf(O.K32[d]);
                 l.e32 = atf(O.e32[d]);
                 l.f32 = atf(O.r32[d]);
+                l.far32 = atf(O.far[d]);
             }
             l.slo = B.bc.type[YLO] == BC_DIRI ? -1.0 : 1.0;
             l.shi = B.bc.type[YHI] == BC_DIRI ? -1.0 : 1.0;
@@ -539,28 +560,13 @@ void BatchKMG::build_tables(TableSet &ts, const std::vector<int> &which) {
                 b = std::max(b, need);
                 return tabs[key];
             };
-            // the order of xline_zebra: even interior rows, odd interior rows
-            // (the first and last relaxing rows 0 and ny-1 after their own),
-            // else rows 0 and ny-1 in a launch of their own
-            const int n_even = ny >= 4 ? (ny - 4) / 2 + 1 : 0;
-            const int n_odd = ny >= 3 ? (ny - 3) / 2 + 1 : 0;
-            if (n_even) {
-                std::vector<XlTask> &v = table(0);
-                for (int k = 0; k < n_even; ++k) v.push_back(XlTask{lev, 2 + 2 * k, -1, 0});
-            }
-            if (n_odd) {
-                std::vector<XlTask> &v = table(1);
-                for (int k = 0; k < n_odd; ++k) {
-                    int extra = -1;
-                    if (n_odd >= 2 && k == 0) extra = 0;
-                    if (n_odd >= 2 && k == n_odd - 1) extra = ny - 1;
-                    v.push_back(XlTask{lev, 1 + 2 * k, extra, 0});
-                }
-            }
-            if (n_odd < 2) {
-                std::vector<XlTask> &v = table(2);
-                v.push_back(XlTask{lev, 0, -1, 0});
-                v.push_back(XlTask{lev, ny - 1, -1, 0});
+            // the order of the single-problem sweep: even rows, odd rows, each
+            // launch saving the far rows of the other colour
+            for (int colour = 0; colour < 2; ++colour) {
+                std::vector<XlTask> &v = table(colour);
+                for (int j = colour; j < ny; j += 2) v.push_back(XlTask{lev, j, 0, 0});
+                if (colour == 1) v.push_back(XlTask{lev, 2, 0, 1});
+                if (((ny - 3) & 1) != colour) v.push_back(XlTask{lev, ny - 3, 1, 1});
             }
             if (set == SET_MID) {
                 tiles_of(trh, lev, nx, L[lev + 1].g.ny);
@@ -664,7 +670,7 @@ BatchKMG::~BatchKMG() {
 }
 
 void BatchKMG::zebra(int d, int set, int sel, int k) {
-    for (int colour = 0; colour < 3; ++colour) {
+    for (int colour = 0; colour < 2; ++colour) {
         std::vector<const XlTable *> tabs;
         for (const XlTable &x : T->xl)
             if (x.d == d && x.set == set && x.colour == colour) tabs.push_back(&x);
@@ -694,7 +700,7 @@ void BatchKMG::zebra(int d, int set, int sel, int k) {
 void BatchKMG::precondition(int sel) {
     // FP32 cycles: the update that produced p or s has set the finest
     // level's f32 and zeroed its e32 (k_b_update with the level table)
-    if (!mixed) k_b_copy<<<T->t0.n, 256, 0, s>>>((const BTile *)T->t0.p, dP, active, sel ? BV_SHAT : BV_PHAT, -1);
+    if (!mixed) k_b_begin<<<T->t0.n, 256, 0, s>>>((const BTile *)T->t0.p, dP, dL, active, sel);
     const int depth = T->depth;
     for (int d = 0; d < depth; ++d) {
         for (int k = 0; k < sd; ++k) zebra(d, SET_MID, sel, -1);
@@ -892,7 +898,8 @@ double BatchKMG::time_fine_xline(int reps, double *bytes) {
         T = &full;
     }
     const int n = count();
-    // the even interior rows of level 0 (colour 0 of the first zebra phase)
+    // the even rows of level 0 (colour 0 of the first zebra phase; the bytes
+    // count its interior rows)
     std::vector<const XlTable *> tabs;
     for (const XlTable &x : T->xl)
         if (x.d == 0 && x.set == SET_MID && x.colour == 0) tabs.push_back(&x);
@@ -1019,7 +1026,7 @@ double BatchKMG::time_shapes(const std::vector<int> &C, const std::vector<int> &
         L[lev].nt = nx / C[p];
         if (ny < 4) continue;
         auto &t = cls[{C[p], NT[p]}];
-        for (int k = 0; k < (ny - 4) / 2 + 1; ++k) t.push_back(XlTask{lev, 2 + 2 * k, -1, 0});
+        for (int k = 0; k < (ny - 4) / 2 + 1; ++k) t.push_back(XlTask{lev, 2 + 2 * k, 0, 0});
         size_t &l = lds[{C[p], NT[p]}];
         l = std::max(l, xline_lds_bytes_for(nx, C[p], elem, NT[p]));
     }

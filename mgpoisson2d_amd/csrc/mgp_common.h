@@ -57,6 +57,20 @@ struct Geo4 {
     const double *A4, *Bx4, *dA, *dBx, *C4, *By4, *dC, *dBy;
 };
 
+// The far rows of a level's x-line relaxation.  A boundary row's extrapolated
+// stencil reaches two rows in, to a row of its own colour: row 0 reads row 2,
+// row ny-1 row ny-3.  So that a boundary row can be relaxed beside the other
+// rows of its colour, it reads that row's values from before the launch from a
+// copy, lo (row 2) or hi (row ny-3), cell i at [OFFX + i].  A launch saves the
+// rows of the other colour, which it does not change, for the next one: row
+// save[k] (< 0: none) into to[k].
+template <typename T>
+struct XlFar {
+    const T *lo, *hi;
+    T *to[2];
+    int save[2];
+};
+
 // Boundary description as the kernels see it.  val[] is the UNIFORM value;
 // data[] points at device NONUNIFORM face data (ny values for x sides, nx for
 // y sides) or is null.
@@ -76,23 +90,29 @@ __host__ __device__ inline size_t ix(int pitch, int i, int j) {
 // neighbour on j's side (J-1 for even j, J+1 for odd j; weight 1/4); beyond a
 // y side the neighbour is the ghost slo*c / shi*c (Neumann: sign +1,
 // reflected; Dirichlet: sign -1, negated).  ef += the interpolated coarse
-// correction.
+// correction.  far: the fine level's copies of rows 2 and ny-3 (XlFar: lo,
+// then hi one pitch on), kept up to date.
 template <typename T>
-__device__ __forceinline__ void prolong_y_cell(T *ef, const T *ec, const Grid &gf, const Grid &gc, T slo, T shi,
-                                               int i, int j, int off = 0) {
+__device__ __forceinline__ void prolong_y_cell(T *ef, const T *ec, T *far, const Grid &gf, const Grid &gc, T slo,
+                                               T shi, int i, int j, int off = 0) {
     const int jc = j - off;  // row within the coarse grid's fine rows
+    T add;
     if (jc < 0 || jc >= 2 * gc.ny) {
         // a row the coarsening left out (at a Neumann side): the correction
         // of the coarse row next to it
-        ef[ix(gf.pitch, i, j)] += ec[ix(gc.pitch, i, jc < 0 ? 0 : gc.ny - 1)];
-        return;
+        add = ec[ix(gc.pitch, i, jc < 0 ? 0 : gc.ny - 1)];
+    } else {
+        const int J = jc >> 1;
+        const T c = ec[ix(gc.pitch, i, J)];
+        T nb;
+        if (jc & 1) nb = J + 1 < gc.ny ? ec[ix(gc.pitch, i, J + 1)] : shi * c;
+        else nb = J - 1 >= 0 ? ec[ix(gc.pitch, i, J - 1)] : slo * c;
+        add = T(0.75) * c + T(0.25) * nb;
     }
-    const int J = jc >> 1;
-    const T c = ec[ix(gc.pitch, i, J)];
-    T nb;
-    if (jc & 1) nb = J + 1 < gc.ny ? ec[ix(gc.pitch, i, J + 1)] : shi * c;
-    else nb = J - 1 >= 0 ? ec[ix(gc.pitch, i, J - 1)] : slo * c;
-    ef[ix(gf.pitch, i, j)] += T(0.75) * c + T(0.25) * nb;
+    const T v = ef[ix(gf.pitch, i, j)] + add;
+    ef[ix(gf.pitch, i, j)] = v;
+    if (j == 2) far[OFFX + i] = v;
+    if (j == gf.ny - 3) far[gf.pitch + OFFX + i] = v;
 }
 
 }  // namespace mgp

@@ -107,11 +107,12 @@ void launch_bicgstab2(hipStream_t s, const BottomArgs &a);
 // Ring-cell stencil table of the homogeneous operator: ring_table_elems(g) doubles.
 int ring_table_elems(const Grid &g);
 void launch_ring_coef(hipStream_t s, double *K, const Grid &g, const Geo &geo, const Bc &bc);
-// rc = 1x2 (y) average of the fine residual f - L e (table at ring cells); ec = 0.
-void launch_residual_restrict_y(hipStream_t s, double *rc, double *ec, const double *e, const double *f,
+// rc = 1x2 (y) average of the fine residual f - L e (table at ring cells); ec = 0
+// and its far rows (farc).
+void launch_residual_restrict_y(hipStream_t s, double *rc, double *ec, double *farc, const double *e, const double *f,
                                 const double *K, const Grid &gf, const Grid &gc, const Geo &geo, int off = 0);
 // FP32 form (mixed-precision preconditioner): same layout and formulas.
-void launch_residual_restrict_y(hipStream_t s, float *rc, float *ec, const float *e, const float *f, const float *K,
+void launch_residual_restrict_y(hipStream_t s, float *rc, float *ec, float *farc, const float *e, const float *f, const float *K,
                                 const Grid &gf, const Grid &gc, const GeoF &geo, int off = 0);
 // Flexible GMRES vector kernels (mgp_gmres.hip); V holds vectors i < nv at
 // V + i * stride (padded level layout, valid cells only).
@@ -187,29 +188,32 @@ int xline_batch_chunk(int nx, int threads, size_t elem);
 size_t xline_lds_bytes(int nx, size_t elem);
 // the same for chunk length C and `threads` threads per row
 size_t xline_lds_bytes_for(int nx, int C, size_t elem, int threads);
-// Relax rows j = row0 + k*rowstep, k < nrows (one workgroup each; no row of a
-// launch may read another: interior rows at least two apart, boundary rows
-// three).  The first workgroup then also relaxes row extra0, the last one row
-// extra1 (< 0: none), each after its own row.
+// Relax rows j = row0 + k*rowstep, k < nrows (one workgroup each; interior
+// rows of a launch are at least two apart, so none reads another).  far: the
+// copies that rows 0 and ny-1 read their far row from, and the rows this
+// launch saves.  part: of rows in segments, the even segments (0) or the odd
+// ones (1) alone; whole rows are part 0.
 void launch_xline(hipStream_t s, double *e, const double *f, const double *K, const Grid &g, const Geo &geo,
-                  int row0, int rowstep, int nrows, int extra0, int extra1);
+                  int row0, int rowstep, int nrows, const XlFar<double> &far, int part = -1);
 void launch_xline(hipStream_t s, float *e, const float *f, const float *K, const Grid &g, const GeoF &geo, int row0,
-                  int rowstep, int nrows, int extra0, int extra1);
+                  int rowstep, int nrows, const XlFar<float> &far);
+// Start of a V-cycle: e = 0 over valid and ghost cells, and its far rows.
+void launch_begin(hipStream_t s, double *e, double *far, const Grid &g);
+void launch_begin(hipStream_t s, float *e, float *far, const Grid &g);
 // ef += 1x2 (y) prolongation of ec (prolong_y_cell); off: the fine row of
 // coarse row 0's first row (semicoarsen_step)
-void launch_prolong_y(hipStream_t s, double *ef, const double *ec, const Grid &gf, const Grid &gc, double slo,
-                      double shi, int off = 0);
-void launch_prolong_y(hipStream_t s, float *ef, const float *ec, const Grid &gf, const Grid &gc, double slo,
-                      double shi, int off = 0);
+void launch_prolong_y(hipStream_t s, double *ef, const double *ec, double *far, const Grid &gf, const Grid &gc,
+                      double slo, double shi, int off = 0);
+void launch_prolong_y(hipStream_t s, float *ef, const float *ec, float *far, const Grid &gf, const Grid &gc,
+                      double slo, double shi, int off = 0);
 // Precision conversions over a level array.  ghosted: also the ghost ring.
-void launch_setval(hipStream_t s, float *y, float v, const Grid &g, int ghosted);
 void launch_convert(hipStream_t s, float *out, const double *in, const Grid &g, int ghosted);
 void launch_convert(hipStream_t s, double *out, const float *in, const Grid &g, int ghosted);
 // out[k] = (float)in[k], k < n (flat arrays: stencil tables, whole padded levels)
 void launch_convert_flat(hipStream_t s, float *out, const double *in, size_t n);
 // Start of an FP32 V-cycle: f32 = (float)f over valid cells, e32 = 0 over
-// valid and ghost cells.
-void launch_begin32(hipStream_t s, float *f32, float *e32, const double *f, const Grid &g);
+// valid and ghost cells, and its far rows.
+void launch_begin32(hipStream_t s, float *f32, float *e32, float *far, const double *f, const Grid &g);
 void launch_axpbypcz(hipStream_t s, double *out, double a, const double *x, double b, const double *y, double c,
                      const double *z, const Grid &g);
 

@@ -1130,11 +1130,12 @@ namespace mgp {
 
 // y-direction prolongation for 1x2 semicoarsening (prolong_y_cell).
 template <typename T>
-__global__ void __launch_bounds__(256) k_prolong_y(T *ef, const T *ec, Grid gf, Grid gc, T slo, T shi, int off) {
+__global__ void __launch_bounds__(256) k_prolong_y(T *ef, const T *ec, T *far, Grid gf, Grid gc, T slo, T shi,
+                                                   int off) {
     const int i = blockIdx.x * 64 + (threadIdx.x & 63);
     const int j = blockIdx.y * 4 + (threadIdx.x >> 6);
     if (i >= gf.nx || j >= gf.ny) return;
-    prolong_y_cell(ef, ec, gf, gc, slo, shi, i, j, off);
+    prolong_y_cell(ef, ec, far, gf, gc, slo, shi, i, j, off);
 }
 
 template <typename TO, typename TI>
@@ -1152,20 +1153,22 @@ __global__ void __launch_bounds__(256) k_convert_flat(float *out, const double *
     if (k < n) out[k] = (float)in[k];
 }
 
-__global__ void __launch_bounds__(256) k_setval_f(float *y, float v, Grid g, int ghosted) {
-    const int o = ghosted ? 1 : 0;
-    const int i = blockIdx.x * 64 + (threadIdx.x & 63) - o;
-    const int j = blockIdx.y * 4 + (threadIdx.x >> 6) - o;
-    if (i >= g.nx + o || j >= g.ny + o) return;
-    y[ix(g.pitch, i, j)] = v;
+template <typename T>
+__global__ void __launch_bounds__(256) k_begin(T *e, T *far, Grid g) {
+    const int i = blockIdx.x * 64 + (threadIdx.x & 63) - 1;
+    const int j = blockIdx.y * 4 + (threadIdx.x >> 6) - 1;
+    if (i > g.nx || j > g.ny) return;
+    e[ix(g.pitch, i, j)] = T(0);
+    if (j == 0 || j == 1) far[j * g.pitch + OFFX + i] = T(0);
 }
 
-__global__ void __launch_bounds__(256) k_begin32(float *f32, float *e32, const double *f, Grid g) {
+__global__ void __launch_bounds__(256) k_begin32(float *f32, float *e32, float *far, const double *f, Grid g) {
     const int i = blockIdx.x * 64 + (threadIdx.x & 63) - 1;
     const int j = blockIdx.y * 4 + (threadIdx.x >> 6) - 1;
     if (i > g.nx || j > g.ny) return;
     const size_t c = ix(g.pitch, i, j);
     e32[c] = 0.0f;
+    if (j == 0 || j == 1) far[j * g.pitch + OFFX + i] = 0.0f;
     if (i >= 0 && i < g.nx && j >= 0 && j < g.ny) f32[c] = (float)f[c];
 }
 
@@ -1395,18 +1398,20 @@ void launch_bicgstab2(hipStream_t s, const BottomArgs &a) {
 }  // namespace mgp
 
 namespace mgp {
-void launch_prolong_y(hipStream_t s, double *ef, const double *ec, const Grid &gf, const Grid &gc, double slo,
-                      double shi, int off) {
-    k_prolong_y<<<tiles(gf.nx, gf.ny), 256, 0, s>>>(ef, ec, gf, gc, slo, shi, off);
+void launch_prolong_y(hipStream_t s, double *ef, const double *ec, double *far, const Grid &gf, const Grid &gc,
+                      double slo, double shi, int off) {
+    k_prolong_y<<<tiles(gf.nx, gf.ny), 256, 0, s>>>(ef, ec, far, gf, gc, slo, shi, off);
 }
-void launch_prolong_y(hipStream_t s, float *ef, const float *ec, const Grid &gf, const Grid &gc, double slo,
-                      double shi, int off) {
-    k_prolong_y<<<tiles(gf.nx, gf.ny), 256, 0, s>>>(ef, ec, gf, gc, (float)slo, (float)shi, off);
+void launch_prolong_y(hipStream_t s, float *ef, const float *ec, float *far, const Grid &gf, const Grid &gc,
+                      double slo, double shi, int off) {
+    k_prolong_y<<<tiles(gf.nx, gf.ny), 256, 0, s>>>(ef, ec, far, gf, gc, (float)slo, (float)shi, off);
 }
 
-void launch_setval(hipStream_t s, float *y, float v, const Grid &g, int ghosted) {
-    const int o = ghosted ? 2 : 0;
-    k_setval_f<<<tiles(g.nx + o, g.ny + o), 256, 0, s>>>(y, v, g, ghosted);
+void launch_begin(hipStream_t s, double *e, double *far, const Grid &g) {
+    k_begin<<<tiles(g.nx + 2, g.ny + 2), 256, 0, s>>>(e, far, g);
+}
+void launch_begin(hipStream_t s, float *e, float *far, const Grid &g) {
+    k_begin<<<tiles(g.nx + 2, g.ny + 2), 256, 0, s>>>(e, far, g);
 }
 
 void launch_convert(hipStream_t s, float *out, const double *in, const Grid &g, int ghosted) {
@@ -1424,8 +1429,8 @@ void launch_convert_flat(hipStream_t s, float *out, const double *in, size_t n) 
     k_convert_flat<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(out, in, n);
 }
 
-void launch_begin32(hipStream_t s, float *f32, float *e32, const double *f, const Grid &g) {
-    k_begin32<<<tiles(g.nx + 2, g.ny + 2), 256, 0, s>>>(f32, e32, f, g);
+void launch_begin32(hipStream_t s, float *f32, float *e32, float *far, const double *f, const Grid &g) {
+    k_begin32<<<tiles(g.nx + 2, g.ny + 2), 256, 0, s>>>(f32, e32, far, f, g);
 }
 void launch_axpbypcz(hipStream_t s, double *out, double a, const double *x, double b, const double *y, double c,
                      const double *z, const Grid &g) {

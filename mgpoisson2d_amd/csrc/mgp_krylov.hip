@@ -9,8 +9,7 @@
 // Preconditioner: one V-cycle on a hierarchy coarsened in y only (1x2, the
 // reference's restrict supports any ratio, MGPoisson2D.f90:145-158), each
 // level re-discretised from restricted metrics with the reference stencil,
-// x-line zebra relaxation (even rows, odd rows, then the two boundary rows,
-// whose extrapolated cross terms reach two rows in), 1x2 averaging
+// x-line zebra relaxation (even rows, then odd rows; zebra() below), 1x2 averaging
 // restriction and linear-in-y prolongation (new: the reference has no
 // semicoarsened prolongation, MGPoisson2D.f90:385-388).
 //
@@ -69,8 +68,8 @@ struct KLevel {
     Geo geo;
     GeoF geo32;
     Bc bc;
-    DevBuf J, Jxx, Jxy, Jyx, Jyy, e, r, w, K;
-    DevBufF Jxx32, Jxy32, Jyx32, Jyy32, e32, r32, K32;  // mixed precision only
+    DevBuf J, Jxx, Jxy, Jyx, Jyy, e, r, w, K, far;
+    DevBufF Jxx32, Jxy32, Jyx32, Jyy32, e32, r32, K32, far32;  // mixed precision only
 };
 
 struct KrylovMG::Impl {
@@ -220,6 +219,8 @@ void KrylovMG::build(hipStream_t s, const DevGeo &top, const Bc &user_bc, const 
         if (!mixed || L.size() == 1)
             for (DevBuf *b : {&l.e, &l.r, &l.w}) b->alloc(n);
         l.K.alloc((size_t)ring_table_elems(l.g));
+        if (mixed) l.far32.alloc((size_t)2 * l.g.pitch);
+        else l.far.alloc((size_t)2 * l.g.pitch);
         l.bc = mg_bc(bc0, MODE_UNIFORM);
         const size_t bytes = n * sizeof(double);
         if (L.size() == 1 && tr) {
@@ -293,34 +294,45 @@ void KrylovMG::build(hipStream_t s, const DevGeo &top, const Bc &user_bc, const 
     built = true;
 }
 
+// One zebra sweep of a level: the even rows, then the odd ones, the boundary
+// rows with their colour.  Rows of a colour do not read one another, except
+// that rows 0 and ny-1 reach two rows in, to a row of their own colour: they
+// read it as the launch found it, from the far copies, which the launch of the
+// other colour has saved (the transfers keep them up to date between the
+// blocks of sweeps).  The line kernel never reads ghosts (ring cells use the
+// level's stencil table, which folds the Dirichlet ghost rule in).
+//
+// Relaxing rows 0 and ny-1 after their neighbours, on the values of both, puts
+// two row solves one after the other into the odd-row launch, and a coarse
+// level's launch takes as long as its longest workgroup.  Solves took as many
+// V-cycles either way (64^2 32 against 40, 512^2 60 against 58, 2048^2 62
+// against 58); 64^2 10.56 -> 6.95 ms, 512^2 43.4 -> 37.5, 2048^2 116.0 -> 104.0.
 template <typename T, typename G>
-static void zebra(hipStream_t s, const Grid &g, const G &geo, const T *K, T *e, const T *f) {
+static void zebra(hipStream_t s, const Grid &g, const G &geo, const T *K, T *e, const T *f, T *far) {
     const int ny = g.ny;
-    // Even interior rows 2, 4, .. <= ny-2, then odd interior rows 1, 3, ..
-    // <= ny-2, then rows 0 and ny-1 (whose extrapolated stencils reach two
-    // rows in).  With two or more odd rows, the first odd-row workgroup relaxes
-    // row 0 after row 1 and the last one row ny-1 after its own: the same
-    // order without a third launch.  The line kernel never reads ghosts (ring
-    // cells use the level's stencil table, which folds the Dirichlet ghost
-    // rule in).
-    const int n_even = ny >= 4 ? (ny - 4) / 2 + 1 : 0;
-    const int n_odd = ny >= 3 ? (ny - 3) / 2 + 1 : 0;
-    launch_xline(s, e, f, K, g, geo, 2, 2, n_even, -1, -1);
-    if (n_odd >= 2) {
-        launch_xline(s, e, f, K, g, geo, 1, 2, n_odd, 0, ny - 1);
-    } else {
-        launch_xline(s, e, f, K, g, geo, 1, 2, n_odd, -1, -1);
-        launch_xline(s, e, f, K, g, geo, 0, ny - 1, 2, -1, -1);
-    }
+    const bool odd = ny & 1;
+    T *lo = far, *hi = far + g.pitch;
+    launch_xline(s, e, f, K, g, geo, 0, 2, (ny + 1) / 2, XlFar<T>{lo, hi, {lo, hi}, {-1, odd ? -1 : ny - 3}});
+    launch_xline(s, e, f, K, g, geo, 1, 2, ny / 2, XlFar<T>{lo, hi, {lo, hi}, {2, odd ? ny - 3 : -1}});
 }
 
 void xline_zebra(hipStream_t s, const Grid &g, const Geo &geo, const double *K, double *e, const double *f) {
-    zebra(s, g, geo, K, e, f);
+    // even interior rows, odd ones, then rows 0 and ny-1 on the values of both
+    // (of rows in segments, each parity's boundary segments after its odd rows')
+    const int ny = g.ny, n_odd = ny >= 3 ? (ny - 3) / 2 + 1 : 0;
+    const XlFar<double> now{e + ix(g.pitch, -OFFX, 2), e + ix(g.pitch, -OFFX, ny - 3), {nullptr, nullptr}, {-1, -1}};
+    launch_xline(s, e, f, K, g, geo, 2, 2, ny >= 4 ? (ny - 4) / 2 + 1 : 0, now);
+    for (int part = n_odd >= 2 ? 0 : -1; part < (n_odd >= 2 ? 2 : 0); ++part) {
+        launch_xline(s, e, f, K, g, geo, 1, 2, n_odd, now, part);
+        launch_xline(s, e, f, K, g, geo, 0, ny - 1, 2, now, part);
+    }
 }
 
-static void zebra_sweep(hipStream_t s, KLevel &l, double *e, const double *f) { zebra(s, l.g, l.geo, l.K.p, e, f); }
+static void zebra_sweep(hipStream_t s, KLevel &l, double *e, const double *f) {
+    zebra(s, l.g, l.geo, l.K.p, e, f, l.far.p);
+}
 static void zebra_sweep(hipStream_t s, KLevel &l, float *e, const float *f) {
-    zebra(s, l.g, l.geo32, l.K32.p, e, f);
+    zebra(s, l.g, l.geo32, l.K32.p, e, f, l.far32.p);
 }
 
 // The coarse level's correction and residual fields of the cycle's type.
@@ -328,6 +340,8 @@ static float *coarse_e(KLevel &c, float *) { return c.e32.p; }
 static float *coarse_r(KLevel &c, float *) { return c.r32.p; }
 static double *coarse_e(KLevel &c, double *) { return c.e.p; }
 static double *coarse_r(KLevel &c, double *) { return c.r.p; }
+static float *far_rows(KLevel &l, float *) { return l.far32.p; }
+static double *far_rows(KLevel &l, double *) { return l.far.p; }
 static const float *table(KLevel &l, float *) { return l.K32.p; }
 static const double *table(KLevel &l, double *) { return l.K.p; }
 static const GeoF &metrics(KLevel &l, float *) { return l.geo32; }
@@ -346,9 +360,9 @@ static void vcycle_t(hipStream_t s, KrylovMG::Impl &K, size_t d, T *e, const T *
     KLevel &c = K.L[d + 1];
     T *ce = coarse_e(c, e), *cr = coarse_r(c, e);
     for (int k = 0; k < K.sd; ++k) zebra_sweep(s, l, e, f);
-    launch_residual_restrict_y(s, cr, ce, e, f, table(l, e), l.g, c.g, metrics(l, e), l.off);
+    launch_residual_restrict_y(s, cr, ce, far_rows(c, e), e, f, table(l, e), l.g, c.g, metrics(l, e), l.off);
     vcycle_t(s, K, d + 1, ce, cr);
-    launch_prolong_y(s, e, ce, l.g, c.g, side_sign(l.bc, YLO), side_sign(l.bc, YHI), l.off);
+    launch_prolong_y(s, e, ce, far_rows(l, e), l.g, c.g, side_sign(l.bc, YLO), side_sign(l.bc, YHI), l.off);
     for (int k = 0; k < K.su; ++k) zebra_sweep(s, l, e, f);
 }
 
@@ -362,23 +376,23 @@ static void precondition(hipStream_t s, KrylovMG::Impl &K, double *e, const doub
     if (K.tr) {
         if (!K.mixed) {
             launch_transpose(s, l.r.p, l.g.pitch, f, tg.pitch, tg.nx, tg.ny);
-            launch_setval(s, l.e.p, 0.0, l.g, 1);
+            launch_begin(s, l.e.p, l.far.p, l.g);
             for (int c = 0; c < K.ncyc; ++c) vcycle_t(s, K, 0, l.e.p, (const double *)l.r.p);
             launch_transpose(s, e, tg.pitch, l.e.p, l.g.pitch, l.g.nx, l.g.ny);
         } else {
             launch_transpose(s, l.r32.p, l.g.pitch, f, tg.pitch, tg.nx, tg.ny);
-            launch_setval(s, l.e32.p, 0.0f, l.g, 1);
+            launch_begin(s, l.e32.p, l.far32.p, l.g);
             for (int c = 0; c < K.ncyc; ++c) vcycle_t(s, K, 0, l.e32.p, (const float *)l.r32.p);
             launch_transpose(s, e, tg.pitch, l.e32.p, l.g.pitch, l.g.nx, l.g.ny);
         }
         return;
     }
     if (!K.mixed) {
-        launch_setval(s, e, 0.0, l.g, 1);
+        launch_begin(s, e, l.far.p, l.g);
         for (int c = 0; c < K.ncyc; ++c) vcycle_t(s, K, 0, e, f);
         return;
     }
-    launch_begin32(s, l.r32.p, l.e32.p, f, l.g);
+    launch_begin32(s, l.r32.p, l.e32.p, l.far32.p, f, l.g);
     for (int c = 0; c < K.ncyc; ++c) vcycle_t(s, K, 0, l.e32.p, (const float *)l.r32.p);
     launch_convert(s, e, l.e32.p, l.g, 0);
 }
@@ -721,10 +735,10 @@ double KrylovMG::time_kernel(hipStream_t s, int kernel, int reps, int cold, doub
         throw Failure(MGP_ERR_ARG);
     }
     auto launch = [&]() {
-        if (kernel == 0) launch_xline(s, l.e.p, l.r.p, l.K.p, g, l.geo, 2, 2, n_even, -1, -1);
+        if (kernel == 0) launch_xline(s, l.e.p, l.r.p, l.K.p, g, l.geo, 2, 2, n_even, XlFar<double>{nullptr, nullptr, {nullptr, nullptr}, {-1, -1}});
         else if (kernel == 1) launch_laplacian(s, l.w.p, l.e.p, l.r.p, g, l.geo, l.bc, 1, 0);
         else if (kernel == 2) launch_lincomb(s, l.w.p, 1.0, l.e.p, 0.0, nullptr, g, 0);
-        else launch_xline(s, l.e32.p, l.r32.p, l.K32.p, g, l.geo32, 2, 2, n_even, -1, -1);
+        else launch_xline(s, l.e32.p, l.r32.p, l.K32.p, g, l.geo32, 2, 2, n_even, XlFar<float>{nullptr, nullptr, {nullptr, nullptr}, {-1, -1}});
     };
     launch();  // warm
     double total = 0.0;
@@ -777,8 +791,8 @@ double KrylovMG::time_kernel(hipStream_t s, int kernel, int reps, int cold, doub
             const Geo geo{c.J.p, c.Jxx.p, c.Jxy.p, c.Jyx.p, c.Jyy.p};
             if (kernel == 3) {
                 const GeoF geo32{nullptr, c.Jxx32.p, c.Jxy32.p, c.Jyx32.p, c.Jyy32.p};
-                launch_xline(s, c.e32.p, c.r32.p, l.K32.p, g, geo32, 2, 2, n_even, -1, -1);
-            } else if (kernel == 0) launch_xline(s, c.e.p, c.r.p, l.K.p, g, geo, 2, 2, n_even, -1, -1);
+                launch_xline(s, c.e32.p, c.r32.p, l.K32.p, g, geo32, 2, 2, n_even, XlFar<float>{nullptr, nullptr, {nullptr, nullptr}, {-1, -1}});
+            } else if (kernel == 0) launch_xline(s, c.e.p, c.r.p, l.K.p, g, geo, 2, 2, n_even, XlFar<double>{nullptr, nullptr, {nullptr, nullptr}, {-1, -1}});
             else if (kernel == 1) launch_laplacian(s, c.w.p, c.e.p, c.r.p, g, geo, l.bc, 1, 0);
             else launch_lincomb(s, c.w.p, 1.0, c.e.p, 0.0, nullptr, g, 0);
         };

@@ -119,15 +119,23 @@ __device__ __forceinline__ int ring_index(int nx, int ny, int i, int j) {
 
 // (L e)(i, j) at a ring cell from the table.  All nine table entries and
 // field values are loaded before any is used (one memory round trip).
+// far: where the window's row two rows in is read from (cell i at
+// [OFFX + i]; rows 0 and ny-1 in the line relaxation), null for the field.
 template <typename T>
-__device__ __forceinline__ T ring_lap(gconst<T> *e, gconst<T> *K, int nring, const Grid &g, int i, int j) {
+__device__ __forceinline__ T ring_lap(gconst<T> *e, gconst<T> *K, int nring, const Grid &g, int i, int j,
+                                      gconst<T> *far = nullptr) {
     const int w0 = window_origin(i, g.nx), v0 = window_origin(j, g.ny);
     const int r = ring_index(g.nx, g.ny, i, j);
+    gconst<T> *row[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) row[a] = e + ix(g.pitch, -OFFX, j + v0 + a);
+    if (far && j == 0) row[2] = far;
+    if (far && j == g.ny - 1) row[0] = far;
     T kv[9], ev[9];
 #pragma unroll
     for (int q = 0; q < 9; ++q) {
         kv[q] = K[(size_t)q * nring + r];
-        ev[q] = e[ix(g.pitch, i + w0 + q % 3, j + v0 + q / 3)];
+        ev[q] = row[q / 3][OFFX + i + w0 + q % 3];
     }
     T lap = 0;
 #pragma unroll
@@ -248,7 +256,8 @@ struct Buf {
 
 template <int C, int NT, bool SEG = false, int RG = 1, typename T, typename GM>
 __device__ __forceinline__ void row_pass(const RowCtx<T> &X, const T *e_, const T *f_, const T *K_, const Grid &g,
-                                         const GM &geo_, int j, T *Ld, T *La, T *Lb, T *Lc, T (&ev)[C + 1]) {
+                                         const GM &geo_, int j, const T *far, T *Ld, T *La, T *Lb, T *Lc,
+                                         T (&ev)[C + 1]) {
     constexpr int U = C + 1;
     gconst<T> *e = gptr(e_), *f = gptr(f_), *K = gptr(K_);
     // SEG: the cells solved may be a segment of the row (xline_rows); whole
@@ -343,7 +352,7 @@ __device__ __forceinline__ void row_pass(const RowCtx<T> &X, const T *e_, const 
             const int i = i0 + il;
             ev[u] = e[ix(P, i, j)];
             const T fv = f[ix(P, i, j)];
-            const T lap = ring_lap(e, K, X.nring, g, i, j);
+            const T lap = ring_lap(e, K, X.nring, g, i, j, gptr(far));
             T a, b, c;
             ring_row_coef(K, X.nring, g, i, j, a, b, c);
             const int o = iraw < nx ? chunk_pos<C>(il, X.rem) : dump;
@@ -517,13 +526,13 @@ __device__ __forceinline__ void interface_solve(const T *I, T *X, int nt, int l)
 // ---------------------------------------------------------------------------
 template <int C, int NT, bool SEG = false, int RG = 1, typename T, typename GM>
 __device__ void xline_row(const RowCtx<T> &X, T *__restrict__ e, const T *__restrict__ f, const T *__restrict__ K,
-                          const Grid &g, const GM &geo, int j, T *lds) {
+                          const Grid &g, const GM &geo, int j, const T *far, T *lds) {
     constexpr int CP = C + 1;
     const int tid = threadIdx.x, nt = X.nt;
     const int NT1 = nt * CP;
     T *Ld = lds, *Lb = lds + NT1, *La = lds + 2 * NT1, *Lc = lds + 3 * NT1;
     T ev[CP];
-    row_pass<C, NT, SEG, RG>(X, e, f, K, g, geo, j, Ld, La, Lb, Lc, ev);
+    row_pass<C, NT, SEG, RG>(X, e, f, K, g, geo, j, far, Ld, La, Lb, Lc, ev);
     __syncthreads();
 
     // each thread takes its chunk into registers
@@ -583,11 +592,14 @@ __device__ void xline_row(const RowCtx<T> &X, T *__restrict__ e, const T *__rest
     row_update_add<C, NT, SEG>(X, e, j, lds, ev);
 }
 
-// Rows j = row0 + slot*rowstep; the workgroup of slot 0 then also relaxes
-// row extra0 and the last slot row extra1 (< 0: none), each after its own
-// row.  The boundary rows ride on the odd-row launch this way: row 0 after
-// row 1 and row ny-1 after the last odd row, the order of a separate third
-// phase, without its launch.
+// Row `row` of e into `to` (XlFar).
+template <int NT, typename T>
+__device__ __forceinline__ void save_row(T *to, const T *e, const Grid &g, int row) {
+    for (int i = threadIdx.x; i < g.nx; i += NT) to[OFFX + i] = e[ix(g.pitch, i, row)];
+}
+
+// Rows j = row0 + slot*rowstep, one workgroup each; the workgroups past the
+// rows save the far rows of the next launch.
 //
 // Rows longer than one workgroup's line solve are cut into segments of
 // seglen cells, each solved as a line (row_pass).  A launch relaxes segments
@@ -599,32 +611,25 @@ __device__ void xline_row(const RowCtx<T> &X, T *__restrict__ e, const T *__rest
 // a segment of the other parity.  A whole row: seglen = nx, nsegl = 1.
 template <int C, int NT, bool SEG, int RG = 3, typename T, typename GM>
 __device__ __forceinline__ void xline_rows(T *__restrict__ e, const T *__restrict__ f, const T *__restrict__ K,
-                                           const Grid &g, const GM &geo, int row0, int rowstep, int nt, int extra0,
-                                           int extra1, int seglen, int seg0, int segstep, int nsegl) {
+                                           const Grid &g, const GM &geo, int row0, int rowstep, int nrows, int nt,
+                                           const XlFar<T> &far, int seglen, int seg0, int segstep, int nsegl) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_bytes[];
     T *lds = reinterpret_cast<T *>(lds_bytes);
-    RowCtx<T> X0 = row_ctx<T>(g, nt, C);
-    int slot = launch_slot(), nslots = (int)gridDim.x;
+    RowCtx<T> X = row_ctx<T>(g, nt, C);
+    int slot = launch_slot();
+    if (slot >= nrows * nsegl) {
+        const bool first = slot == nrows * nsegl && far.save[0] >= 0;
+        save_row<NT>(first ? far.to[0] : far.to[1], e, g, first ? far.save[0] : far.save[1]);
+        return;
+    }
     if (SEG) {
-        X0.nx = seglen;
-        X0.rem = seglen - nt * C;
-        X0.i0 = (seg0 + segstep * (slot % nsegl)) * seglen;
+        X.nx = seglen;
+        X.rem = seglen - nt * C;
+        X.i0 = (seg0 + segstep * (slot % nsegl)) * seglen;
         slot /= nsegl;
-        nslots /= nsegl;
     }
-    const int ex0 = slot == 0 ? extra0 : -1, ex1 = slot == nslots - 1 ? extra1 : -1;
-#pragma unroll 1
-    for (int r = 0; r < 3; ++r) {
-        const int jr = r == 0 ? row0 + slot * rowstep : (r == 1 ? ex0 : ex1);
-        if (jr < 0) continue;  // uniform over the workgroup
-        if (r) __syncthreads();
-        // the chunk remainder is made opaque per row, so the per-thread LDS
-        // positions derived from it are recomputed in the row (a few integer
-        // ops) instead of being hoisted out of the loop and spilled
-        RowCtx<T> X = X0;
-        asm volatile("" : "+s"(X.rem));
-        xline_row<C, NT, SEG, RG>(X, e, f, K, g, geo, jr, lds);
-    }
+    const int j = row0 + slot * rowstep;
+    xline_row<C, NT, SEG, RG>(X, e, f, K, g, geo, j, j == 0 ? far.lo : far.hi, lds);
 }
 
 // Waves per SIMD of the fine-level kernel: the LDS of one workgroup at
@@ -641,34 +646,34 @@ constexpr int xl_waves() {
 template <int C, bool SEG, typename T, typename GM>
 __global__ void __launch_bounds__(XL_THREADS) __attribute__((amdgpu_waves_per_eu(xl_waves<T>(), xl_waves<T>())))
 k_xline(T *__restrict__ e, const T *__restrict__ f, const T *__restrict__ K, Grid g, GM geo, int row0, int rowstep,
-        int nt, int extra0, int extra1, int seglen, int seg0, int segstep, int nsegl) {
-    xline_rows<C, XL_THREADS, SEG>(e, f, K, g, geo, row0, rowstep, nt, extra0, extra1, seglen, seg0, segstep, nsegl);
+        int nrows, int nt, XlFar<T> far, int seglen, int seg0, int segstep, int nsegl) {
+    xline_rows<C, XL_THREADS, SEG>(e, f, K, g, geo, row0, rowstep, nrows, nt, far, seglen, seg0, segstep, nsegl);
 }
 
 // Rows of at most 512 cells: one 64-thread wave per row (as in the batch).
 template <int C, bool SEG, typename T, typename GM>
 __global__ void __launch_bounds__(XL_SHORT) __attribute__((amdgpu_waves_per_eu(2)))
 k_xline_short(T *__restrict__ e, const T *__restrict__ f, const T *__restrict__ K, Grid g, GM geo, int row0,
-              int rowstep, int nt, int extra0, int extra1, int seglen, int seg0, int segstep, int nsegl) {
-    xline_rows<C, XL_SHORT, SEG>(e, f, K, g, geo, row0, rowstep, nt, extra0, extra1, seglen, seg0, segstep, nsegl);
+              int rowstep, int nrows, int nt, XlFar<T> far, int seglen, int seg0, int segstep, int nsegl) {
+    xline_rows<C, XL_SHORT, SEG>(e, f, K, g, geo, row0, rowstep, nrows, nt, far, seglen, seg0, segstep, nsegl);
 }
 
 // FP32 rows past 4111 cells (C = 16, 512 threads): one workgroup per CU.
 template <int C, typename T, typename GM>
 __global__ void __launch_bounds__(XL_WIDE) k_xline_wide(T *__restrict__ e, const T *__restrict__ f,
                                                         const T *__restrict__ K, Grid g, GM geo, int row0,
-                                                        int rowstep, int nt, int extra0, int extra1, int seglen,
+                                                        int rowstep, int nrows, int nt, XlFar<T> far, int seglen,
                                                         int seg0, int segstep, int nsegl) {
-    xline_rows<C, XL_WIDE, false>(e, f, K, g, geo, row0, rowstep, nt, extra0, extra1, seglen, seg0, segstep, nsegl);
+    xline_rows<C, XL_WIDE, false>(e, f, K, g, geo, row0, rowstep, nrows, nt, far, seglen, seg0, segstep, nsegl);
 }
 
 // Longer rows (C = 16): one workgroup per CU in FP64 (139 KB of LDS), all registers.
 template <int C, bool SEG, typename T, typename GM>
 __global__ void __launch_bounds__(XL_THREADS) k_xline_long(T *__restrict__ e, const T *__restrict__ f,
                                                            const T *__restrict__ K, Grid g, GM geo, int row0,
-                                                           int rowstep, int nt, int extra0, int extra1,
+                                                           int rowstep, int nrows, int nt, XlFar<T> far,
                                                            int seglen, int seg0, int segstep, int nsegl) {
-    xline_rows<C, XL_THREADS, SEG>(e, f, K, g, geo, row0, rowstep, nt, extra0, extra1, seglen, seg0, segstep, nsegl);
+    xline_rows<C, XL_THREADS, SEG>(e, f, K, g, geo, row0, rowstep, nrows, nt, far, seglen, seg0, segstep, nsegl);
 }
 
 // (L e)(i, j) at an interior cell from the face metrics: the stencil of
@@ -689,10 +694,11 @@ __device__ __forceinline__ T interior_lap(gconst<T> *e, const G &geo_, int P, si
 
 // Preconditioner residual restricted 1x2 in y, with the coarse correction
 // cleared:  rc(i, J) = (r(i, 2J) + r(i, 2J+1)) / 2,  r = f - L e  (interior
-// stencil from the metrics, ring cells from the table),  ec(i, J) = 0.
+// stencil from the metrics, ring cells from the table),  ec(i, J) = 0, with
+// its far rows farc (XlFar: lo, then hi one pitch on).
 template <typename T, typename G>
-__device__ __forceinline__ void restrict_cell(T *rc, T *ec, const T *e, const T *f, const T *K, const Grid &gf,
-                                              const Grid &gc, const G &geo, int i, int J, int off) {
+__device__ __forceinline__ void restrict_cell(T *rc, T *ec, T *farc, const T *e, const T *f, const T *K,
+                                              const Grid &gf, const Grid &gc, const G &geo, int i, int J, int off) {
     const int nring = ring_count(gf.nx, gf.ny);
     const T idx = (T)(1.0 / gf.dx), idy = (T)(1.0 / gf.dy);
     T s = 0;
@@ -707,15 +713,16 @@ __device__ __forceinline__ void restrict_cell(T *rc, T *ec, const T *e, const T 
     const size_t c = ix(gc.pitch, i, J);
     rc[c] = s;
     ec[c] = 0;
+    if (J < 2) farc[J * gc.pitch + OFFX + i] = 0;
 }
 
 template <typename T, typename G>
-__global__ void __launch_bounds__(256) k_residual_restrict_y(T *rc, T *ec, const T *e, const T *f, const T *K,
-                                                             Grid gf, Grid gc, G geo, int off) {
+__global__ void __launch_bounds__(256) k_residual_restrict_y(T *rc, T *ec, T *farc, const T *e, const T *f,
+                                                             const T *K, Grid gf, Grid gc, G geo, int off) {
     const int i = blockIdx.x * 64 + (threadIdx.x & 63);
     const int J = blockIdx.y * 4 + (threadIdx.x >> 6);
     if (i >= gc.nx || J >= gc.ny) return;
-    restrict_cell(rc, ec, e, f, K, gf, gc, geo, i, J, off);
+    restrict_cell(rc, ec, farc, e, f, K, gf, gc, geo, i, J, off);
 }
 
 // ---------------------------------------------------------------------------
@@ -724,14 +731,16 @@ __global__ void __launch_bounds__(256) k_residual_restrict_y(T *rc, T *ec, const
 // ---------------------------------------------------------------------------
 // The level's fields of the cycle's element type.
 __device__ __forceinline__ void level_fields(const BLev *L, int sel, double *&e, const double *&f, const double *&K,
-                                             Geo &geo) {
+                                             double *&far, Geo &geo) {
+    far = L->far;
     e = L->e[sel];
     f = L->f[sel];
     K = L->K;
     geo = L->geo;
 }
 __device__ __forceinline__ void level_fields(const BLev *L, int, float *&e, const float *&f, const float *&K,
-                                             GeoF &geo) {
+                                             float *&far, GeoF &geo) {
+    far = L->far32;
     e = L->e32;
     f = L->f32;
     K = L->K32;
@@ -757,20 +766,16 @@ __device__ __forceinline__ void xline_task(const XlTask *tasks, const BLev *levs
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_bytes[];
     T *lds = reinterpret_cast<T *>(lds_bytes);
     const Grid g = L->g;
-    T *e;
+    T *e, *far;
     const T *f, *K;
     typename std::conditional<sizeof(T) == 8, Geo, GeoF>::type geo;
-    level_fields(L, sel, e, f, K, geo);
-    const RowCtx<T> X0 = row_ctx<T>(g, L->nt, C);
-#pragma unroll 1
-    for (int r = 0; r < 2; ++r) {
-        const int jr = r == 0 ? t.row : t.extra;
-        if (jr < 0) continue;  // uniform over the workgroup
-        if (r) __syncthreads();
-        RowCtx<T> X = X0;
-        asm volatile("" : "+s"(X.rem));
-        xline_row<C, NT, false, batch_rg<C, T>()>(X, e, f, K, g, geo, jr, lds);
+    level_fields(L, sel, e, f, K, far, geo);
+    if (t.save) {
+        save_row<NT>(far + t.side * g.pitch, (const T *)e, g, t.row);
+        return;
     }
+    const RowCtx<T> X = row_ctx<T>(g, L->nt, C);
+    xline_row<C, NT, false, batch_rg<C, T>()>(X, e, f, K, g, geo, t.row, t.row == 0 ? far : far + g.pitch, lds);
 }
 
 template <int C, typename T>
@@ -808,16 +813,16 @@ __global__ void __launch_bounds__(256) k_restrict_batch(const BTile *tiles, cons
     const int i = t.tx * 64 + (threadIdx.x & 63);
     const Grid gc = Cl->g;
     if (i >= gc.nx) return;
-    T *fe, *ce, *cf;
+    T *fe, *ce, *cf, *far, *cfar;
     const T *ff, *K, *cff, *cK;
     typename std::conditional<sizeof(T) == 8, Geo, GeoF>::type geo, cgeo;
-    level_fields(F, sel, fe, ff, K, geo);
-    level_fields(Cl, 0, ce, cff, cK, cgeo);
+    level_fields(F, sel, fe, ff, K, far, geo);
+    level_fields(Cl, 0, ce, cff, cK, cfar, cgeo);
     cf = const_cast<T *>(cff);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int J = t.ty * BT_ROWS + (threadIdx.x >> 6) + 4 * r;
-        if (J < gc.ny) restrict_cell(cf, ce, (const T *)fe, ff, K, F->g, gc, geo, i, J, F->off);
+        if (J < gc.ny) restrict_cell(cf, ce, cfar, (const T *)fe, ff, K, F->g, gc, geo, i, J, F->off);
     }
 }
 
@@ -830,15 +835,15 @@ __global__ void __launch_bounds__(256) k_prolong_batch(const BTile *tiles, const
     const int i = t.tx * 64 + (threadIdx.x & 63);
     const Grid gf = F->g, gc = Cl->g;
     if (i >= gf.nx) return;
-    T *fe, *ce;
+    T *fe, *ce, *far, *cfar;
     const T *ff, *K, *cf, *cK;
     typename std::conditional<sizeof(T) == 8, Geo, GeoF>::type geo, cgeo;
-    level_fields(F, sel, fe, ff, K, geo);
-    level_fields(Cl, 0, ce, cf, cK, cgeo);
+    level_fields(F, sel, fe, ff, K, far, geo);
+    level_fields(Cl, 0, ce, cf, cK, cfar, cgeo);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int j = t.ty * BT_ROWS + (threadIdx.x >> 6) + 4 * r;
-        if (j < gf.ny) prolong_y_cell(fe, (const T *)ce, gf, gc, (T)F->slo, (T)F->shi, i, j, F->off);
+        if (j < gf.ny) prolong_y_cell(fe, (const T *)ce, far, gf, gc, (T)F->slo, (T)F->shi, i, j, F->off);
     }
 }
 
@@ -898,41 +903,41 @@ void xline_batch_shape(int nx, int &C, int &threads) {
 }
 
 template <typename T, typename G>
-static void residual_restrict_y(hipStream_t s, T *rc, T *ec, const T *e, const T *f, const T *K, const Grid &gf,
-                                const Grid &gc, const G &geo, int off) {
+static void residual_restrict_y(hipStream_t s, T *rc, T *ec, T *farc, const T *e, const T *f, const T *K,
+                                const Grid &gf, const Grid &gc, const G &geo, int off) {
     const dim3 grid((unsigned)((gc.nx + 63) / 64), (unsigned)((gc.ny + 3) / 4));
-    k_residual_restrict_y<<<grid, 256, 0, s>>>(rc, ec, e, f, K, gf, gc, geo, off);
+    k_residual_restrict_y<<<grid, 256, 0, s>>>(rc, ec, farc, e, f, K, gf, gc, geo, off);
 }
 
-void launch_residual_restrict_y(hipStream_t s, double *rc, double *ec, const double *e, const double *f,
+void launch_residual_restrict_y(hipStream_t s, double *rc, double *ec, double *farc, const double *e, const double *f,
                                 const double *K, const Grid &gf, const Grid &gc, const Geo &geo, int off) {
-    residual_restrict_y(s, rc, ec, e, f, K, gf, gc, geo, off);
+    residual_restrict_y(s, rc, ec, farc, e, f, K, gf, gc, geo, off);
 }
 
-void launch_residual_restrict_y(hipStream_t s, float *rc, float *ec, const float *e, const float *f, const float *K,
+void launch_residual_restrict_y(hipStream_t s, float *rc, float *ec, float *farc, const float *e, const float *f, const float *K,
                                 const Grid &gf, const Grid &gc, const GeoF &geo, int off) {
-    residual_restrict_y(s, rc, ec, e, f, K, gf, gc, geo, off);
+    residual_restrict_y(s, rc, ec, farc, e, f, K, gf, gc, geo, off);
 }
 
 // One launch of the line kernel for rows (SEG = false) or segments of seglen cells.
 template <bool SEG, typename T, typename G>
 static void xline_launch(hipStream_t s, T *e, const T *f, const T *K, const Grid &g, const G &geo, int row0,
-                         int rowstep, int extra0, int extra1, int seglen, int seg0, int segstep, int nsegl,
+                         int rowstep, int nrows, const XlFar<T> &far, int seglen, int seg0, int segstep, int nsegl,
                          unsigned grid) {
     if (xline_chunk(seglen) == 0) {
         // only whole FP32 rows get here (xline_segments): the 512-thread form
         if constexpr (sizeof(T) == 4 && !SEG) {
             const int nt = seglen / 16;
             const size_t lds = xline_lds_bytes_for(seglen, 16, sizeof(T), XL_WIDE);
-            k_xline_wide<16><<<grid, XL_WIDE, lds, s>>>(e, f, K, g, geo, row0, rowstep, nt, extra0, extra1, seglen, seg0, segstep, nsegl);
+            k_xline_wide<16><<<grid, XL_WIDE, lds, s>>>(e, f, K, g, geo, row0, rowstep, nrows, nt, far, seglen, seg0, segstep, nsegl);
         }
     } else if (seglen <= XL_SHORT_MAX_NX) {
         const int C = xline_chunk(seglen, XL_SHORT), nt = seglen / C;
         const size_t lds = xline_lds_bytes_for(seglen, C, sizeof(T), XL_SHORT);
         switch (C) {
-            case 2: k_xline_short<2, SEG><<<grid, XL_SHORT, lds, s>>>(e, f, K, g, geo, row0, rowstep, nt, extra0, extra1, seglen, seg0, segstep, nsegl); break;
-            case 4: k_xline_short<4, SEG><<<grid, XL_SHORT, lds, s>>>(e, f, K, g, geo, row0, rowstep, nt, extra0, extra1, seglen, seg0, segstep, nsegl); break;
-            default: k_xline_short<8, SEG><<<grid, XL_SHORT, lds, s>>>(e, f, K, g, geo, row0, rowstep, nt, extra0, extra1, seglen, seg0, segstep, nsegl); break;
+            case 2: k_xline_short<2, SEG><<<grid, XL_SHORT, lds, s>>>(e, f, K, g, geo, row0, rowstep, nrows, nt, far, seglen, seg0, segstep, nsegl); break;
+            case 4: k_xline_short<4, SEG><<<grid, XL_SHORT, lds, s>>>(e, f, K, g, geo, row0, rowstep, nrows, nt, far, seglen, seg0, segstep, nsegl); break;
+            default: k_xline_short<8, SEG><<<grid, XL_SHORT, lds, s>>>(e, f, K, g, geo, row0, rowstep, nrows, nt, far, seglen, seg0, segstep, nsegl); break;
         }
     } else {
         const int C = xline_chunk(seglen);
@@ -943,17 +948,17 @@ static void xline_launch(hipStream_t s, T *e, const T *f, const T *K, const Grid
         }
         const int nt = seglen / C;
         switch (C) {
-            case 2: k_xline<2, SEG><<<grid, XL_THREADS, lds, s>>>(e, f, K, g, geo, row0, rowstep, nt, extra0, extra1, seglen, seg0, segstep, nsegl); break;
-            case 4: k_xline<4, SEG><<<grid, XL_THREADS, lds, s>>>(e, f, K, g, geo, row0, rowstep, nt, extra0, extra1, seglen, seg0, segstep, nsegl); break;
-            case 8: k_xline<8, SEG><<<grid, XL_THREADS, lds, s>>>(e, f, K, g, geo, row0, rowstep, nt, extra0, extra1, seglen, seg0, segstep, nsegl); break;
-            default: k_xline_long<16, SEG><<<grid, XL_THREADS, lds, s>>>(e, f, K, g, geo, row0, rowstep, nt, extra0, extra1, seglen, seg0, segstep, nsegl); break;
+            case 2: k_xline<2, SEG><<<grid, XL_THREADS, lds, s>>>(e, f, K, g, geo, row0, rowstep, nrows, nt, far, seglen, seg0, segstep, nsegl); break;
+            case 4: k_xline<4, SEG><<<grid, XL_THREADS, lds, s>>>(e, f, K, g, geo, row0, rowstep, nrows, nt, far, seglen, seg0, segstep, nsegl); break;
+            case 8: k_xline<8, SEG><<<grid, XL_THREADS, lds, s>>>(e, f, K, g, geo, row0, rowstep, nrows, nt, far, seglen, seg0, segstep, nsegl); break;
+            default: k_xline_long<16, SEG><<<grid, XL_THREADS, lds, s>>>(e, f, K, g, geo, row0, rowstep, nrows, nt, far, seglen, seg0, segstep, nsegl); break;
         }
     }
 }
 
 template <typename T, typename G>
 static void xline(hipStream_t s, T *e, const T *f, const T *K, const Grid &g, const G &geo, int row0, int rowstep,
-                  int nrows, int extra0, int extra1) {
+                  int nrows, const XlFar<T> &far, int part = -1) {
     if (nrows <= 0) return;
     const int nseg = xline_segments(g.nx, sizeof(T));
     if (nseg == 0) {
@@ -963,10 +968,11 @@ static void xline(hipStream_t s, T *e, const T *f, const T *K, const Grid &g, co
     const int seglen = g.nx / nseg;
     // whole rows in one launch; segmented rows: the even segments, then the odd ones
     const int nlaunch = nseg == 1 ? 1 : 2, segstep = nseg == 1 ? 1 : 2, nsegl = nseg == 1 ? 1 : nseg / 2;
-    const unsigned grid = (unsigned)(nrows * nsegl);
+    const unsigned grid = (unsigned)(nrows * nsegl + (far.save[0] >= 0) + (far.save[1] >= 0));
     for (int seg0 = 0; seg0 < nlaunch; ++seg0) {
-        if (nseg > 1) xline_launch<true>(s, e, f, K, g, geo, row0, rowstep, extra0, extra1, seglen, seg0, segstep, nsegl, grid);
-        else xline_launch<false>(s, e, f, K, g, geo, row0, rowstep, extra0, extra1, seglen, seg0, segstep, nsegl, grid);
+        if (part >= 0 && seg0 != part) continue;
+        if (nseg > 1) xline_launch<true>(s, e, f, K, g, geo, row0, rowstep, nrows, far, seglen, seg0, segstep, nsegl, grid);
+        else xline_launch<false>(s, e, f, K, g, geo, row0, rowstep, nrows, far, seglen, seg0, segstep, nsegl, grid);
         const hipError_t err = hipGetLastError();
         if (err != hipSuccess) {
             g_last_error = std::string("k_xline launch: ") + hipGetErrorString(err);
@@ -976,8 +982,8 @@ static void xline(hipStream_t s, T *e, const T *f, const T *K, const Grid &g, co
 }
 
 void launch_xline(hipStream_t s, double *e, const double *f, const double *K, const Grid &g, const Geo &geo,
-                  int row0, int rowstep, int nrows, int extra0, int extra1) {
-    xline(s, e, f, K, g, geo, row0, rowstep, nrows, extra0, extra1);
+                  int row0, int rowstep, int nrows, const XlFar<double> &far, int part) {
+    xline(s, e, f, K, g, geo, row0, rowstep, nrows, far, part);
 }
 
 template <typename T>
@@ -1025,8 +1031,8 @@ void launch_xline_batch(hipStream_t s, const XlTask *tasks, int ntasks, const BL
 }
 
 void launch_xline(hipStream_t s, float *e, const float *f, const float *K, const Grid &g, const GeoF &geo, int row0,
-                  int rowstep, int nrows, int extra0, int extra1) {
-    xline(s, e, f, K, g, geo, row0, rowstep, nrows, extra0, extra1);
+                  int rowstep, int nrows, const XlFar<float> &far) {
+    xline(s, e, f, K, g, geo, row0, rowstep, nrows, far);
 }
 
 void launch_restrict_batch(hipStream_t s, const BTile *tiles, int ntiles, const BLev *levs, const int *active,

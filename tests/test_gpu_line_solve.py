@@ -22,3 +22,28 @@ def test_row_solve_edges(nx, ny, types):
     # the row system's condition number is about 2 (dy / dx)^2 where the x couplings dominate
     tol = max(1e-10, 4 * np.finfo(float).eps * 2.0 * (geo.dy / geo.dx) ** 2)
     np.testing.assert_allclose(got, want, rtol=0, atol=tol * np.max(np.abs(want)))
+
+
+@pytest.mark.parametrize("ny", [4, 5, 6, 7, 9, 16])
+@pytest.mark.parametrize("types", [(1, 1, 0, 0), (1, 1, 1, 1), (1, 0, 0, 1)])
+@pytest.mark.parametrize("method", [mg.METHOD_KRYLOV_MG, mg.METHOD_KRYLOV_MG32])
+def test_sweeps_of_few_rows(ny, types, method):
+    """The boundary rows relax beside the other rows of their colour, on saved
+    copies of the rows they reach; with few rows each row is a boundary row or
+    next to one, and rows 2 and ny-3 may be the same or swap roles.  The solve
+    must reach the direct solution, and the batch the same as the single
+    solver."""
+    import scipy.sparse.linalg as spl
+    from cases import probed_matrix
+    geo, bc, _, rhs = setup(40, ny, 0.08, 3.0, types, seed=ny)
+    exact = spl.spsolve(probed_matrix(geo, bc).tocsc(), rhs.ravel()).reshape(geo.ny, geo.nx)
+    s = mg.Solver(geo, bc, method=method)
+    s.set_rhs(rhs)
+    _, iters, oc = s.solve(1e-12, 100)
+    assert oc == mg.CONVERGED and iters <= 30, iters
+    np.testing.assert_allclose(s.get_phi()[1:-1, 1:-1], exact, rtol=0, atol=1e-10 * np.max(np.abs(exact)))
+    b = mg.Batch([geo], [bc], method=method)
+    b.set_rhs(0, rhs)
+    its, oc = b.solve(1e-12, 100)
+    assert oc[0] == mg.CONVERGED and its[0] <= 30
+    np.testing.assert_allclose(b.get_phi(0), exact, rtol=0, atol=1e-10 * np.max(np.abs(exact)))
