@@ -51,6 +51,17 @@ constexpr int XL_MID_MAX_NX = 1024;
 // FP32 rows of 4112 .. 8207 cells: 512 threads, chunks of 16 (139 KB of LDS),
 // so the mixed-precision cycle solves rows of 8192 cells whole.
 constexpr int XL_WIDE = 512;
+// The single-problem solver's launches of few rows (up to two per CU: every
+// coarse level) take as long as one row solve, so they use more threads per
+// row than the fine levels' launches, whose many rows fill the CUs: rows of
+// 129 .. 512 cells 256 threads instead of one wave (512^2 FP64 35.5 -> 28.8 ms;
+// at 128 cells and below one wave is as fast or faster), FP32 rows of 1025 ..
+// 2048 cells 512 threads (1500 x 800: 18.7 -> 16.9 ms; FP64 rows of that length
+// and rows of 513 .. 1024 cells were slower by 7 and 12 %).
+constexpr unsigned XL_FEW_ROWS = 512;
+constexpr int XL_SHORT_FEW_MAX_NX = 128;
+constexpr int XL_LONG_MIN_NX = 1024, XL_LONG_MAX_NX = 2048;
+constexpr int XL_WIDEST = 1024;  // FP32 rows past 4111 cells, few of them
 constexpr int RING_PLANES = 9;
 
 // Impulse whose ghosts follow the homogeneous fill of the MG levels
@@ -659,12 +670,12 @@ k_xline_short(T *__restrict__ e, const T *__restrict__ f, const T *__restrict__ 
 }
 
 // FP32 rows past 4111 cells (C = 16, 512 threads): one workgroup per CU.
-template <int C, typename T, typename GM>
-__global__ void __launch_bounds__(XL_WIDE) k_xline_wide(T *__restrict__ e, const T *__restrict__ f,
+template <int C, int NT, typename T, typename GM>
+__global__ void __launch_bounds__(NT) k_xline_wide(T *__restrict__ e, const T *__restrict__ f,
                                                         const T *__restrict__ K, Grid g, GM geo, int row0,
                                                         int rowstep, int nrows, int nt, XlFar<T> far, int seglen,
                                                         int seg0, int segstep, int nsegl) {
-    xline_rows<C, XL_WIDE, false>(e, f, K, g, geo, row0, rowstep, nrows, nt, far, seglen, seg0, segstep, nsegl);
+    xline_rows<C, NT, false>(e, f, K, g, geo, row0, rowstep, nrows, nt, far, seglen, seg0, segstep, nsegl);
 }
 
 // Longer rows (C = 16): one workgroup per CU in FP64 (139 KB of LDS), all registers.
@@ -924,14 +935,22 @@ template <bool SEG, typename T, typename G>
 static void xline_launch(hipStream_t s, T *e, const T *f, const T *K, const Grid &g, const G &geo, int row0,
                          int rowstep, int nrows, const XlFar<T> &far, int seglen, int seg0, int segstep, int nsegl,
                          unsigned grid) {
-    if (xline_chunk(seglen) == 0) {
-        // only whole FP32 rows get here (xline_segments): the 512-thread form
+    const bool few = grid <= XL_FEW_ROWS;
+    if (sizeof(T) == 4 && !SEG && (xline_chunk(seglen) == 0 || (few && seglen > XL_LONG_MIN_NX && seglen <= XL_LONG_MAX_NX))) {
         if constexpr (sizeof(T) == 4 && !SEG) {
-            const int nt = seglen / 16;
-            const size_t lds = xline_lds_bytes_for(seglen, 16, sizeof(T), XL_WIDE);
-            k_xline_wide<16><<<grid, XL_WIDE, lds, s>>>(e, f, K, g, geo, row0, rowstep, nrows, nt, far, seglen, seg0, segstep, nsegl);
+            // few rows: the widest form; rows past 4111 cells always (xline_segments)
+            if (xline_chunk(seglen) != 0) {
+                const size_t lds = xline_lds_bytes_for(seglen, 4, sizeof(T), XL_WIDE);
+                k_xline_wide<4, XL_WIDE><<<grid, XL_WIDE, lds, s>>>(e, f, K, g, geo, row0, rowstep, nrows, seglen / 4, far, seglen, seg0, segstep, nsegl);
+            } else if (few && xline_chunk(seglen, XL_WIDEST) == 8) {
+                const size_t lds = xline_lds_bytes_for(seglen, 8, sizeof(T), XL_WIDEST);
+                k_xline_wide<8, XL_WIDEST><<<grid, XL_WIDEST, lds, s>>>(e, f, K, g, geo, row0, rowstep, nrows, seglen / 8, far, seglen, seg0, segstep, nsegl);
+            } else {
+                const size_t lds = xline_lds_bytes_for(seglen, 16, sizeof(T), XL_WIDE);
+                k_xline_wide<16, XL_WIDE><<<grid, XL_WIDE, lds, s>>>(e, f, K, g, geo, row0, rowstep, nrows, seglen / 16, far, seglen, seg0, segstep, nsegl);
+            }
         }
-    } else if (seglen <= XL_SHORT_MAX_NX) {
+    } else if (seglen <= (few ? XL_SHORT_FEW_MAX_NX : XL_SHORT_MAX_NX)) {
         const int C = xline_chunk(seglen, XL_SHORT), nt = seglen / C;
         const size_t lds = xline_lds_bytes_for(seglen, C, sizeof(T), XL_SHORT);
         switch (C) {

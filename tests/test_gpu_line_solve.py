@@ -47,3 +47,29 @@ def test_sweeps_of_few_rows(ny, types, method):
     its, oc = b.solve(1e-12, 100)
     assert oc[0] == mg.CONVERGED and its[0] <= 30
     np.testing.assert_allclose(b.get_phi(0), exact, rtol=0, atol=1e-10 * np.max(np.abs(exact)))
+
+
+def test_many_rows_use_one_wave_each():
+    """Past 512 rows in a launch, rows of 129 .. 512 cells take one wave each
+    instead of 256 threads: 514 rows per colour here."""
+    nx, ny = 300, 1030
+    geo, bc, phi, rhs = setup(nx, ny, 0.05, 1.0, (1, 1, 0, 0), seed=2)
+    got = mg.xline_relax(geo, bc, rhs, phi, 1)[1:-1, 1:-1]
+    want = zebra_reference(geo, bc, rhs, phi, 1)
+    np.testing.assert_allclose(got, want, rtol=0, atol=1e-10 * np.max(np.abs(want)))
+
+
+@pytest.mark.parametrize("nx", [1025, 2048, 2049, 4112, 8192, 8200])
+def test_fp32_rows_of_each_width(nx):
+    """FP32 cycles with few rows: 512 threads for 1025 .. 2048 cells, 256 up to
+    4111, 1024 up to 8199 and 512 for the last few lengths.  x-lines are nearly
+    a direct solve on this grid, so a wrong row solve shows as iterations."""
+    import refcall as rc
+    ny = 12
+    geo, bc, _, rhs = setup(nx, ny, 0.0, 0.0, (1, 1, 0, 0), seed=nx)
+    s = mg.Solver(geo, bc, method=mg.METHOD_KRYLOV_MG32, lines=mg.LINES_X)
+    s.set_rhs(rhs)
+    hist, iters, oc = s.solve(1e-9, 60)
+    assert oc == mg.CONVERGED and iters <= 12, (iters, hist[-3:])
+    r, _ = rc.oracle().residual(geo, bc, 1, rhs, s.get_phi())
+    assert np.linalg.norm(r) <= 1.5e-9 * np.linalg.norm(rhs)
