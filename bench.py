@@ -18,7 +18,7 @@ Beside it, in the same run:
   latency; the ratio value / plain is the metric's "mixed/batched vs plain";
 * the batched solver with FP64 cycles;
 * roofline: the batch's dominant kernel, the finest-level line relaxation of
-  every problem (one launch per chunk class, side by side), cache-cold;
+  every problem (launched as inside a solve), cache-cold;
 * single_2048: the FP64 drop-in single solve (2048^2 stretched, warped map);
 * serving: continuous batching of an open-loop request stream, against the
   plain FP64 one-at-a-time path on the same arrivals;
@@ -905,7 +905,7 @@ def main():
         "roofline": {
             "bound": "hbm",
             "kernel": "k_xline_batch_* FP32 (finest-level line relaxation, even rows, of all 1024 problems: "
-                      "one launch per chunk class, side by side)",
+                      "launched as inside a solve)",
             "achieved": achieved,
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",

@@ -397,8 +397,8 @@ int mgp_batch_solve(mgp_batch *b, double tol, int maxiters, int zerophi, int *it
 /* V-cycle applications of the longest-running problem in the last solve. */
 int mgp_batch_last_cycles(const mgp_batch *b);
 /* Measurement hook (between solves): times `reps` back-to-back launch sets of the finest-level
- * line relaxation of the even interior rows of every problem (kernel 0; one launch per chunk
- * class, side by side, as inside a solve) with HIP events on the batch's stream.  *avg_ms is the
+ * line relaxation of the even interior rows of every problem (kernel 0; launched as inside a
+ * solve) with HIP events on the batch's stream.  *avg_ms is the
  * mean per set, *bytes the algorithmic bytes of one set (each array element it needs once, at
  * the element size of the cycle: 8 bytes, or 4 with KRYLOV_MG32).  Changes the resident
  * finest-level corrections, nothing else. */

@@ -8,6 +8,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <map>
 #include <memory>
 #include <vector>
 
@@ -59,6 +60,13 @@ struct XlTask {
     int lev, row, side, save;
 };
 
+// A workgroup of the mixed line launch: tasks first .. first + count - 1, of one
+// class (chunk length and threads per row).
+struct XlBlock {
+    int first, count, cls, pad;
+};
+__host__ __device__ constexpr int xl_class(int C, int threads) { return C * 1024 + threads; }
+
 // Cell tile: cells (64 tx .. 64 tx + 63, BT_ROWS ty .. BT_ROWS ty + 15) of
 // item `item` (a problem or a level, as the kernel says), each thread of a
 // 256-thread workgroup taking four rows 4 apart; for reductions, tx is the
@@ -74,6 +82,9 @@ struct BTile {
 // fp32: the FP32 fields of the levels (e32/f32, geo32, K32) instead of e[sel]/f[sel]
 void launch_xline_batch(hipStream_t s, const XlTask *tasks, int ntasks, const BLev *levs, const int *active, int sel,
                         int C, int threads, size_t lds, int k, bool fp32);
+// the same for tasks of several classes in one launch
+void launch_xline_mixed(hipStream_t s, const XlBlock *blocks, int nblocks, const XlTask *tasks, const BLev *levs,
+                        const int *active, int sel, size_t lds, int k, bool fp32);
 // coarse (lev+1) r = 1x2 restriction of f - L e on lev, coarse e = 0; tiles over the coarse cells
 void launch_restrict_batch(hipStream_t s, const BTile *tiles, int ntiles, const BLev *levs, const int *active,
                            int sel, bool fp32);
@@ -126,8 +137,7 @@ class BatchKMG {
     static size_t problem_bytes(const Problem &q, const mgp_solver_opts &o);
     // Measurement hook: mean ms of `reps` back-to-back launch sets of the
     // finest-level line relaxation of the even interior rows of every problem
-    // (one launch per chunk class, side by side, as in a solve), timed with
-    // HIP events on the batch's stream; *bytes the algorithmic bytes of one
+    // (as in a solve), timed with HIP events on the batch's stream; *bytes the algorithmic bytes of one
     // set (each array element it needs once, the element size of the cycle).
     // Between solves only: it relaxes the resident finest-level corrections.
     double time_fine_xline(int reps, double *bytes);
@@ -180,31 +190,36 @@ class BatchKMG {
     BProb *dP = nullptr;
     BLev *dL = nullptr;
     int *active = nullptr, *mask = nullptr;
-    // The x-line launches of one phase (one per chunk class) cover different
-    // problems: they run side by side on streams forked from s and joined
-    // back (in the captured iteration, parallel branches).
-    std::vector<hipStream_t> aux;
-    hipEvent_t fork_ev = nullptr;
-    std::vector<hipEvent_t> join_ev;
     double *host_sc = nullptr;  // pinned: all problems' scalars
     // launch tables (device) with their lengths
     struct Table {
         void *p = nullptr;
         int n = 0;
-        int C = 0;        // x-line tables: chunk length
-        int threads = 0;  // x-line tables: threads per row
-        size_t lds = 0;   // x-line tables: dynamic LDS
     };
     enum { SET_MID = 0, SET_BOTTOM = 1 };
-    struct XlTable {
+    // One phase of the line relaxation (level, set, colour): its row tasks by
+    // class, and the workgroups of the launch that takes them all.
+    struct XlClass {
+        int C, threads, first, n;
+        size_t lds;
+    };
+    struct XlPhase {
         int d, set, colour;
-        Table t;
+        Table tasks, blocks;
+        std::vector<XlClass> cls;
+        size_t lds = 0;  // of a mixed workgroup
+    };
+    // Rows of a phase with their shapes, grouped by class.
+    struct XlRows {
+        std::map<std::pair<int, int>, std::vector<XlTask>> tasks;  // (C, threads)
+        std::map<std::pair<int, int>, size_t> lds;
+        void add(int C, int threads, size_t bytes, const XlTask &t);
     };
     // the launch tables of a set of problems, with the captured iteration
     struct TableSet {
         Table t0;                    // finest-level tiles, item = problem
         Table tred;                  // reduction row blocks, item = problem (tx = block)
-        std::vector<XlTable> xl;     // x-line task tables per (level, set, colour, chunk class)
+        std::vector<XlPhase> xl;     // line relaxation phases per (level, set, colour)
         std::vector<Table> tr, tp;   // per level: restriction (coarse tiles) / prolongation (fine tiles)
         std::vector<int> bottom;     // per level: most coarsest-level sweeps of a problem ending there
         hipGraphExec_t graph = nullptr;
@@ -217,6 +232,9 @@ class BatchKMG {
         size_t dcap = 0, hcap = 0, used = 0;
     };
     Table stage(TableSet &ts, const void *host, size_t bytes, int n);
+    XlPhase stage_phase(TableSet &ts, int d, int set, int colour, const XlRows &rows);
+    void upload(TableSet &ts);
+    void launch_phase(const XlPhase &ph, int sel, int k);
     void build_tables(TableSet &ts, const std::vector<int> &which);
     void release(TableSet &ts);       // the graph and the tables' contents (waits for the stream)
     void free_buffers(TableSet &ts);  // and the buffers

@@ -21,7 +21,6 @@
 #include <map>
 #include <string>
 #include <thread>
-#include <tuple>
 
 #include "mgp_batch.h"
 #include "mgp_geometry.h"
@@ -497,21 +496,6 @@ BatchKMG::BatchKMG(hipStream_t s_, const std::vector<Problem> &probs, const mgp_
     mask = static_cast<int *>(dev_alloc_zero(n * sizeof(int)));
     hip_check(hipHostMalloc((void **)&host_sc, (size_t)n * SC_COUNT * sizeof(double)), "hipHostMalloc");
     use_graph = o.use_graph != 0;
-    {
-        // streams for the chunk classes of a phase (default priority)
-        std::map<int, int> classes;
-        for (int p = 0; p < n; ++p) classes[Cp[p] * 1024 + NTp[p]] = 1;
-        const int nc = (int)classes.size();
-        hip_check(hipEventCreateWithFlags(&fork_ev, hipEventDisableTiming), "hipEventCreate");
-        for (int c = 0; c < nc; ++c) {
-            hipStream_t st = nullptr;
-            hip_check(hipStreamCreateWithFlags(&st, hipStreamNonBlocking), "hipStreamCreate");
-            aux.push_back(st);
-            hipEvent_t ev = nullptr;
-            hip_check(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "hipEventCreate");
-            join_ev.push_back(ev);
-        }
-    }
     act_.assign(n, 0);
     it_.assign(n, 0);
     oc_.assign(n, MGP_MAXITERS);
@@ -543,8 +527,7 @@ void BatchKMG::build_tables(TableSet &ts, const std::vector<int> &which) {
     ts.tp.assign(ts.depth, Table());
     ts.bottom.assign(ts.depth, 0);
     for (int d = 0; d < ts.depth; ++d) {
-        std::map<std::tuple<int, int, int, int>, std::vector<XlTask>> tabs;  // (set, colour, C, threads)
-        std::map<std::tuple<int, int, int, int>, size_t> lds;
+        std::map<std::pair<int, int>, XlRows> phases;  // (set, colour)
         std::vector<BTile> trh, tph;
         for (int p : which) {
             if (d >= nlev[p]) continue;
@@ -554,60 +537,24 @@ void BatchKMG::build_tables(TableSet &ts, const std::vector<int> &which) {
             const int C = Cp[p], NT = NTp[p];
             if (set == SET_BOTTOM) ts.bottom[d] = std::max(ts.bottom[d], L[lev].sweeps);
             const size_t need = xline_lds_bytes_for(nx, C, mixed ? sizeof(float) : sizeof(double), NT);
-            auto table = [&](int colour) -> std::vector<XlTask> & {
-                const auto key = std::make_tuple(set, colour, C, NT);
-                size_t &b = lds[key];
-                b = std::max(b, need);
-                return tabs[key];
-            };
             // the order of the single-problem sweep: even rows, odd rows, each
             // launch saving the far rows of the other colour
             for (int colour = 0; colour < 2; ++colour) {
-                std::vector<XlTask> &v = table(colour);
-                for (int j = colour; j < ny; j += 2) v.push_back(XlTask{lev, j, 0, 0});
-                if (colour == 1) v.push_back(XlTask{lev, 2, 0, 1});
-                if (((ny - 3) & 1) != colour) v.push_back(XlTask{lev, ny - 3, 1, 1});
+                XlRows &v = phases[{set, colour}];
+                for (int j = colour; j < ny; j += 2) v.add(C, NT, need, XlTask{lev, j, 0, 0});
+                if (colour == 1) v.add(C, NT, need, XlTask{lev, 2, 0, 1});
+                if (((ny - 3) & 1) != colour) v.add(C, NT, need, XlTask{lev, ny - 3, 1, 1});
             }
             if (set == SET_MID) {
                 tiles_of(trh, lev, nx, L[lev + 1].g.ny);
                 tiles_of(tph, lev, nx, ny);
             }
         }
-        for (auto &kv : tabs) {
-            XlTable x;
-            x.d = d;
-            x.set = std::get<0>(kv.first);
-            x.colour = std::get<1>(kv.first);
-            x.t = stage(ts, kv.second.data(), kv.second.size() * sizeof(XlTask), (int)kv.second.size());
-            x.t.C = std::get<2>(kv.first);
-            x.t.threads = std::get<3>(kv.first);
-            x.t.lds = lds[kv.first];
-            ts.xl.push_back(x);
-        }
+        for (const auto &kv : phases) ts.xl.push_back(stage_phase(ts, d, kv.first.first, kv.first.second, kv.second));
         ts.tr[d] = stage(ts, trh.data(), trh.size() * sizeof(BTile), (int)trh.size());
         ts.tp[d] = stage(ts, tph.data(), tph.size() * sizeof(BTile), (int)tph.size());
     }
-    // one upload of the staged set; the offsets become device addresses
-    if (ts.used > ts.dcap) {
-        if (ts.dev) dev_free(ts.dev);
-        ts.dev = nullptr;
-        ts.dcap = 0;
-        ts.dev = dev_alloc_zero(ts.used);
-        ts.dcap = ts.used;
-    }
-    auto place = [&](Table &t) {
-        if (t.n) t.p = static_cast<unsigned char *>(ts.dev) + reinterpret_cast<size_t>(t.p);
-    };
-    place(ts.t0);
-    place(ts.tred);
-    for (XlTable &x : ts.xl) place(x.t);
-    for (Table &t : ts.tr) place(t);
-    for (Table &t : ts.tp) place(t);
-    if (ts.used) hip_check(hipMemcpyAsync(ts.dev, ts.host, ts.used, hipMemcpyHostToDevice, s), "table upload");
-    std::sort(ts.xl.begin(), ts.xl.end(), [](const XlTable &a, const XlTable &b) {
-        return std::make_tuple(a.d, a.set, a.colour, a.t.C, a.t.threads) <
-               std::make_tuple(b.d, b.set, b.colour, b.t.C, b.t.threads);
-    });
+    upload(ts);
     hip_check(hipStreamSynchronize(s), "batch tables");
     if (use_graph) {
         TableSet *const saved = T;
@@ -627,6 +574,79 @@ void BatchKMG::build_tables(TableSet &ts, const std::vector<int> &which) {
         hip_check(hipGraphInstantiate(&ts.graph, g, nullptr, nullptr, 0), "graph instantiate");
         (void)hipGraphDestroy(g);
     }
+}
+
+void BatchKMG::XlRows::add(int C, int threads, size_t bytes, const XlTask &t) {
+    const std::pair<int, int> key{C, threads};
+    tasks[key].push_back(t);
+    lds[key] = std::max(lds[key], bytes);
+}
+
+// The tables of one phase: the tasks class by class, and the workgroups of
+// the mixed launch (each holds rows of one class).
+BatchKMG::XlPhase BatchKMG::stage_phase(TableSet &ts, int d, int set, int colour, const XlRows &rows) {
+    XlPhase ph;
+    ph.d = d;
+    ph.set = set;
+    ph.colour = colour;
+    std::vector<XlTask> tasks;
+    std::vector<XlBlock> blocks;
+    for (const auto &kv : rows.tasks) {
+        const int C = kv.first.first, threads = kv.first.second, per = xline_block_rows(threads);
+        const int first = (int)tasks.size(), n = (int)kv.second.size();
+        ph.cls.push_back(XlClass{C, threads, first, n, rows.lds.at(kv.first)});
+        tasks.insert(tasks.end(), kv.second.begin(), kv.second.end());
+        for (int k = 0; k < n; k += per)
+            blocks.push_back(XlBlock{first + k, std::min(per, n - k), xl_class(C, threads), 0});
+        ph.lds = std::max(ph.lds, xline_block_lds(C, threads, mixed ? sizeof(float) : sizeof(double)));
+    }
+    ph.tasks = stage(ts, tasks.data(), tasks.size() * sizeof(XlTask), (int)tasks.size());
+    ph.blocks = stage(ts, blocks.data(), blocks.size() * sizeof(XlBlock), (int)blocks.size());
+    return ph;
+}
+
+// One upload of the staged set; the tables' offsets become device addresses.
+void BatchKMG::upload(TableSet &ts) {
+    if (ts.used > ts.dcap) {
+        if (ts.dev) dev_free(ts.dev);
+        ts.dev = nullptr;
+        ts.dcap = 0;
+        ts.dev = dev_alloc_zero(ts.used);
+        ts.dcap = ts.used;
+    }
+    auto place = [&](Table &t) {
+        if (t.n) t.p = static_cast<unsigned char *>(ts.dev) + reinterpret_cast<size_t>(t.p);
+    };
+    place(ts.t0);
+    place(ts.tred);
+    for (XlPhase &x : ts.xl) {
+        place(x.tasks);
+        place(x.blocks);
+    }
+    for (Table &t : ts.tr) place(t);
+    for (Table &t : ts.tp) place(t);
+    if (ts.used) hip_check(hipMemcpyAsync(ts.dev, ts.host, ts.used, hipMemcpyHostToDevice, s), "table upload");
+}
+
+// The rows of one phase: one launch of all classes up to 1024 workgroups, four
+// per CU, past that one launch per class.  The classes' launches one after the
+// other, or side by side on forked streams, cost a coarse level a row solve or
+// a fork and a join each; the mixed launch has the registers and the LDS of its
+// largest class, which costs the short rows occupancy where there are many.
+// Solves, mixed never / up to 1024 / always: 24 problems of 33..400 cells in
+// FP64 47 / 41 / 41 ms (forked streams 53..114), 38 of 64..990 in FP64 153 / 123
+// / 132, 256 of 32..1024 in FP32 263 / 218 / 245.
+constexpr int XL_MIXED_MAX_BLOCKS = 1024;
+
+void BatchKMG::launch_phase(const XlPhase &ph, int sel, int k) {
+    if (ph.cls.size() > 1 && ph.blocks.n <= XL_MIXED_MAX_BLOCKS) {
+        launch_xline_mixed(s, (const XlBlock *)ph.blocks.p, ph.blocks.n, (const XlTask *)ph.tasks.p, dL, active, sel,
+                           ph.lds, k, mixed);
+        return;
+    }
+    for (const XlClass &c : ph.cls)
+        launch_xline_batch(s, (const XlTask *)ph.tasks.p + c.first, c.n, dL, active, sel, c.C, c.threads, c.lds, k,
+                           mixed);
 }
 
 void BatchKMG::release(TableSet &ts) {
@@ -654,12 +674,6 @@ void BatchKMG::free_buffers(TableSet &ts) {
 BatchKMG::~BatchKMG() {
     free_buffers(part);
     free_buffers(full);
-    for (hipStream_t st : aux) {
-        (void)hipStreamSynchronize(st);
-        (void)hipStreamDestroy(st);
-    }
-    for (hipEvent_t ev : join_ev) (void)hipEventDestroy(ev);
-    if (fork_ev) (void)hipEventDestroy(fork_ev);
     if (dP) dev_free(dP);
     if (dL) dev_free(dL);
     if (active) dev_free(active);
@@ -670,27 +684,8 @@ BatchKMG::~BatchKMG() {
 }
 
 void BatchKMG::zebra(int d, int set, int sel, int k) {
-    for (int colour = 0; colour < 2; ++colour) {
-        std::vector<const XlTable *> tabs;
-        for (const XlTable &x : T->xl)
-            if (x.d == d && x.set == set && x.colour == colour) tabs.push_back(&x);
-        if (tabs.empty()) continue;
-        if (tabs.size() == 1 || tabs.size() > aux.size()) {
-            for (const XlTable *x : tabs)
-                launch_xline_batch(s, (const XlTask *)x->t.p, x->t.n, dL, active, sel, x->t.C, x->t.threads,
-                                   x->t.lds, k, mixed);
-            continue;
-        }
-        // one launch per chunk class, side by side
-        hip_check(hipEventRecord(fork_ev, s), "fork");
-        for (size_t i = 0; i < tabs.size(); ++i) {
-            hip_check(hipStreamWaitEvent(aux[i], fork_ev, 0), "fork wait");
-            launch_xline_batch(aux[i], (const XlTask *)tabs[i]->t.p, tabs[i]->t.n, dL, active, sel, tabs[i]->t.C,
-                               tabs[i]->t.threads, tabs[i]->t.lds, k, mixed);
-            hip_check(hipEventRecord(join_ev[i], aux[i]), "join");
-        }
-        for (size_t i = 0; i < tabs.size(); ++i) hip_check(hipStreamWaitEvent(s, join_ev[i], 0), "join wait");
-    }
+    for (const XlPhase &x : T->xl)  // even rows before odd ones (build_tables' order)
+        if (x.d == d && x.set == set) launch_phase(x, sel, k);
 }
 
 // e = M f for the pair `sel` of every active problem (phat from p: 0, shat
@@ -900,9 +895,6 @@ double BatchKMG::time_fine_xline(int reps, double *bytes) {
     const int n = count();
     // the even rows of level 0 (colour 0 of the first zebra phase; the bytes
     // count its interior rows)
-    std::vector<const XlTable *> tabs;
-    for (const XlTable &x : T->xl)
-        if (x.d == 0 && x.set == SET_MID && x.colour == 0) tabs.push_back(&x);
     const double es = mixed ? 4.0 : 8.0;
     double b = 0.0;
     for (int p = 0; p < n; ++p) {
@@ -917,20 +909,8 @@ double BatchKMG::time_fine_xline(int reps, double *bytes) {
     std::vector<int> all(n, 1);
     upload_flags(active, all);
     auto launch_set = [&]() {
-        if (tabs.size() == 1 || tabs.size() > aux.size()) {
-            for (const XlTable *x : tabs)
-                launch_xline_batch(s, (const XlTask *)x->t.p, x->t.n, dL, active, 0, x->t.C, x->t.threads, x->t.lds,
-                                   -1, mixed);
-            return;
-        }
-        hip_check(hipEventRecord(fork_ev, s), "fork");
-        for (size_t i = 0; i < tabs.size(); ++i) {
-            hip_check(hipStreamWaitEvent(aux[i], fork_ev, 0), "fork wait");
-            launch_xline_batch(aux[i], (const XlTask *)tabs[i]->t.p, tabs[i]->t.n, dL, active, 0, tabs[i]->t.C,
-                               tabs[i]->t.threads, tabs[i]->t.lds, -1, mixed);
-            hip_check(hipEventRecord(join_ev[i], aux[i]), "join");
-        }
-        for (size_t i = 0; i < tabs.size(); ++i) hip_check(hipStreamWaitEvent(s, join_ev[i], 0), "join wait");
+        for (const XlPhase &x : T->xl)
+            if (x.d == 0 && x.set == SET_MID && x.colour == 0) launch_phase(x, 0, -1);
     };
     hipEvent_t a = nullptr, e = nullptr;
     hip_check(hipEventCreate(&a), "event");
@@ -964,23 +944,13 @@ std::vector<BatchKMG::TuneEntry> BatchKMG::tuning() const {
     return out;
 }
 
-// After a change of shapes: the level table's chunk counts, enough streams
-// for the chunk classes of a phase, the launch tables and the captured graph.
+// After a change of shapes: the level table's chunk counts, the launch tables
+// and the captured graph.
 void BatchKMG::apply_shapes() {
     const int n = count();
     for (int p = 0; p < n; ++p)
         for (int d = 0; d < nlev[p]; ++d) L[P[p].lev0 + d].nt = P[p].g.nx / Cp[p];
     hip_check(hipMemcpyAsync(dL, L.data(), L.size() * sizeof(BLev), hipMemcpyHostToDevice, s), "level table");
-    std::map<int, int> classes;
-    for (int p = 0; p < n; ++p) classes[Cp[p] * 1024 + NTp[p]] = 1;
-    while (aux.size() < classes.size()) {
-        hipStream_t st = nullptr;
-        hip_check(hipStreamCreateWithFlags(&st, hipStreamNonBlocking), "hipStreamCreate");
-        aux.push_back(st);
-        hipEvent_t ev = nullptr;
-        hip_check(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "hipEventCreate");
-        join_ev.push_back(ev);
-    }
     release(part);
     release(full);
     T = &full;
@@ -1013,54 +983,23 @@ int BatchKMG::set_tuning(const std::vector<TuneEntry> &t) {
 }
 
 // Mean ms of `reps` launch sets of the finest-level even-row line relaxation
-// of every problem with shapes (C[p], NT[p]): one launch per chunk class, side
-// by side on the forked streams, as inside a solve.  Sets the level table's
+// of every problem with shapes (C[p], NT[p]), launched as inside a solve.  Sets the level table's
 // finest-level chunk counts to those shapes (apply_shapes restores them).
 double BatchKMG::time_shapes(const std::vector<int> &C, const std::vector<int> &NT, int reps) {
     const int n = count();
     const size_t elem = mixed ? sizeof(float) : sizeof(double);
-    std::map<std::pair<int, int>, std::vector<XlTask>> cls;
-    std::map<std::pair<int, int>, size_t> lds;
+    XlRows rows;
     for (int p = 0; p < n; ++p) {
         const int nx = P[p].g.nx, ny = P[p].g.ny, lev = P[p].lev0;
         L[lev].nt = nx / C[p];
-        if (ny < 4) continue;
-        auto &t = cls[{C[p], NT[p]}];
-        for (int k = 0; k < (ny - 4) / 2 + 1; ++k) t.push_back(XlTask{lev, 2 + 2 * k, 0, 0});
-        size_t &l = lds[{C[p], NT[p]}];
-        l = std::max(l, xline_lds_bytes_for(nx, C[p], elem, NT[p]));
+        for (int j = 2; j < ny - 1; j += 2)
+            rows.add(C[p], NT[p], xline_lds_bytes_for(nx, C[p], elem, NT[p]), XlTask{lev, j, 0, 0});
     }
     hip_check(hipMemcpyAsync(dL, L.data(), L.size() * sizeof(BLev), hipMemcpyHostToDevice, s), "level table");
-    while (aux.size() < cls.size()) {
-        hipStream_t st = nullptr;
-        hip_check(hipStreamCreateWithFlags(&st, hipStreamNonBlocking), "hipStreamCreate");
-        aux.push_back(st);
-        hipEvent_t ev = nullptr;
-        hip_check(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "hipEventCreate");
-        join_ev.push_back(ev);
-    }
-    struct Cls {
-        void *t;
-        int n, C, NT;
-        size_t lds;
-    };
-    std::vector<Cls> v;
-    for (auto &kv : cls) {
-        void *d = dev_alloc_zero(kv.second.size() * sizeof(XlTask));
-        v.push_back(Cls{d, (int)kv.second.size(), kv.first.first, kv.first.second, lds[kv.first]});
-        hip_check(hipMemcpyAsync(d, kv.second.data(), kv.second.size() * sizeof(XlTask), hipMemcpyHostToDevice, s),
-                  "tasks");
-    }
-    auto launch_set = [&]() {
-        hip_check(hipEventRecord(fork_ev, s), "fork");
-        for (size_t i = 0; i < v.size(); ++i) {
-            hip_check(hipStreamWaitEvent(aux[i], fork_ev, 0), "fork wait");
-            launch_xline_batch(aux[i], (const XlTask *)v[i].t, v[i].n, dL, active, 0, v[i].C, v[i].NT, v[i].lds, -1,
-                               mixed);
-            hip_check(hipEventRecord(join_ev[i], aux[i]), "join");
-        }
-        for (size_t i = 0; i < v.size(); ++i) hip_check(hipStreamWaitEvent(s, join_ev[i], 0), "join wait");
-    };
+    TableSet ts;
+    ts.xl.push_back(stage_phase(ts, 0, SET_MID, 0, rows));
+    upload(ts);
+    auto launch_set = [&]() { launch_phase(ts.xl[0], 0, -1); };
     hipEvent_t a = nullptr, e = nullptr;
     float ms = 0.0f;
     try {
@@ -1073,14 +1012,12 @@ double BatchKMG::time_shapes(const std::vector<int> &C, const std::vector<int> &
         hip_check(hipEventSynchronize(e), "event");
         hip_check(hipEventElapsedTime(&ms, a, e), "event");
     } catch (...) {
-        (void)hipStreamSynchronize(s);
-        for (Cls &c : v) dev_free(c.t);
+        free_buffers(ts);
         if (a) (void)hipEventDestroy(a);
         if (e) (void)hipEventDestroy(e);
         throw;
     }
-    hip_check(hipStreamSynchronize(s), "sync");
-    for (Cls &c : v) dev_free(c.t);
+    free_buffers(ts);
     (void)hipEventDestroy(a);
     (void)hipEventDestroy(e);
     return ms / reps;

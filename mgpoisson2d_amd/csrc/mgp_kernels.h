@@ -188,6 +188,10 @@ int xline_batch_chunk(int nx, int threads, size_t elem);
 size_t xline_lds_bytes(int nx, size_t elem);
 // the same for chunk length C and `threads` threads per row
 size_t xline_lds_bytes_for(int nx, int C, size_t elem, int threads);
+// Rows of `threads` threads that a workgroup of the mixed batched launch holds,
+// and its LDS for rows of chunk length C.
+int xline_block_rows(int threads);
+size_t xline_block_lds(int C, int threads, size_t elem);
 // Relax rows j = row0 + k*rowstep, k < nrows (one workgroup each; interior
 // rows of a launch are at least two apart, so none reads another).  far: the
 // copies that rows 0 and ny-1 read their far row from, and the rows this

@@ -205,6 +205,11 @@ __device__ __forceinline__ int launch_slot() {
     return x * q8 + (x < r8 ? x : r8) + (b >> 3);
 }
 
+// LDS elements of a row of NT full chunks (xline_lds_bytes_for).
+__host__ __device__ constexpr int row_lds_elems(int C, int NT) {
+    return 4 * NT * (C + 1) > NT * (C + 1) + 8 * NT ? 4 * NT * (C + 1) : NT * (C + 1) + 8 * NT;
+}
+
 template <typename T>
 struct RowCtx {
     int nx, ny, P, nt, rem, nring;
@@ -267,13 +272,13 @@ struct Buf {
 
 template <int C, int NT, bool SEG = false, int RG = 1, typename T, typename GM>
 __device__ __forceinline__ void row_pass(const RowCtx<T> &X, const T *e_, const T *f_, const T *K_, const Grid &g,
-                                         const GM &geo_, int j, const T *far, T *Ld, T *La, T *Lb, T *Lc,
+                                         const GM &geo_, int j, const T *far, int tid, T *Ld, T *La, T *Lb, T *Lc,
                                          T (&ev)[C + 1]) {
     constexpr int U = C + 1;
     gconst<T> *e = gptr(e_), *f = gptr(f_), *K = gptr(K_);
     // SEG: the cells solved may be a segment of the row (xline_rows); whole
     // rows compile without the segment terms
-    const int tid = threadIdx.x, nx = X.nx, ny = X.ny, P = X.P, i0 = SEG ? X.i0 : 0, nxg = SEG ? X.nxg : X.nx;
+    const int nx = X.nx, ny = X.ny, P = X.P, i0 = SEG ? X.i0 : 0, nxg = SEG ? X.nxg : X.nx;
     const T fourth = T(0.25);
     const int dump = X.nt * (C + 1) - 1;
     // A segment of a longer row is solved as a line of its own: its couplings
@@ -384,11 +389,12 @@ constexpr bool keep_values() {
 }
 
 template <int C, int NT, bool SEG = false, typename T>
-__device__ __forceinline__ void row_update_add(const RowCtx<T> &X, T *e_, int j, const T *Lx, const T (&ev)[C + 1]) {
+__device__ __forceinline__ void row_update_add(const RowCtx<T> &X, T *e_, int j, int tid, const T *Lx,
+                                               const T (&ev)[C + 1]) {
     __attribute__((address_space(1))) T *e = (__attribute__((address_space(1))) T *)e_;
 #pragma unroll
     for (int u = 0; u < C + 1; ++u) {
-        const int i = threadIdx.x + NT * u;
+        const int i = tid + NT * u;
         if (i >= X.nx) continue;
         const size_t c = ix(X.P, (SEG ? X.i0 : 0) + i, j);
         e[c] = (keep_values<C, SEG>() ? ev[u] : e[c]) + Lx[chunk_pos<C>(i, X.rem)];
@@ -535,16 +541,29 @@ __device__ __forceinline__ void interface_solve(const T *I, T *X, int nt, int l)
 // interface solve and back substitution per call.
 // LDS: 4 nt (C+1) elements, or nt (C+1) + 8 NT (rows of more than one wave).
 // ---------------------------------------------------------------------------
-template <int C, int NT, bool SEG = false, int RG = 1, typename T, typename GM>
-__device__ void xline_row(const RowCtx<T> &X, T *__restrict__ e, const T *__restrict__ f, const T *__restrict__ K,
-                          const Grid &g, const GM &geo, int j, const T *far, T *lds) {
+// Barrier of a row's NT threads.  ALONE: they are the workgroup; else the
+// workgroup holds 256 / NT rows of the same NT, which pass the barriers
+// together (waves that have ended do not count), a row of one wave by itself.
+template <int NT, bool ALONE>
+__device__ __forceinline__ void row_sync() {
+    if (!ALONE && NT == 64) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    } else {
+        __syncthreads();
+    }
+}
+
+template <int C, int NT, bool SEG = false, int RG = 1, bool ALONE = true, typename T, typename GM>
+__device__ __forceinline__ void xline_row(const RowCtx<T> &X, T *__restrict__ e, const T *__restrict__ f, const T *__restrict__ K,
+                          const Grid &g, const GM &geo, int j, const T *far, int tid, T *lds) {
     constexpr int CP = C + 1;
-    const int tid = threadIdx.x, nt = X.nt;
+    const int nt = X.nt;
     const int NT1 = nt * CP;
     T *Ld = lds, *Lb = lds + NT1, *La = lds + 2 * NT1, *Lc = lds + 3 * NT1;
     T ev[CP];
-    row_pass<C, NT, SEG, RG>(X, e, f, K, g, geo, j, far, Ld, La, Lb, Lc, ev);
-    __syncthreads();
+    row_pass<C, NT, SEG, RG>(X, e, f, K, g, geo, j, far, tid, Ld, La, Lb, Lc, ev);
+    row_sync<NT, ALONE>();
 
     // each thread takes its chunk into registers
     T ca[CP], cb[CP], cc[CP], cd[CP];
@@ -557,7 +576,7 @@ __device__ void xline_row(const RowCtx<T> &X, T *__restrict__ e, const T *__rest
             ca[k] = La[tid * CP + k];
             cc[k] = Lc[tid * CP + k];
         }
-    __syncthreads();
+    row_sync<NT, ALONE>();
 
     // chunks past the row's end are identity rows
     Row4<T> last{0, 1, 0, 0};
@@ -584,9 +603,9 @@ __device__ void xline_row(const RowCtx<T> &X, T *__restrict__ e, const T *__rest
         I[4 * NT + q] = g0;
         I[5 * NT + q] = h0;
         I[6 * NT + q] = m0;
-        __syncthreads();
+        row_sync<NT, ALONE>();
         if (tid < 64) interface_solve<NT>(I, IX, nt, tid);
-        __syncthreads();
+        row_sync<NT, ALONE>();
         xe = IX[tid];
         xp = tid ? IX[tid - 1] : T(0);
     }
@@ -599,14 +618,14 @@ __device__ void xline_row(const RowCtx<T> &X, T *__restrict__ e, const T *__rest
             if (k <= len - 2) lds[tid * CP + k] = cd[k] + ca[k] * xp + cc[k] * xe;
         lds[tid * CP + (longc ? C : C - 1)] = xe;
     }
-    __syncthreads();
-    row_update_add<C, NT, SEG>(X, e, j, lds, ev);
+    row_sync<NT, ALONE>();
+    row_update_add<C, NT, SEG>(X, e, j, tid, lds, ev);
 }
 
 // Row `row` of e into `to` (XlFar).
 template <int NT, typename T>
-__device__ __forceinline__ void save_row(T *to, const T *e, const Grid &g, int row) {
-    for (int i = threadIdx.x; i < g.nx; i += NT) to[OFFX + i] = e[ix(g.pitch, i, row)];
+__device__ __forceinline__ void save_row(T *to, const T *e, const Grid &g, int row, int tid) {
+    for (int i = tid; i < g.nx; i += NT) to[OFFX + i] = e[ix(g.pitch, i, row)];
 }
 
 // Rows j = row0 + slot*rowstep, one workgroup each; the workgroups past the
@@ -630,7 +649,8 @@ __device__ __forceinline__ void xline_rows(T *__restrict__ e, const T *__restric
     int slot = launch_slot();
     if (slot >= nrows * nsegl) {
         const bool first = slot == nrows * nsegl && far.save[0] >= 0;
-        save_row<NT>(first ? far.to[0] : far.to[1], e, g, first ? far.save[0] : far.save[1]);
+        save_row<NT>(first ? far.to[0] : far.to[1], e, g, first ? far.save[0] : far.save[1],
+                     (int)threadIdx.x);
         return;
     }
     if (SEG) {
@@ -640,7 +660,7 @@ __device__ __forceinline__ void xline_rows(T *__restrict__ e, const T *__restric
         slot /= nsegl;
     }
     const int j = row0 + slot * rowstep;
-    xline_row<C, NT, SEG, RG>(X, e, f, K, g, geo, j, j == 0 ? far.lo : far.hi, lds);
+    xline_row<C, NT, SEG, RG>(X, e, f, K, g, geo, j, j == 0 ? far.lo : far.hi, (int)threadIdx.x, lds);
 }
 
 // Waves per SIMD of the fine-level kernel: the LDS of one workgroup at
@@ -769,50 +789,88 @@ constexpr int batch_rg() {
     return sizeof(T) == 8 ? 2 : (C == 4 ? 3 : 2);
 }
 
-template <int C, int NT, typename T>
-__device__ __forceinline__ void xline_task(const XlTask *tasks, const BLev *levs, const int *active, int sel, int k) {
-    const XlTask t = tasks[launch_slot()];
+template <int C, int NT, bool ALONE, typename T>
+__device__ __forceinline__ void xline_task(const XlTask &t, const BLev *levs, const int *active, int sel, int k, int tid,
+                                           T *lds) {
     const BLev *L = levs + t.lev;
     if (!active[L->prob] || (k >= 0 && k >= L->sweeps)) return;
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds_bytes[];
-    T *lds = reinterpret_cast<T *>(lds_bytes);
     const Grid g = L->g;
     T *e, *far;
     const T *f, *K;
     typename std::conditional<sizeof(T) == 8, Geo, GeoF>::type geo;
     level_fields(L, sel, e, f, K, far, geo);
     if (t.save) {
-        save_row<NT>(far + t.side * g.pitch, (const T *)e, g, t.row);
+        save_row<NT>(far + t.side * g.pitch, (const T *)e, g, t.row, tid);
         return;
     }
     const RowCtx<T> X = row_ctx<T>(g, L->nt, C);
-    xline_row<C, NT, false, batch_rg<C, T>()>(X, e, f, K, g, geo, t.row, t.row == 0 ? far : far + g.pitch, lds);
+    xline_row<C, NT, false, batch_rg<C, T>(), ALONE>(X, e, f, K, g, geo, t.row, t.row == 0 ? far : far + g.pitch, tid,
+                                                     lds);
+}
+
+template <int C, int NT, typename T>
+__device__ __forceinline__ void xline_alone(const XlTask *tasks, const BLev *levs, const int *active, int sel, int k) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds_bytes[];
+    xline_task<C, NT, true, T>(tasks[launch_slot()], levs, active, sel, k, (int)threadIdx.x,
+                               reinterpret_cast<T *>(lds_bytes));
 }
 
 template <int C, typename T>
 __global__ void __launch_bounds__(XL_THREADS) __attribute__((amdgpu_waves_per_eu(xl_waves<T>(), xl_waves<T>())))
 k_xline_batch(const XlTask *tasks, const BLev *levs, const int *active, int sel, int k) {
-    xline_task<C, XL_THREADS, T>(tasks, levs, active, sel, k);
+    xline_alone<C, XL_THREADS, T>(tasks, levs, active, sel, k);
 }
 
 template <int C, typename T>
 __global__ void __launch_bounds__(XL_THREADS) k_xline_batch_long(const XlTask *tasks, const BLev *levs,
                                                                  const int *active, int sel, int k) {
-    xline_task<C, XL_THREADS, T>(tasks, levs, active, sel, k);
+    xline_alone<C, XL_THREADS, T>(tasks, levs, active, sel, k);
 }
 
 // Short rows (nx <= 512): one wave per row.
 template <int C, typename T>
 __global__ void __launch_bounds__(XL_SHORT) __attribute__((amdgpu_waves_per_eu(2)))
 k_xline_batch_short(const XlTask *tasks, const BLev *levs, const int *active, int sel, int k) {
-    xline_task<C, XL_SHORT, T>(tasks, levs, active, sel, k);
+    xline_alone<C, XL_SHORT, T>(tasks, levs, active, sel, k);
 }
 
 // Rows of 513..1024 cells: two waves per row.
 template <int C, typename T>
 __global__ void __launch_bounds__(XL_MID) __attribute__((amdgpu_waves_per_eu(2)))
 k_xline_batch_mid(const XlTask *tasks, const BLev *levs, const int *active, int sel, int k) {
-    xline_task<C, XL_MID, T>(tasks, levs, active, sel, k);
+    xline_alone<C, XL_MID, T>(tasks, levs, active, sel, k);
+}
+
+// Rows of every width in one launch: a workgroup of 256 threads takes 4, 2 or
+// 1 rows of one class (XlBlock).  A phase's classes cover different problems,
+// and on the coarse levels each class's launch would cost one row solve (or,
+// side by side on several streams, a fork and a join) for a handful of rows.
+template <int C, int NT, typename T>
+__device__ __forceinline__ void xline_block(const XlBlock &b, const XlTask *tasks, const BLev *levs, const int *active,
+                                            int sel, int k, T *lds) {
+    const int sub = (int)threadIdx.x / NT, tid = (int)threadIdx.x % NT;
+    if (sub >= b.count) return;
+    xline_task<C, NT, NT == XL_THREADS, T>(tasks[b.first + sub], levs, active, sel, k, tid, lds + sub * row_lds_elems(C, NT));
+}
+
+template <typename T>
+__global__ void __launch_bounds__(XL_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
+k_xline_mixed(const XlBlock *blocks, const XlTask *tasks, const BLev *levs, const int *active, int sel, int k) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds_bytes[];
+    T *lds = reinterpret_cast<T *>(lds_bytes);
+    const XlBlock b = blocks[launch_slot()];
+    switch (b.cls) {
+        case xl_class(2, XL_SHORT): xline_block<2, XL_SHORT, T>(b, tasks, levs, active, sel, k, lds); break;
+        case xl_class(4, XL_SHORT): xline_block<4, XL_SHORT, T>(b, tasks, levs, active, sel, k, lds); break;
+        case xl_class(8, XL_SHORT): xline_block<8, XL_SHORT, T>(b, tasks, levs, active, sel, k, lds); break;
+        case xl_class(2, XL_MID): xline_block<2, XL_MID, T>(b, tasks, levs, active, sel, k, lds); break;
+        case xl_class(4, XL_MID): xline_block<4, XL_MID, T>(b, tasks, levs, active, sel, k, lds); break;
+        case xl_class(8, XL_MID): xline_block<8, XL_MID, T>(b, tasks, levs, active, sel, k, lds); break;
+        case xl_class(2, XL_THREADS): xline_block<2, XL_THREADS, T>(b, tasks, levs, active, sel, k, lds); break;
+        case xl_class(4, XL_THREADS): xline_block<4, XL_THREADS, T>(b, tasks, levs, active, sel, k, lds); break;
+        case xl_class(8, XL_THREADS): xline_block<8, XL_THREADS, T>(b, tasks, levs, active, sel, k, lds); break;
+        default: xline_block<16, XL_THREADS, T>(b, tasks, levs, active, sel, k, lds); break;
+    }
 }
 
 template <typename T>
@@ -884,6 +942,12 @@ size_t xline_lds_bytes_for(int nx, int C, size_t elem, int threads) {
     // chunk staging (4 arrays), or one chunk array plus the interface rows and unknowns
     const size_t tr = 4 * nt * (C + 1), iface = nt * (C + 1) + (threads > 64 ? 8 * (size_t)threads : 0);
     return (tr > iface ? tr : iface) * elem;
+}
+
+int xline_block_rows(int threads) { return XL_THREADS / threads; }
+
+size_t xline_block_lds(int C, int threads, size_t elem) {
+    return (size_t)xline_block_rows(threads) * row_lds_elems(C, threads) * elem;
 }
 
 bool xline_supported(int nx) { return xline_segments(nx, sizeof(double)) != 0; }
@@ -1052,6 +1116,18 @@ void launch_xline_batch(hipStream_t s, const XlTask *tasks, int ntasks, const BL
 void launch_xline(hipStream_t s, float *e, const float *f, const float *K, const Grid &g, const GeoF &geo, int row0,
                   int rowstep, int nrows, const XlFar<float> &far) {
     xline(s, e, f, K, g, geo, row0, rowstep, nrows, far);
+}
+
+void launch_xline_mixed(hipStream_t s, const XlBlock *blocks, int nblocks, const XlTask *tasks, const BLev *levs,
+                        const int *active, int sel, size_t lds, int k, bool fp32) {
+    if (nblocks <= 0) return;
+    if (fp32) k_xline_mixed<float><<<nblocks, XL_THREADS, lds, s>>>(blocks, tasks, levs, active, sel, k);
+    else k_xline_mixed<double><<<nblocks, XL_THREADS, lds, s>>>(blocks, tasks, levs, active, sel, k);
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) {
+        g_last_error = std::string("k_xline_mixed launch: ") + hipGetErrorString(err);
+        throw Failure(MGP_ERR_HIP);
+    }
 }
 
 void launch_restrict_batch(hipStream_t s, const BTile *tiles, int ntiles, const BLev *levs, const int *active,
