@@ -9,6 +9,7 @@
 #include <cmath>
 #include <cstring>
 #include <functional>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -79,10 +80,12 @@ void down_cc(hipStream_t s, double *h, const DevBuf &d, const Grid &g) { downloa
 
 struct Call {
     hipStream_t s;
+    std::unique_ptr<DevArena> arena;  // the metrics and the call's fields
     DevGeo geo;
     DevBc bc;
     Call(const mgp_geo *g, const mgp_bc *b) : s(thread_stream()) {
         check_geo(g);
+        arena = std::make_unique<DevArena>(10 * (level_elems(g->nx, g->ny) * sizeof(double) + 256));
         geo.upload(s, *g);
         if (b) {
             check_bc(b);
@@ -859,7 +862,8 @@ namespace {
 
 // Shared body of the two create calls: make_geo(stream) fills s->geo.
 template <class MakeGeo>
-int create_solver(mgp_solver **out, int nx, int ny, const mgp_bc *bc, const mgp_solver_opts *opts, MakeGeo make_geo,
+int create_solver(mgp_solver **out, int nx, int ny, double dx, double dy, const mgp_bc *bc,
+                  const mgp_solver_opts *opts, MakeGeo make_geo,
                   const mgp_mapping *map = nullptr) {
     *out = nullptr;
     mgp_solver *s = new mgp_solver;
@@ -879,6 +883,9 @@ int create_solver(mgp_solver **out, int nx, int ny, const mgp_bc *bc, const mgp_
             throw Failure(MGP_ERR_ARG);
         }
         hip_check(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking), "hipStreamCreate");
+        const bool krylov = o.method == MGP_METHOD_KRYLOV_MG || o.method == MGP_METHOD_KRYLOV_MG32;
+        const DevArena arena(7 * (level_elems(nx, ny) * sizeof(double) + 256) + 64 * (size_t)(nx + ny) +
+                             (krylov ? KrylovMG::bytes(nx, ny, o) : RefHierarchy::bytes(nx, ny, dx, dy, o.maxdepth)));
         make_geo(s->stream, s->geo);
         s->ubc.upload(s->stream, *bc, nx, ny);
         const size_t n = level_elems(nx, ny);
@@ -913,7 +920,7 @@ int mgp_solver_create(mgp_solver **out, const mgp_geo *geo, const mgp_bc *bc, co
         *out = nullptr;
         return st;
     }
-    return create_solver(out, geo->nx, geo->ny, bc, opts,
+    return create_solver(out, geo->nx, geo->ny, geo->dx, geo->dy, bc, opts,
                          [&](hipStream_t stream, DevGeo &dg) { dg.upload(stream, *geo); });
 }
 
@@ -932,7 +939,7 @@ int mgp_solver_create_mapped(mgp_solver **out, const mgp_mapping *m, int nx, int
         return st;
     }
     return create_solver(
-        out, nx, ny, bc, opts, [&](hipStream_t stream, DevGeo &dg) { dg.generate(stream, *m, nx, ny, dx, dy); }, m);
+        out, nx, ny, dx, dy, bc, opts, [&](hipStream_t stream, DevGeo &dg) { dg.generate(stream, *m, nx, ny, dx, dy); }, m);
 }
 
 int mgp_metric_fill(const mgp_mapping *m, int nx, int ny, double dx, double dy, double *J, double *Jxx, double *Jxy,

@@ -4,7 +4,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <memory>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "mgp2d.h"
@@ -26,28 +28,59 @@ void hip_check(hipError_t e, const char *what);
 void *dev_alloc_zero(size_t bytes);
 void dev_free(void *p);
 
+// One zero-filled device allocation that several arrays share; freed with the
+// last of them.
+struct DevBlock {
+    char *p = nullptr;
+    size_t bytes = 0, used = 0;
+    ~DevBlock() {
+        if (p) dev_free(p);
+    }
+};
+
+// While one exists, DevArr allocations of this thread come out of one block of
+// `bytes` as long as they fit (a solver makes some 80 arrays, and each
+// allocation of its own costs a hipMalloc, a fill, a wait for the device and a
+// hipFree).  Without the memory for the block, and past its end, arrays are
+// allocated one by one.
+class DevArena {
+  public:
+    explicit DevArena(size_t bytes);
+    ~DevArena();
+    DevArena(const DevArena &) = delete;
+    DevArena &operator=(const DevArena &) = delete;
+    // `bytes` of the current block (null: none, or no room), and the block
+    static void *take(size_t bytes, std::shared_ptr<DevBlock> &owner);
+
+  private:
+    std::shared_ptr<DevBlock> block, outer;
+};
+
 // Owning device allocation of `count` elements of T, zero-filled on allocation.
 template <typename T>
 struct DevArr {
     T *p = nullptr;
     size_t n = 0;
+    std::shared_ptr<DevBlock> block;  // where p lies (null: an allocation of its own)
     DevArr() = default;
     DevArr(const DevArr &) = delete;
     DevArr &operator=(const DevArr &) = delete;
-    DevArr(DevArr &&o) noexcept : p(o.p), n(o.n) { o.p = nullptr; o.n = 0; }
+    DevArr(DevArr &&o) noexcept : p(o.p), n(o.n), block(std::move(o.block)) { o.p = nullptr; o.n = 0; }
     DevArr &operator=(DevArr &&o) noexcept {
-        if (this != &o) { release(); p = o.p; n = o.n; o.p = nullptr; o.n = 0; }
+        if (this != &o) { release(); p = o.p; n = o.n; block = std::move(o.block); o.p = nullptr; o.n = 0; }
         return *this;
     }
     ~DevArr() { release(); }
     void alloc(size_t count) {
         release();
         if (count == 0) return;
-        p = static_cast<T *>(dev_alloc_zero(count * sizeof(T)));
+        p = static_cast<T *>(DevArena::take(count * sizeof(T), block));
+        if (!p) p = static_cast<T *>(dev_alloc_zero(count * sizeof(T)));
         n = count;
     }
     void release() {
-        if (p) dev_free(p);
+        if (p && !block) dev_free(p);
+        block.reset();
         p = nullptr;
         n = 0;
     }
@@ -114,6 +147,8 @@ struct RefHierarchy {
     DevBuf bt_pt, bt_st, bt_r, bt_rt, bt_p, bt_t, bt_v, bt_e, bt_mod, bt_scal;
 
     void build(hipStream_t s, const DevGeo &top, const Bc &user_bc, int dc, int ordering, int maxdepth_user);
+    // device bytes build() allocates
+    static size_t bytes(int nx, int ny, double dx, double dy, int maxdepth_user);
     void relax(hipStream_t s, int d, double *phi, const double *rhs, int sweeps, double omega);
     // Measurement of the finest-level DC red-black smoother (2 sweeps):
     // kernel 4 the relax with LDS tiles, 5 with one launch per colour, 6 the

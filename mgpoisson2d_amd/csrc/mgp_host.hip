@@ -51,6 +51,30 @@ void *dev_alloc_zero(size_t bytes) {
 }
 void dev_free(void *p) { (void)hipFree(p); }
 
+static thread_local std::shared_ptr<DevBlock> t_block;
+
+DevArena::DevArena(size_t bytes) : outer(t_block) {
+    try {
+        block = std::make_shared<DevBlock>();
+        block->p = static_cast<char *>(dev_alloc_zero(bytes));
+        block->bytes = bytes;
+    } catch (const Failure &) {
+        (void)hipGetLastError();
+        block.reset();
+    }
+    t_block = block;
+}
+DevArena::~DevArena() { t_block = outer; }
+
+void *DevArena::take(size_t bytes, std::shared_ptr<DevBlock> &owner) {
+    const size_t b = (bytes + 255) / 256 * 256;
+    if (!t_block || b > t_block->bytes - t_block->used) return nullptr;
+    void *p = t_block->p + t_block->used;
+    t_block->used += b;
+    owner = t_block;
+    return p;
+}
+
 Grid make_grid(int nx, int ny, double dx, double dy) {
     Grid g;
     g.nx = nx;
@@ -378,6 +402,19 @@ void RefHierarchy::build(hipStream_t s, const DevGeo &top, const Bc &user_bc, in
     const size_t nb = level_elems(b.g.nx, b.g.ny);
     for (DevBuf *w : {&bt_pt, &bt_st, &bt_r, &bt_rt, &bt_p, &bt_t, &bt_v, &bt_e, &bt_mod}) w->alloc(nb);
     bt_scal.alloc(8);
+}
+
+size_t RefHierarchy::bytes(int nx, int ny, double dx, double dy, int maxdepth_user) {
+    std::vector<int> rx, ry;
+    const int depth = reference_schedule(nx, ny, dx, dy, maxdepth_user, rx, ry);
+    size_t b = 4096;
+    for (int d = 0;; ++d) {
+        const size_t n = level_elems(nx, ny) * sizeof(double) + 256;
+        b += 10 * n;
+        if (d == depth) return b + 9 * n;
+        nx /= rx[d];
+        ny /= ry[d];
+    }
 }
 
 static bool removes_average(const Bc &b) {

@@ -138,6 +138,23 @@ void KrylovMG::ensure_fgmres(const Grid &g) {
     hip_check(hipHostMalloc((void **)&K.ghost, (size_t)(4 * m + 6) * sizeof(double)), "hipHostMalloc");
 }
 
+size_t KrylovMG::bytes(int nx, int ny, const mgp_solver_opts &o) {
+    const bool mixed = o.method == MGP_METHOD_KRYLOV_MG32;
+    const size_t n0 = level_elems(nx, ny) * sizeof(double) + 256;
+    size_t b = 65536 + 9 * n0;                                           // Krylov vectors
+    if (o.refine == MGP_REFINE_DD) b += 3 * n0;
+    if (o.order == 4) b += 8 * n0;
+    for (int lev = 0; ny >= MIN_COARSE_NY; ++lev) {
+        const size_t n = level_elems(nx, ny) * sizeof(double) + 256;
+        const size_t small = (size_t)ring_table_elems(make_grid(nx, ny, 1.0, 1.0)) * 12 + (size_t)level_pitch(nx) * 16 + 1024;
+        b += 5 * n + small + (!mixed || lev == 0 ? 3 * n : 0) + (mixed ? 3 * n + 1024 : 0);
+        if (o.maxdepth >= 0 && lev >= o.maxdepth) break;
+        int off = 0;
+        ny = semicoarsen_step(ny, MIN_COARSE_NY, true, true, off);
+    }
+    return b;
+}
+
 void KrylovMG::build(hipStream_t s, const DevGeo &top, const Bc &user_bc, const mgp_solver_opts &o,
                      const mgp_mapping *map) {
     if (top.g.ny < 4 || top.g.nx < 4) {
