@@ -156,7 +156,7 @@ struct RefHierarchy {
     // bytes of one call (7 fields read, 1 written).
     double time_relax(hipStream_t s, int kernel, int reps, double *bytes);
     void bottom(hipStream_t s, int d);
-    void vcycle_noinit(Workspace &W, hipStream_t s, int d, int numcycles, int sd, int su, int sb);
+    void vcycle_noinit(Workspace &W, hipStream_t s, int d, int numcycles, int sd, int su, int sb, bool e_ready = false);
     void fmg_noinit(Workspace &W, hipStream_t s, int d, int numcycles, int sd, int su, int sb);
     int solve(Workspace &W, hipStream_t s, const DevGeo &top, const Bc &user_bc, int homog, double *phi,
               double *rhs, double tol, int maxiters, int numcycles, int sd, int su, int sb, int zerophi,

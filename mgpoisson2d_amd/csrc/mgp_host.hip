@@ -580,10 +580,12 @@ void RefHierarchy::bottom(hipStream_t s, int d) {
     launch_bicgstab2(s, a);
 }
 
-void RefHierarchy::vcycle_noinit(Workspace &W, hipStream_t s, int d, int numcycles, int sd, int su, int sb) {
+// e_ready: the restriction has set this level's initial guess.
+void RefHierarchy::vcycle_noinit(Workspace &W, hipStream_t s, int d, int numcycles, int sd, int su, int sb,
+                                 bool e_ready) {
     HLevel &l = levels[d];
     const double omega = dc ? 4.0 / 5.0 : 1.0;
-    if (dc) launch_einit(s, l.e.p, l.r.p, l.invd.p, l.g);  // MGPoisson2D_DD.f90:931,971
+    if (dc && !e_ready) launch_einit(s, l.e.p, l.r.p, l.invd.p, l.g);  // MGPoisson2D_DD.f90:931,971
     if (d == maxdepth) {
         relax(s, d, l.e.p, l.r.p, sb, omega);
         bottom(s, d);
@@ -591,7 +593,14 @@ void RefHierarchy::vcycle_noinit(Workspace &W, hipStream_t s, int d, int numcycl
     }
     HLevel &c = levels[d + 1];
     relax(s, d, l.e.p, l.r.p, sd, omega);
-    if (dc) {
+    // The DC transfers with the ghosts formed on the way leave e's stored ghosts
+    // as the smoother wrote them; the smoother after the correction fills them
+    // again, as every sweep does.
+    Lah lah;
+    const bool fused = dc && su > 0 && refx[d] == 2 && refy[d] == 2 && lah_sides(l.bc, lah);
+    if (fused) {
+        launch_dc_restrict2x2(s, c.r.p, c.e.p, c.invd.p, l.e.p, l.r.p, l.g, c.g, l.geo, lah);
+    } else if (dc) {
         launch_fill_ghosts(s, l.e.p, l.g, l.geo, l.bc, 1, 1);
         launch_dc_laplacian(s, l.w.p, l.e.p, l.r.p, l.g, l.geo);
         launch_restrict_cc(s, c.r.p, l.w.p, c.g, l.g.pitch, refx[d], refy[d], nullptr, nullptr);
@@ -601,12 +610,17 @@ void RefHierarchy::vcycle_noinit(Workspace &W, hipStream_t s, int d, int numcycl
         // e(d+1) = r(d+1) * invdiags(d+1) fused (MGPoisson2D.f90:805-806)
         launch_restrict_cc(s, c.r.p, l.w.p, c.g, l.g.pitch, refx[d], refy[d], c.e.p, c.invd.p);
     }
-    for (int k = 0; k < numcycles; ++k) vcycle_noinit(W, s, d + 1, numcycles, sd, su, sb);
+    for (int k = 0; k < numcycles; ++k) vcycle_noinit(W, s, d + 1, numcycles, sd, su, sb, fused && k == 0);
     if (refx[d] != 2 || refy[d] != 2) {
         g_last_error = "prolong: only 2x2 coarsening is defined by the reference (MGPoisson2D.f90:385-388)";
         throw Failure(MGP_ERR_UNSUPPORTED);
     }
-    prolong_level(W, s, l, c, 1, nullptr);
+    if (fused) {
+        launch_dc_prolong2x2(s, l.e.p, l.g.pitch, c.e.p, c.g, lah);
+        if (removes_average(c.bc)) remove_average(W, s, l.e.p, l.g, l.J.p);
+    } else {
+        prolong_level(W, s, l, c, 1, nullptr);
+    }
     relax(s, d, l.e.p, l.r.p, su, omega);
 }
 

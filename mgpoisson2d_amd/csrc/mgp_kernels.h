@@ -57,6 +57,17 @@ int dc_rb_tile_once(hipStream_t s, const double *phi, double *out, const double 
                     const Grid &g, const Geo &geo, const Bc &bc, double omega, int S);
 void launch_restrict_cc(hipStream_t s, double *crse, const double *fine, const Grid &cg, int fpitch, int rx,
                         int ry, double *e, const double *invd);
+// The DC cycle's transfers on levels whose sides are all Neumann or Dirichlet
+// in LAH mode (lah_sides): the ghosts are formed in the kernels.
+struct Lah {
+    double sgn[4];  // ghost = sgn * the adjacent cell
+};
+bool lah_sides(const Bc &bc, Lah &lah);
+// rc = 2x2 average of rhs - L_dc e, ec = rc invdc
+void launch_dc_restrict2x2(hipStream_t s, double *rc, double *ec, const double *invdc, const double *e,
+                           const double *rhs, const Grid &fg, const Grid &cg, const Geo &geo, const Lah &lah);
+// fine += linear prolongation of crse
+void launch_dc_prolong2x2(hipStream_t s, double *fine, int fpitch, const double *crse, const Grid &cg, const Lah &lah);
 void launch_restrict_xf(hipStream_t s, double *crse, const double *fine, const Grid &cg, int fpitch, int rx,
                         int ry);
 void launch_restrict_yf(hipStream_t s, double *crse, const double *fine, const Grid &cg, int fpitch, int rx,

@@ -213,7 +213,7 @@ __device__ __forceinline__ void block_fill_ghosts(Fld f, const Grid &g, const Ge
     __syncthreads();
 }
 
-__global__ void __launch_bounds__(256) k_fill_ghosts(Fld f, Grid g, Geo geo, Bc bc, int homog, int do_neum) {
+__global__ void __launch_bounds__(1024) k_fill_ghosts(Fld f, Grid g, Geo geo, Bc bc, int homog, int do_neum) {
     block_fill_ghosts(f, g, geo, bc, homog, do_neum);
 }
 
@@ -531,6 +531,71 @@ __global__ void __launch_bounds__(256) k_restrict_cc(double *crse, const double 
     const size_t c = ix(cg.pitch, ci, cj);
     crse[c] = s;
     if (e) e[c] = s * invd[c];
+}
+
+// Reads of a field whose ghosts follow the LAH fill (the DC cycle's levels: a
+// Neumann side's ghost is the adjacent cell, a Dirichlet side's its negative),
+// formed from the valid cells: what fill_ghosts(homog, do_neum) would have
+// stored before the read.  Neighbours across a side only, no corners.
+struct LahGet {
+    const double *p;
+    int pitch, nx, ny;
+    Lah lah;
+    __device__ __forceinline__ double operator()(int i, int j) const {
+        if (i < 0) return lah.sgn[XLO] * p[ix(pitch, 0, j)];
+        if (i >= nx) return lah.sgn[XHI] * p[ix(pitch, nx - 1, j)];
+        if (j < 0) return lah.sgn[YLO] * p[ix(pitch, i, 0)];
+        if (j >= ny) return lah.sgn[YHI] * p[ix(pitch, i, ny - 1)];
+        return p[ix(pitch, i, j)];
+    }
+};
+
+// The DC cycle's way down in one pass (MGPoisson2D_DD.f90:941-985): the
+// residual rhs - L e of each 2 x 2 block of fine cells, its average into the
+// coarse r and the next level's initial guess e = r invd.  A fill of e's ghosts,
+// the residual, the restriction and the guess as launches of their own are
+// four to six latencies a level and write the residual for one reader.
+__global__ void __launch_bounds__(256) k_dc_restrict2x2(double *rc, double *ec, const double *invdc, const double *e,
+                                                        const double *rhs, Grid fg, Grid cg, Geo geo, Lah lah) {
+    const int ci = blockIdx.x * 64 + (threadIdx.x & 63);
+    const int cj = blockIdx.y * 4 + (threadIdx.x >> 6);
+    if (ci >= cg.nx || cj >= cg.ny) return;
+    const LahGet get{e, fg.pitch, fg.nx, fg.ny, lah};
+    const CFld f{e, fg.pitch};
+    const double idx = 1.0 / fg.dx, idy = 1.0 / fg.dy, scale = 1.0 / 4;
+    double s = 0.0;
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+            const int i = 2 * ci + a, j = 2 * cj + b;
+            const size_t c = ix(fg.pitch, i, j);
+            double ax, ay;
+            dc_five_vals(e[c], get(i + 1, j), get(i - 1, j), get(i, j + 1), get(i, j - 1), geo.Jxx[c + 1], geo.Jxx[c],
+                         geo.Jyy[c + fg.pitch], geo.Jyy[c], idx, idy, ax, ay);
+            const double v = dc_cross(f, fg, geo, i, j) + ax + ay;
+            s = s + scale * (rhs[c] - v);
+        }
+    const size_t c = ix(cg.pitch, ci, cj);
+    rc[c] = s;
+    ec[c] = s * invdc[c];
+}
+
+// Linear 2 x 2 prolongation of a DC level's correction with its LAH ghosts
+// formed on the way (k_prolong2x2 of order 1 after a fill).
+__global__ void __launch_bounds__(256) k_dc_prolong2x2(Fld fine, const double *crse, Grid cg, Lah lah) {
+    const int ci = blockIdx.x * 64 + (threadIdx.x & 63);
+    const int cj = blockIdx.y * 4 + (threadIdx.x >> 6);
+    if (ci >= cg.nx || cj >= cg.ny) return;
+    const LahGet get{crse, cg.pitch, cg.nx, cg.ny, lah};
+    const int fi = 2 * ci, fj = 2 * cj;
+    const double c = crse[ix(cg.pitch, ci, cj)];
+    const double mx = 0.5 * (get(ci + 1, cj) - get(ci - 1, cj));
+    const double my = 0.5 * (get(ci, cj + 1) - get(ci, cj - 1));
+    fine(fi, fj) = fine(fi, fj) + c + 0.25 * (-mx - my);
+    fine(fi + 1, fj) = fine(fi + 1, fj) + c + 0.25 * (mx - my);
+    fine(fi, fj + 1) = fine(fi, fj + 1) + c + 0.25 * (-mx + my);
+    fine(fi + 1, fj + 1) = fine(fi + 1, fj + 1) + c + 0.25 * (mx + my);
 }
 
 // Face-centred metric restriction: injection at coincident faces times the
@@ -1245,7 +1310,7 @@ void launch_fill_ghosts(hipStream_t s, double *phi, const Grid &g, const Geo &ge
                         int do_neum) {
     const Fld f{phi, g.pitch};
     if (!wide_perimeter(g)) {
-        k_fill_ghosts<<<1, 256, 0, s>>>(f, g, geo, bc, homog, do_neum);
+        k_fill_ghosts<<<1, 1024, 0, s>>>(f, g, geo, bc, homog, do_neum);
         return;
     }
     k_fill_x_ghosts<<<(2 * (g.ny + 2) + 255) / 256, 256, 0, s>>>(f, g, geo, bc, homog, do_neum);
@@ -1314,6 +1379,21 @@ void launch_dc_lex(hipStream_t s, double *phi, const double *modrhs, const doubl
 void launch_restrict_cc(hipStream_t s, double *crse, const double *fine, const Grid &cg, int fpitch, int rx,
                         int ry, double *e, const double *invd) {
     k_restrict_cc<<<tiles(cg.nx, cg.ny), 256, 0, s>>>(crse, fine, cg, fpitch, rx, ry, e, invd);
+}
+bool lah_sides(const Bc &bc, Lah &lah) {
+    for (int k = 0; k < 4; ++k) {
+        if (bc.mode[k] != MODE_LAH || (bc.type[k] != BC_NEUM && bc.type[k] != BC_DIRI)) return false;
+        lah.sgn[k] = bc.type[k] == BC_NEUM ? 1.0 : -1.0;
+    }
+    return true;
+}
+void launch_dc_restrict2x2(hipStream_t s, double *rc, double *ec, const double *invdc, const double *e,
+                           const double *rhs, const Grid &fg, const Grid &cg, const Geo &geo, const Lah &lah) {
+    k_dc_restrict2x2<<<tiles(cg.nx, cg.ny), 256, 0, s>>>(rc, ec, invdc, e, rhs, fg, cg, geo, lah);
+}
+void launch_dc_prolong2x2(hipStream_t s, double *fine, int fpitch, const double *crse, const Grid &cg,
+                          const Lah &lah) {
+    k_dc_prolong2x2<<<tiles(cg.nx, cg.ny), 256, 0, s>>>(Fld{fine, fpitch}, crse, cg, lah);
 }
 void launch_restrict_xf(hipStream_t s, double *crse, const double *fine, const Grid &cg, int fpitch, int rx,
                         int ry) {

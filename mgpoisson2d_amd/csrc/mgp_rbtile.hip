@@ -226,7 +226,7 @@ struct RbShape {
     int H, NW;  // window rows, waves
 };
 // candidate shapes, in the numbering of the tuning switch (k >= 1 is entry k-1)
-constexpr RbShape RB_SHAPES[] = {{16, 4}, {32, 4}, {32, 8}, {64, 8}};
+constexpr RbShape RB_SHAPES[] = {{16, 4}, {32, 4}, {32, 8}, {64, 8}, {16, 8}};
 constexpr int RB_NSHAPES = sizeof(RB_SHAPES) / sizeof(RB_SHAPES[0]);
 
 int rb_tiles(const Grid &g, int shape, int S, int &ntx) {
@@ -255,6 +255,7 @@ void launch_s(hipStream_t s, int shape, const double *in, double *out, const dou
         MGP_RB_SHAPE(1)
         MGP_RB_SHAPE(2)
         MGP_RB_SHAPE(3)
+        MGP_RB_SHAPE(4)
         default: break;
     }
 #undef MGP_RB_SHAPE
@@ -275,17 +276,10 @@ std::mutex rb_mu;
 int rb_choice = -1;  // -1: timed pick; 0: one colour per launch; k >= 1: shape k - 1
 std::map<std::tuple<int, int, int, int>, int> rb_picked;
 
-// The shape with the fewest window cells over the level (small levels).
-int rb_fewest_cells(const Grid &g, int S) {
-    int best = 0;
-    long long bestc = -1;
-    for (int k = 0; k < RB_NSHAPES; ++k) {
-        int ntx;
-        const long long c = (long long)rb_tiles(g, k, S, ntx) * RB_WW * RB_SHAPES[k].H;
-        if (bestc < 0 || c < bestc) best = k, bestc = c;
-    }
-    return best;
-}
+// Small levels do not fill the CUs: a launch takes as long as one window, and
+// that grows with the rows each wave holds (a level of 64^2: 21 us with 8 rows
+// a wave, 8 to 10 us with 4).
+constexpr int RB_SMALL = 4;  // {16, 8}: two rows a wave
 
 // The shape for this level, sweeps per load and form: timed once per
 // (nx, ny, S, fuse) on the call's own operands (the timing launches write
@@ -305,7 +299,7 @@ int rb_pick(hipStream_t s, int S, bool fuse, const double *in, double *out, cons
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     hip_check(hipStreamIsCapturing(s, &cs), "hipStreamIsCapturing");
     if ((long long)g.nx * g.ny < 256LL * 256 || cs != hipStreamCaptureStatusNone) {
-        const int k = rb_fewest_cells(g, S);
+        const int k = RB_SMALL;
         if (cs == hipStreamCaptureStatusNone) {
             std::lock_guard<std::mutex> lk(rb_mu);
             rb_picked.emplace(key, k);
