@@ -48,7 +48,10 @@ __device__ __forceinline__ void tile_cells(const BTile &t, const Grid &g, F &&f)
 }
 
 // v[out] = (v[rhs] -) A v[in], A the reference operator with the problem's
-// homogeneous BCs (ghosts synthesised from the valid cells).
+// homogeneous BCs (ghosts synthesised from the valid cells).  Bound by memory
+// (48 bytes a cell).  Four rows a thread: 81 us over the batch of 256 problems
+// and 11.7 over 24 odd ones, 146 and 26 with the rows' cells loaded each by
+// itself and the ring's stencil among them.
 __global__ void __launch_bounds__(256) k_b_apply(const BTile *tiles, const BProb *P, const int *mask, int out, int in,
                                                  int rhs) {
     const BTile t = tiles[blockIdx.x];
@@ -57,15 +60,11 @@ __global__ void __launch_bounds__(256) k_b_apply(const BTile *tiles, const BProb
     const Grid g = p->g;
     const Geo geo = p->geo;
     const Bc bc = p->bc;
-    const double *phi = p->v[in];
     double *o = p->v[out];
     const double *r = rhs >= 0 ? p->v[rhs] : nullptr;
-    tile_cells(t, g, [&](int i, int j) {
+    lap_tile<BT_ROWS / 4>(p->v[in], g, geo, bc, t.tx * 64, t.ty * BT_ROWS, [&](int i, int j, double v) {
         const size_t c = ix(g.pitch, i, j);
-        const bool interior = i > 0 && i < g.nx - 1 && j > 0 && j < g.ny - 1;
-        const double v = interior ? cell_lap_interior(CFld{phi, g.pitch}, g, geo, i, j)
-                                  : cell_lap(synth(phi, g, bc), g, geo, bc, 1, i, j);
-        o[c] = r ? r[c] - v : v;
+        o[c] = r ? gptr(r)[c] - v : v;
     });
 }
 
@@ -80,7 +79,7 @@ __global__ void __launch_bounds__(256) k_b_reduce_partial(const BTile *tiles, co
     const BProb *p = P + t.item;
     const Grid g = p->g;
     const double vol = g.dx * g.dy;
-    const double *A = p->v[a], *B = p->v[b], *C = c2 >= 0 ? p->v[c2] : nullptr;
+    gconst<double> *A = gptr(p->v[a]), *B = gptr(p->v[b]), *C = gptr(c2 >= 0 ? p->v[c2] : nullptr);
     const int nb = p->nb;
     Acc acc{0.0, 0.0}, acc2{0.0, 0.0};
     // The thread's cells, in the order of the sum: rows tx, tx + nb, .. and in
@@ -238,6 +237,12 @@ __global__ void __launch_bounds__(256) k_b_end32(const BTile *tiles, const BProb
     });
 }
 
+// Row blocks of a problem's reductions: about 2048 cells each, 8 per thread,
+// which is one round of k_b_reduce_partial's loads (rows b, b + nb, ..): with
+// 8192 cells, four rounds one after the other, a pass took 29 us over 24 odd
+// problems and 47 over 256, now 11 and 30.
+int reduce_rows(int nx, int ny) { return std::max(1, std::min(ny, (nx * ny + 2047) / 2048)); }
+
 size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 
 void tiles_of(std::vector<BTile> &out, int item, int nx, int ny) {
@@ -281,7 +286,7 @@ size_t BatchKMG::problem_bytes(const Problem &q, const mgp_solver_opts &o) {
     size_t b = 0;
     const size_t n0 = level_elems(q.nx, q.ny);
     b += BV_COUNT * round256(n0 * sizeof(double));
-    const int nb = std::max(1, std::min(q.ny, (q.nx * q.ny + 8191) / 8192));
+    const int nb = reduce_rows(q.nx, q.ny);
     b += round256((size_t)2 * nb * sizeof(double));
     int ny = q.ny, lev = 0;
     size_t levels = 0;
@@ -355,7 +360,7 @@ BatchKMG::BatchKMG(hipStream_t s_, const std::vector<Problem> &probs, const mgp_
         Off &O = off[p];
         const size_t n0 = level_elems(q.nx, q.ny);
         for (int k = 0; k < BV_COUNT; ++k) O.v[k] = take(n0);
-        const int nb = std::max(1, std::min(q.ny, (q.nx * q.ny + 8191) / 8192));
+        const int nb = reduce_rows(q.nx, q.ny);
         O.partial = take((size_t)2 * nb);  // two products' partials per reduction pass
         while (true) {
             const size_t nl = level_elems(q.nx, ny);
@@ -407,7 +412,7 @@ BatchKMG::BatchKMG(hipStream_t s_, const std::vector<Problem> &probs, const mgp_
         for (int k = 0; k < BV_COUNT; ++k) B.v[k] = at(O.v[k]);
         B.sc = scal + (size_t)p * SC_COUNT;
         B.partial = at(O.partial);
-        B.nb = std::max(1, std::min(q.ny, (q.nx * q.ny + 8191) / 8192));
+        B.nb = reduce_rows(q.nx, q.ny);
         B.lev0 = (int)L.size();
         int ny = q.ny;
         double dy = q.dy;

@@ -85,6 +85,16 @@ __host__ __device__ inline size_t ix(int pitch, int i, int j) {
     return (size_t)(j + 1) * (size_t)pitch + (size_t)(OFFX + i);
 }
 
+// Device-memory pointers typed as global: the compiler then knows they
+// cannot alias LDS and may issue loads ahead of LDS stores (with generic
+// pointers every LDS store would wait for the loads before it).
+template <typename T>
+using gconst = const __attribute__((address_space(1))) T;
+template <typename T>
+__device__ __forceinline__ gconst<T> *gptr(const T *p) {
+    return (gconst<T> *)p;
+}
+
 // y-direction prolongation for 1x2 semicoarsening at fine cell (i, j):
 // linear in y between the coarse centre J = j/2 (weight 3/4) and its
 // neighbour on j's side (J-1 for even j, J+1 for odd j; weight 1/4); beyond a

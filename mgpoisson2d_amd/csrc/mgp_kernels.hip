@@ -235,17 +235,18 @@ __global__ void __launch_bounds__(256) k_laplacian(double *out, CFld phi, const 
     out[c] = rhs ? rhs[c] - v : v;
 }
 
-// out = rhs - L[phi] on a homogeneous MG level without a prior ghost fill.
+// out = rhs - L[phi] (L[phi] without rhs) on a homogeneous MG level without a
+// prior ghost fill.  Bound by memory: 48 bytes a cell (phi, the four metrics,
+// out).  Two rows a thread: 49 us on 2048 x 2048 cells (4.1 TB/s), 99 with one
+// cell a thread and the ring's stencil in the interior's waves; one row 62 and
+// 8.7 (512 x 512), four rows 46 and 9.7, two 49 and 9.1.
+constexpr int APPLY_ROWS = 2;
 __global__ void __launch_bounds__(256) k_residual_synth(double *out, const double *phi, const double *rhs, Grid g,
                                                         Geo geo, Bc bc) {
-    const int i = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int j = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (i >= g.nx || j >= g.ny) return;
-    const size_t c = ix(g.pitch, i, j);
-    const bool interior = i > 0 && i < g.nx - 1 && j > 0 && j < g.ny - 1;
-    const double v = interior ? cell_lap_interior(CFld{phi, g.pitch}, g, geo, i, j)
-                              : cell_lap(synth(phi, g, bc), g, geo, bc, 1, i, j);
-    out[c] = rhs ? rhs[c] - v : v;
+    lap_tile<APPLY_ROWS>(phi, g, geo, bc, blockIdx.x * 64, blockIdx.y * 4 * APPLY_ROWS, [&](int i, int j, double v) {
+        const size_t c = ix(g.pitch, i, j);
+        out[c] = rhs ? rhs[c] - v : v;
+    });
 }
 
 __global__ void __launch_bounds__(256) k_invdiags(double *out, Grid g, Geo geo, Bc bc, int homog) {
@@ -1323,7 +1324,8 @@ void launch_laplacian(hipStream_t s, double *out, const double *phi, const doubl
 }
 void launch_residual_synth(hipStream_t s, double *out, const double *phi, const double *rhs, const Grid &g,
                            const Geo &geo, const Bc &bc) {
-    k_residual_synth<<<tiles(g.nx, g.ny), 256, 0, s>>>(out, phi, rhs, g, geo, bc);
+    const dim3 grid = tiles(g.nx, (g.ny + APPLY_ROWS - 1) / APPLY_ROWS);
+    k_residual_synth<<<grid, 256, 0, s>>>(out, phi, rhs, g, geo, bc);
 }
 void launch_invdiags(hipStream_t s, double *out, const Grid &g, const Geo &geo, const Bc &bc, int homog) {
     k_invdiags<<<tiles(g.nx, g.ny), 256, 0, s>>>(out, g, geo, bc, homog);

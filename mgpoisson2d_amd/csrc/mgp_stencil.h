@@ -40,7 +40,7 @@ struct SynthGet {
     const double *p;
     int pitch, nx, ny;
     int t[4], m[4];
-    __device__ __forceinline__ double raw(int i, int j) const { return p[ix(pitch, i, j)]; }
+    __device__ __forceinline__ double raw(int i, int j) const { return gptr(p)[ix(pitch, i, j)]; }
     // Side indices are compile-time constants below (a runtime index into
     // t[] / m[] would place them in scratch memory).
     __device__ __forceinline__ static double dg(int mode, double p0, double p1, double p2) {
@@ -218,6 +218,92 @@ __device__ __forceinline__ double cell_lap_interior(const CFld &f, const Grid &g
     const double idx = 1.0 / g.dx, idy = 1.0 / g.dy;
     return interior_lap_values(geo, c, P, idx, idy, q[0], q[1], q[-1], q[P], q[-P], q[P + 1], q[P - 1], q[-P + 1],
                                q[-P - 1]);
+}
+
+// The interior stencil at the R rows upward from the cell at c, in the element
+// type T (metrics geo, inverse spacings idx, idy): the expression of
+// interior_lap_values, every load issued before the first use.  A row is
+// loaded once for the three stencils that read it, and the flux through the
+// face between two rows is computed once: it is the same expression seen from
+// either side.
+template <int R, typename T, typename G>
+__device__ __forceinline__ void lap_rows(const T *e, const G &geo, int P, size_t c, T idx, T idy, T (&out)[R]) {
+    const T fourth = T(0.25);
+    gconst<T> *q = gptr(e) + c - P;
+    gconst<T> *Jxx = gptr(geo.Jxx) + c, *Jxy = gptr(geo.Jxy) + c, *Jyx = gptr(geo.Jyx) + c, *Jyy = gptr(geo.Jyy) + c;
+    T w[R + 2], p[R + 2], a[R + 2], xxw[R], xxe[R], xyw[R], xye[R], yy[R + 1], yx[R + 1];
+#pragma unroll
+    for (int r = 0; r < R + 2; ++r) {
+        w[r] = q[r * P - 1];
+        p[r] = q[r * P];
+        a[r] = q[r * P + 1];
+    }
+#pragma unroll
+    for (int r = 0; r < R + 1; ++r) {
+        yy[r] = Jyy[r * P];
+        yx[r] = Jyx[r * P];
+        if (r < R) {
+            xxw[r] = Jxx[r * P];
+            xxe[r] = Jxx[r * P + 1];
+            xyw[r] = Jxy[r * P];
+            xye[r] = Jxy[r * P + 1];
+        }
+    }
+    T yfs = yy[0] * (p[1] - p[0]) * idy + yx[0] * fourth * (a[1] - w[1] + a[0] - w[0]) * idx;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const T *pw = w + r, *pp = p + r, *pe = a + r;  // rows south, centre, north
+        const T xfe = xxe[r] * (pe[1] - pp[1]) * idx + xye[r] * fourth * (pe[2] - pe[0] + pp[2] - pp[0]) * idy;
+        const T xfw = xxw[r] * (pp[1] - pw[1]) * idx + xyw[r] * fourth * (pp[2] - pp[0] + pw[2] - pw[0]) * idy;
+        const T yfn = yy[r + 1] * (pp[2] - pp[1]) * idy + yx[r + 1] * fourth * (pe[2] - pw[2] + pe[1] - pw[1]) * idx;
+        out[r] = (xfe - xfw) * idx + (yfn - yfs) * idy;
+        yfs = yfn;
+    }
+}
+
+// Cell `lane` of the side `side` (0: row 0, 1: row ny-1, 2: column 0,
+// 3: column nx-1; the corners belong to the rows) of an nx x ny grid within
+// the tile of 64 x H cells from (i0, j0), H <= 64; false if there is none.
+__device__ __forceinline__ bool tile_ring_cell(int nx, int ny, int i0, int j0, int H, int side, int lane, int &i,
+                                               int &j) {
+    if (side < 2) {
+        i = i0 + lane;
+        j = side == 0 ? 0 : ny - 1;
+        return i < nx && j >= j0 && j < j0 + H && (side == 0 || ny > 1);
+    }
+    i = side == 2 ? 0 : nx - 1;
+    j = j0 + lane;
+    return lane < H && j > 0 && j < ny - 1 && i >= i0 && i < i0 + 64 && (side == 2 || nx > 1);
+}
+
+// put(i, j, (L phi)(i, j)) over the tile of 64 x 4 R cells from (i0, j0) by a
+// workgroup of 256 threads, homogeneous BCs with the ghosts synthesised.  A
+// wave takes R rows of the tile's interior cells at a stretch (lap_rows), then
+// one side of its ring cells, which keeps the long one-sided stencils out of
+// the waves that stream the interior.
+template <int R, typename Put>
+__device__ __forceinline__ void lap_tile(const double *phi, const Grid &g, const Geo &geo, const Bc &bc, int i0, int j0,
+                                         Put &&put) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const double idx = 1.0 / g.dx, idy = 1.0 / g.dy;
+    int i = i0 + lane, j = j0 + wave * R;
+    if (i > 0 && i < g.nx - 1) {
+        if (j > 0 && j + R - 1 < g.ny - 1) {
+            double v[R];
+            lap_rows<R>(phi, geo, g.pitch, ix(g.pitch, i, j), idx, idy, v);
+#pragma unroll
+            for (int r = 0; r < R; ++r) put(i, j + r, v[r]);
+        } else {
+            for (int r = 0; r < R; ++r) {
+                if (j + r <= 0 || j + r >= g.ny - 1) continue;
+                double v[1];
+                lap_rows<1>(phi, geo, g.pitch, ix(g.pitch, i, j + r), idx, idy, v);
+                put(i, j + r, v[0]);
+            }
+        }
+    }
+    if (tile_ring_cell(g.nx, g.ny, i0, j0, 4 * R, wave, lane, i, j))
+        put(i, j, cell_lap(synth(phi, g, bc), g, geo, bc, 1, i, j));
 }
 
 // GS/SOR point update (poisson2d.f90:1770-1771, MGPoisson2D_DD.f90:303-304).

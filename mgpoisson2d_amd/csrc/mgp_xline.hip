@@ -88,16 +88,6 @@ struct ImpulseFilled {
     }
 };
 
-// Device-memory pointers typed as global: the compiler then knows they
-// cannot alias LDS and may issue loads ahead of LDS stores (with generic
-// pointers every LDS store would wait for the loads before it).
-template <typename T>
-using gconst = const __attribute__((address_space(1))) T;
-template <typename T>
-__device__ __forceinline__ gconst<T> *gptr(const T *p) {
-    return (gconst<T> *)p;
-}
-
 __host__ __device__ inline int ring_count(int nx, int ny) { return 2 * nx + 2 * (ny - 2); }
 
 // Every ring-cell stencil lies in a 3x3 window of valid cells: the window
@@ -707,53 +697,92 @@ __global__ void __launch_bounds__(XL_THREADS) k_xline_long(T *__restrict__ e, co
     xline_rows<C, XL_THREADS, SEG>(e, f, K, g, geo, row0, rowstep, nrows, nt, far, seglen, seg0, segstep, nsegl);
 }
 
-// (L e)(i, j) at an interior cell from the face metrics: the stencil of
-// cell_lap_interior in the element type T (inverse spacings idx, idy).
-template <typename T, typename G>
-__device__ __forceinline__ T interior_lap(gconst<T> *e, const G &geo_, int P, size_t c, T idx, T idy) {
-    gconst<T> *Jxx = gptr(geo_.Jxx), *Jxy = gptr(geo_.Jxy), *Jyx = gptr(geo_.Jyx), *Jyy = gptr(geo_.Jyy);
-    const T fourth = T(0.25);
-    gconst<T> *q = e + c;
-    const T p = q[0], pe = q[1], pw = q[-1], pn = q[P], ps = q[-P];
-    const T ene = q[P + 1], enw = q[P - 1], ese = q[-P + 1], esw = q[-P - 1];
-    const T xfe = Jxx[c + 1] * (pe - p) * idx + Jxy[c + 1] * fourth * (ene - ese + pn - ps) * idy;
-    const T xfw = Jxx[c] * (p - pw) * idx + Jxy[c] * fourth * (pn - ps + enw - esw) * idy;
-    const T yfn = Jyy[c + P] * (pn - p) * idy + Jyx[c + P] * fourth * (ene - enw + pe - pw) * idx;
-    const T yfs = Jyy[c] * (p - ps) * idy + Jyx[c] * fourth * (pe - pw + ese - esw) * idx;
-    return (xfe - xfw) * idx + (yfn - yfs) * idy;
-}
-
 // Preconditioner residual restricted 1x2 in y, with the coarse correction
 // cleared:  rc(i, J) = (r(i, 2J) + r(i, 2J+1)) / 2,  r = f - L e  (interior
 // stencil from the metrics, ring cells from the table),  ec(i, J) = 0, with
-// its far rows farc (XlFar: lo, then hi one pitch on).
-template <typename T, typename G>
-__device__ __forceinline__ void restrict_cell(T *rc, T *ec, T *farc, const T *e, const T *f, const T *K,
-                                              const Grid &gf, const Grid &gc, const G &geo, int i, int J, int off) {
-    const int nring = ring_count(gf.nx, gf.ny);
+// its far rows farc (XlFar: lo, then hi one pitch on).  Over the tile of
+// 64 x 4 R N coarse cells from (i0, J0) by a workgroup of 256 threads: a wave
+// takes N times R coarse rows of the interior columns, 2 R fine rows at a
+// stretch (lap_rows), then the coarse cells of one side of the ring.  Bound by
+// memory on the fine levels.  One level a launch, R = 1: 11.9 us over the nine
+// levels of 2048 x 2048 cells (16.1 with the ring's cells among the others; R =
+// 2 the same, and 5.6 against 4.8 on the levels of 512 x 512).  Batched, R = 2
+// and N = 2: 7.4 us (13.3) over 24 odd FP64 problems, 19.1 (25.5) over 256 FP32
+// ones; R = 1 takes 7.8 and 19.9, R = 4 7.3 and 18.8 with 190 registers.
+template <int R, int N, typename T, typename G>
+__device__ __forceinline__ void restrict_tile(T *rc, T *ec, T *farc, const T *e, const T *f, const T *K,
+                                              const Grid &gf, const Grid &gc, const G &geo, int off, int i0, int J0) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, P = gf.pitch;
     const T idx = (T)(1.0 / gf.dx), idy = (T)(1.0 / gf.dy);
+    const auto put = [&](int i, int J, T s) {
+        const size_t c = ix(gc.pitch, i, J);
+        rc[c] = s;
+        ec[c] = 0;
+        if (J < 2) farc[J * gc.pitch + OFFX + i] = 0;
+    };
+    int i = i0 + lane;
+    if (i > 0 && i < gf.nx - 1) {
+#pragma unroll
+        for (int n = 0; n < N; ++n) {
+            const int J = J0 + (wave * N + n) * R, j = off + 2 * J;
+            if (J + R <= gc.ny && j > 0 && j + 2 * R - 1 < gf.ny - 1) {
+                const size_t c = ix(P, i, j);
+                T v[2 * R], rhs[2 * R];
+#pragma unroll
+                for (int r = 0; r < 2 * R; ++r) rhs[r] = gptr(f)[c + r * P];
+                lap_rows<2 * R>(e, geo, P, c, idx, idy, v);
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    T s = 0;
+                    s = s + T(0.5) * (rhs[2 * r] - v[2 * r]);
+                    put(i, J + r, s + T(0.5) * (rhs[2 * r + 1] - v[2 * r + 1]));
+                }
+            } else if (R > 1) {
+                for (int r = 0; r < R; ++r) {
+                    const int jr = j + 2 * r;
+                    if (J + r >= gc.ny || jr <= 0 || jr + 1 >= gf.ny - 1) continue;
+                    const size_t c = ix(P, i, jr);
+                    T v[2], s = 0;
+                    lap_rows<2>(e, geo, P, c, idx, idy, v);
+                    s = s + T(0.5) * (gptr(f)[c] - v[0]);
+                    put(i, J + r, s + T(0.5) * (gptr(f)[c + P] - v[1]));
+                }
+            }
+        }
+    }
+    // Coarse cells with a fine cell on the ring: rows 0 and gc.ny - 1 where
+    // they cover the fine grid's first and last row, and the end columns.
+    const bool lo = off == 0, hi = off + 2 * gc.ny == gf.ny;
+    int J;
+    if (wave < 2) {
+        J = wave == 0 ? 0 : gc.ny - 1;
+        i = i0 + lane;
+        if (i >= gc.nx || J < J0 || J >= J0 + 4 * R * N || !(wave == 0 ? lo : hi)) return;
+        if (wave == 1 && lo && J == 0) return;
+    } else {
+        J = J0 + lane;
+        i = wave == 2 ? 0 : gc.nx - 1;
+        if (lane >= 4 * R * N || J >= gc.ny || i < i0 || i >= i0 + 64) return;
+        if ((lo && J == 0) || (hi && J == gc.ny - 1)) return;
+    }
+    const int nring = ring_count(gf.nx, gf.ny);
     T s = 0;
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
         const int j = off + 2 * J + b;
-        const bool ring = i == 0 || i == gf.nx - 1 || j == 0 || j == gf.ny - 1;
-        const T lap = ring ? ring_lap(gptr(e), gptr(K), nring, gf, i, j)
-                           : interior_lap(gptr(e), geo, gf.pitch, ix(gf.pitch, i, j), idx, idy);
-        s = s + T(0.5) * (f[ix(gf.pitch, i, j)] - lap);
+        const size_t c = ix(P, i, j);
+        T v[1];
+        if (i == 0 || i == gf.nx - 1 || j == 0 || j == gf.ny - 1) v[0] = ring_lap(gptr(e), gptr(K), nring, gf, i, j);
+        else lap_rows<1>(e, geo, P, c, idx, idy, v);
+        s = s + T(0.5) * (f[c] - v[0]);
     }
-    const size_t c = ix(gc.pitch, i, J);
-    rc[c] = s;
-    ec[c] = 0;
-    if (J < 2) farc[J * gc.pitch + OFFX + i] = 0;
+    put(i, J, s);
 }
 
 template <typename T, typename G>
 __global__ void __launch_bounds__(256) k_residual_restrict_y(T *rc, T *ec, T *farc, const T *e, const T *f,
                                                              const T *K, Grid gf, Grid gc, G geo, int off) {
-    const int i = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int J = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (i >= gc.nx || J >= gc.ny) return;
-    restrict_cell(rc, ec, farc, e, f, K, gf, gc, geo, i, J, off);
+    restrict_tile<1, 1>(rc, ec, farc, e, f, K, gf, gc, geo, off, blockIdx.x * 64, blockIdx.y * 4);
 }
 
 // ---------------------------------------------------------------------------
@@ -879,20 +908,13 @@ __global__ void __launch_bounds__(256) k_restrict_batch(const BTile *tiles, cons
     const BTile t = tiles[blockIdx.x];
     const BLev *F = levs + t.item, *Cl = levs + t.item + 1;
     if (!active[F->prob]) return;
-    const int i = t.tx * 64 + (threadIdx.x & 63);
-    const Grid gc = Cl->g;
-    if (i >= gc.nx) return;
     T *fe, *ce, *cf, *far, *cfar;
     const T *ff, *K, *cff, *cK;
     typename std::conditional<sizeof(T) == 8, Geo, GeoF>::type geo, cgeo;
     level_fields(F, sel, fe, ff, K, far, geo);
     level_fields(Cl, 0, ce, cff, cK, cfar, cgeo);
     cf = const_cast<T *>(cff);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int J = t.ty * BT_ROWS + (threadIdx.x >> 6) + 4 * r;
-        if (J < gc.ny) restrict_cell(cf, ce, cfar, (const T *)fe, ff, K, F->g, gc, geo, i, J, F->off);
-    }
+    restrict_tile<2, BT_ROWS / 8>(cf, ce, cfar, (const T *)fe, ff, K, F->g, Cl->g, geo, F->off, t.tx * 64, t.ty * BT_ROWS);
 }
 
 template <typename T>

@@ -73,3 +73,29 @@ def test_fp32_rows_of_each_width(nx):
     assert oc == mg.CONVERGED and iters <= 12, (iters, hist[-3:])
     r, _ = rc.oracle().residual(geo, bc, 1, rhs, s.get_phi())
     assert np.linalg.norm(r) <= 1.5e-9 * np.linalg.norm(rhs)
+
+
+@pytest.mark.parametrize("nx,ny", [(4, 16), (63, 8), (64, 9), (65, 15), (66, 17), (128, 32), (129, 33), (130, 66)])
+@pytest.mark.parametrize("types", [(1, 1, 0, 0), (1, 1, 1, 1), (0, 0, 1, 1)])
+@pytest.mark.parametrize("method", [mg.METHOD_KRYLOV_MG, mg.METHOD_KRYLOV_MG32])
+def test_operator_and_restriction_tiles(nx, ny, types, method):
+    """The operator and the residual's restriction split a tile into interior
+    cells and one side of the ring per wave: sizes one off the tile's 64
+    columns and its 8, 16 and 32 rows.  The solvers' recurrences apply the
+    operator tile by tile and the residual they end on is checked cell by
+    cell, so the solution is the direct one only if no cell is left out or
+    counted twice."""
+    import scipy.sparse.linalg as spl
+    from cases import probed_matrix
+    geo, bc, _, rhs = setup(nx, ny, 0.08, 3.0, types, seed=ny)
+    exact = spl.spsolve(probed_matrix(geo, bc).tocsc(), rhs.ravel()).reshape(geo.ny, geo.nx)
+    s = mg.Solver(geo, bc, method=method)
+    s.set_rhs(rhs)
+    _, _, oc = s.solve(1e-12, 100)
+    assert oc == mg.CONVERGED
+    np.testing.assert_allclose(s.get_phi()[1:-1, 1:-1], exact, rtol=0, atol=1e-10 * np.max(np.abs(exact)))
+    b = mg.Batch([geo], [bc], method=method)
+    b.set_rhs(0, rhs)
+    _, oc = b.solve(1e-12, 100)
+    assert oc[0] == mg.CONVERGED
+    np.testing.assert_allclose(b.get_phi(0), exact, rtol=0, atol=1e-10 * np.max(np.abs(exact)))
