@@ -671,7 +671,8 @@ k_xline(T *__restrict__ e, const T *__restrict__ f, const T *__restrict__ K, Gri
     xline_rows<C, XL_THREADS, SEG>(e, f, K, g, geo, row0, rowstep, nrows, nt, far, seglen, seg0, segstep, nsegl);
 }
 
-// Rows of at most 512 cells: one 64-thread wave per row (as in the batch).
+// Rows one 64-thread wave takes: at most 512 cells, or 128 in launches of few
+// rows (XL_SHORT_FEW_MAX_NX).
 template <int C, bool SEG, typename T, typename GM>
 __global__ void __launch_bounds__(XL_SHORT) __attribute__((amdgpu_waves_per_eu(2)))
 k_xline_short(T *__restrict__ e, const T *__restrict__ f, const T *__restrict__ K, Grid g, GM geo, int row0,
@@ -679,7 +680,7 @@ k_xline_short(T *__restrict__ e, const T *__restrict__ f, const T *__restrict__ 
     xline_rows<C, XL_SHORT, SEG>(e, f, K, g, geo, row0, rowstep, nrows, nt, far, seglen, seg0, segstep, nsegl);
 }
 
-// FP32 rows past 4111 cells (C = 16, 512 threads): one workgroup per CU.
+// FP32 rows past 4111 cells, and rows of 1025 .. 2048 in launches of few rows.
 template <int C, int NT, typename T, typename GM>
 __global__ void __launch_bounds__(NT) k_xline_wide(T *__restrict__ e, const T *__restrict__ f,
                                                         const T *__restrict__ K, Grid g, GM geo, int row0,
