@@ -139,7 +139,7 @@ __global__ void __launch_bounds__(256) k_b_reduce_final(const BProb *P, const in
     }
 }
 
-// BiCGStab scalars of every masked problem (the ops of k_bicg_scalars).
+// BiCGStab scalars of every masked problem (bicg_scalars of the single solver).
 __global__ void k_b_scalars(const BProb *P, const int *mask, int n, int op) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n || !mask[k]) return;
@@ -159,7 +159,7 @@ __global__ void k_b_scalars(const BProb *P, const int *mask, int n, int op) {
     }
 }
 
-// Vector updates (the ops of k_bicg_update):
+// Vector updates:
 //  0: p = r + beta (p - omega v)   1: s = r - alpha v   2: phi += alpha phat
 //  3: phi += omega shat            4: r = s - omega t
 // With L (FP32 cycles), ops 0 and 1 also start the cycle that preconditions

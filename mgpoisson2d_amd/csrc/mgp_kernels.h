@@ -98,9 +98,37 @@ void launch_sub_mean(hipStream_t s, double *fine, const double *sums, const Grid
 // BiCGStab device scalars
 enum { SC_RHO = 0, SC_RHO_NEW = 1, SC_ALPHA = 2, SC_OMEGA = 3, SC_BETA = 4, SC_RV = 5, SC_TS = 6, SC_TT = 7,
        SC_RN = 8, SC_COUNT = 16 };
-void launch_bicg_scalars(hipStream_t s, double *sc, int op);
-void launch_bicg_update(hipStream_t s, double *out, const double *x, const double *y, const double *sc,
-                        const Grid &g, int op);
+// The sums of one solver's iterations: partial needs 2 reduce_blocks(g)
+// doubles, count is 0 between launches.  A launch that sums also computes the
+// scalars that follow from the sums.
+struct BicgSums {
+    double *partial;
+    unsigned *count;
+    double *sc;
+};
+// A run's start: sc[SC_RHO_NEW] = rhat . r, beta and rho of its first iteration.
+void launch_bicg_restart(hipStream_t s, const BicgSums &q, const double *rhat, const double *r, double vol,
+                         const Grid &g);
+void launch_bicg_alpha(hipStream_t s, const BicgSums &q, const double *rhat, const double *v, double vol,
+                       const Grid &g);
+void launch_bicg_omega(hipStream_t s, const BicgSums &q, const double *t, const double *sv, double vol,
+                       const Grid &g);
+struct BicgTail {
+    double *phi, *r;
+    const double *phat, *shat, *s, *t, *rhat;
+    double *partial;
+    unsigned *count;
+    double *sc;
+    double vol;
+    Grid g;
+};
+void launch_bicg_tail(hipStream_t s, const BicgTail &a);
+// p: out = r + beta (out - omega v), else out = r - alpha v; e (may be null),
+// f: the cycle's finest level, started by the same launch.
+void launch_bicg_update(hipStream_t s, bool p, double *out, const double *r, const double *v, const double *sc,
+                        const Grid &g, double *e, double *far);
+void launch_bicg_update(hipStream_t s, bool p, double *out, const double *r, const double *v, const double *sc,
+                        const Grid &g, float *f, float *e, float *far);
 
 struct BottomArgs {
     Grid g;

@@ -1261,42 +1261,151 @@ __global__ void __launch_bounds__(256) k_axpbypcz(double *out, double a, const d
 // round trip and can be replayed as a graph).  Layout of sc[]: see SC_* in
 // mgp_kernels.h.  Reductions deliver sum(vol * a * b).
 // ---------------------------------------------------------------------------
-__global__ void k_bicg_scalars(double *sc, int op) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    if (op == 0) {          // beta = (rho_new/rho)(alpha/omega); rho = rho_new
+// The scalars a reduction's result leads to, by one thread.
+enum { BI_BETA, BI_ALPHA, BI_OMEGA, BI_RESTART };
+__device__ __forceinline__ void bicg_scalars(double *sc, int op) {
+    if (op == BI_BETA) {          // beta = (rho_new/rho)(alpha/omega); rho = rho_new
         sc[SC_BETA] = (sc[SC_RHO_NEW] / sc[SC_RHO]) * (sc[SC_ALPHA] / sc[SC_OMEGA]);
         sc[SC_RHO] = sc[SC_RHO_NEW];
-    } else if (op == 1) {   // alpha = rho / (rhat . v)
+    } else if (op == BI_ALPHA) {  // alpha = rho / (rhat . v)
         sc[SC_ALPHA] = sc[SC_RHO] / sc[SC_RV];
-    } else if (op == 2) {   // omega = (t . s) / (t . t)
+    } else if (op == BI_OMEGA) {  // omega = (t . s) / (t . t)
         sc[SC_OMEGA] = sc[SC_TT] > 0.0 ? sc[SC_TS] / sc[SC_TT] : 0.0;
-    } else {                // restart
+    } else {                      // a run's first iteration: rho_old = alpha = omega = 1
         sc[SC_RHO] = 1.0;
         sc[SC_ALPHA] = 1.0;
         sc[SC_OMEGA] = 1.0;
-        sc[SC_BETA] = 0.0;
+        bicg_scalars(sc, BI_BETA);
     }
 }
 
-// Vector updates with device scalars (valid cells):
-//  0: p = r + beta (p - omega v)     (out=p, x=r, y=v)
-//  1: s = r - alpha v                (out=s, x=r, y=v)
-//  2: phi = phi + alpha phat         (out=phi, x=phat)
-//  3: phi = phi + omega shat         (out=phi, x=shat)
-//  4: r = s - omega t                (out=r, x=s, y=t)
-__global__ void __launch_bounds__(256) k_bicg_update(double *out, const double *x, const double *y,
-                                                     const double *sc, Grid g, int op) {
+// The end of a reduction pass within its launch: block b has put its partial
+// sums into partial[b] and (N = 2) partial[n + b]; the last block to arrive
+// adds them up in block order (so the sum does not depend on which block that
+// is) into sc[slot0] and sc[slot1] and computes the scalars that follow.
+// count is 0 before and after.  No block waits for another.  The partial sums
+// pass from block to block by agent-scope atomics, each performed before the
+// count goes up: a release and acquire instead write back and drop the L2 in
+// every block, 12 to 20 us a pass with 512 to 1024 blocks.
+template <int N>
+__device__ __forceinline__ void bicg_finish(double *ss, double *cc, double *partial, unsigned *count, double *sc,
+                                            const double (&sum)[N], int slot0, int slot1, int op) {
+    __shared__ int last;
+    const unsigned n = gridDim.x;
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int h = 0; h < N; ++h) {
+            double old = __hip_atomic_exchange(partial + h * n + blockIdx.x, sum[h], __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT);
+            asm volatile("" : "+v"(old) : : "memory");  // the exchange has returned: it is performed
+        }
+        last = __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == n - 1;
+    }
+    __syncthreads();
+    if (!last) return;
+#pragma unroll
+    for (int h = 0; h < N; ++h) {
+        Acc acc{0.0, 0.0};
+        for (unsigned k = threadIdx.x; k < n; k += blockDim.x)
+            acc.add(__hip_atomic_load(partial + h * n + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        const double v = block_combine(ss, cc, acc, 0.0, 0);
+        if (threadIdx.x == 0) sc[h ? slot1 : slot0] = v;
+    }
+    if (threadIdx.x == 0) {
+        bicg_scalars(sc, op);
+        __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+// sc[slot] = sum(vol a b), with TWO also sc[slot2] = sum(vol a a), then the
+// scalars of op.  Rows and cells in k_reduce_partial's order.
+template <bool TWO>
+__global__ void __launch_bounds__(256) k_bicg_dot(double *partial, unsigned *count, double *sc, const double *a,
+                                                  const double *b, double vol, Grid g, int slot, int slot2, int op) {
+    __shared__ double ss[256], cc[256];
+    Acc acc[2] = {{0.0, 0.0}, {0.0, 0.0}};
+    for (int j = blockIdx.x; j < g.ny; j += gridDim.x) {
+        const size_t row = ix(g.pitch, 0, j);
+#pragma unroll 4
+        for (int i = threadIdx.x; i < g.nx; i += blockDim.x) {
+            const double x = a[row + i];
+            acc[0].add(vol * (x * b[row + i]));
+            if (TWO) acc[1].add(vol * (x * x));
+        }
+    }
+    double sum[TWO ? 2 : 1];
+    sum[0] = block_combine(ss, cc, acc[0], 0.0, 0);
+    if (TWO) sum[TWO] = block_combine(ss, cc, acc[1], 0.0, 0);
+    bicg_finish(ss, cc, partial, count, sc, sum, slot, slot2, op);
+}
+
+// A small solve's time is its launches (64 x 64 cells: 120 an iteration), a
+// large one's outer vectors are bound by memory: sums, scalars and updates that
+// took 22 launches an iteration take 7, and phi and r pass once.  Against one
+// launch each: 64 x 64 cells 6.95 to 6.61 ms, 1024 x 768 with FP32 cycles 12.4
+// to 12.0, 2048 x 2048 97.9 to 95.7.
+//
+// The end of an iteration in one pass: phi = (phi + alpha phat) + omega shat,
+// r = s - omega t, sc[SC_RN] = sum(vol r r), sc[SC_RHO_NEW] = sum(vol rhat r)
+// and the next iteration's beta and rho.
+__global__ void __launch_bounds__(256) k_bicg_tail(BicgTail A) {
+    __shared__ double ss[256], cc[256];
+    const Grid g = A.g;
+    const double alpha = A.sc[SC_ALPHA], omega = A.sc[SC_OMEGA], vol = A.vol;
+    Acc rr{0.0, 0.0}, rho{0.0, 0.0};
+    for (int j = blockIdx.x; j < g.ny; j += gridDim.x) {
+        const size_t row = ix(g.pitch, 0, j);
+        for (int i0 = threadIdx.x; i0 < g.nx; i0 += 2 * blockDim.x) {
+            // two cells' loads together
+            double x[2], ph[2], sh[2], sv[2], tv[2], rh[2];
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const int i = i0 + q * 256;
+                if (i >= g.nx) continue;
+                const size_t c = row + i;
+                x[q] = A.phi[c];
+                ph[q] = A.phat[c];
+                sh[q] = A.shat[c];
+                sv[q] = A.s[c];
+                tv[q] = A.t[c];
+                rh[q] = A.rhat[c];
+            }
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const int i = i0 + q * 256;
+                if (i >= g.nx) continue;
+                const size_t c = row + i;
+                const double r = sv[q] - omega * tv[q];
+                const double p1 = x[q] + alpha * ph[q];
+                A.phi[c] = p1 + omega * sh[q];
+                A.r[c] = r;
+                rr.add(vol * (r * r));
+                rho.add(vol * (rh[q] * r));
+            }
+        }
+    }
+    double sum[2];
+    sum[0] = block_combine(ss, cc, rr, 0.0, 0);
+    sum[1] = block_combine(ss, cc, rho, 0.0, 0);
+    bicg_finish(ss, cc, A.partial, A.count, A.sc, sum, SC_RN, SC_RHO_NEW, BI_BETA);
+}
+
+// P: out = p = r + beta (p - omega v); else out = s = r - alpha v.  With e it
+// also starts the cycle that preconditions the vector: e = 0 with its far
+// rows, and (FP32) f = the vector.
+template <bool P, typename T>
+__global__ void __launch_bounds__(256) k_bicg_update(double *out, const double *r, const double *v, const double *sc,
+                                                     Grid g, T *f, T *e, T *far) {
     const int i = blockIdx.x * 64 + (threadIdx.x & 63);
     const int j = blockIdx.y * 4 + (threadIdx.x >> 6);
     if (i >= g.nx || j >= g.ny) return;
     const size_t c = ix(g.pitch, i, j);
-    switch (op) {
-    case 0: out[c] = x[c] + sc[SC_BETA] * (out[c] - sc[SC_OMEGA] * y[c]); break;
-    case 1: out[c] = x[c] - sc[SC_ALPHA] * y[c]; break;
-    case 2: out[c] = out[c] + sc[SC_ALPHA] * x[c]; break;
-    case 3: out[c] = out[c] + sc[SC_OMEGA] * x[c]; break;
-    default: out[c] = x[c] - sc[SC_OMEGA] * y[c]; break;
-    }
+    const double x = P ? r[c] + sc[SC_BETA] * (out[c] - sc[SC_OMEGA] * v[c]) : r[c] - sc[SC_ALPHA] * v[c];
+    out[c] = x;
+    if (!e) return;
+    if (f) f[c] = (T)x;
+    e[c] = T(0);
+    if (j < 2) far[j * g.pitch + OFFX + i] = T(0);
 }
 
 }  // namespace mgp
@@ -1455,10 +1564,34 @@ void launch_reduce(hipStream_t s, double *out, double *partial, const double *a,
     k_reduce_partial<<<nb, 256, 0, s>>>(partial, a, b, J, vol, g, kind, p);
     k_reduce_final<<<1, 256, 0, s>>>(out, partial, nb, kind);
 }
-void launch_bicg_scalars(hipStream_t s, double *sc, int op) { k_bicg_scalars<<<1, 64, 0, s>>>(sc, op); }
-void launch_bicg_update(hipStream_t s, double *out, const double *x, const double *y, const double *sc,
-                        const Grid &g, int op) {
-    k_bicg_update<<<tiles(g.nx, g.ny), 256, 0, s>>>(out, x, y, sc, g, op);
+static int bicg_blocks(const Grid &g) { return reduce_blocks(g) < g.ny ? reduce_blocks(g) : g.ny; }
+void launch_bicg_restart(hipStream_t s, const BicgSums &q, const double *rhat, const double *r, double vol,
+                         const Grid &g) {
+    k_bicg_dot<false><<<bicg_blocks(g), 256, 0, s>>>(q.partial, q.count, q.sc, rhat, r, vol, g, SC_RHO_NEW, 0,
+                                                     BI_RESTART);
+}
+void launch_bicg_alpha(hipStream_t s, const BicgSums &q, const double *rhat, const double *v, double vol,
+                       const Grid &g) {
+    k_bicg_dot<false><<<bicg_blocks(g), 256, 0, s>>>(q.partial, q.count, q.sc, rhat, v, vol, g, SC_RV, 0, BI_ALPHA);
+}
+void launch_bicg_omega(hipStream_t s, const BicgSums &q, const double *t, const double *sv, double vol,
+                       const Grid &g) {
+    k_bicg_dot<true><<<bicg_blocks(g), 256, 0, s>>>(q.partial, q.count, q.sc, t, sv, vol, g, SC_TS, SC_TT, BI_OMEGA);
+}
+void launch_bicg_tail(hipStream_t s, const BicgTail &a) { k_bicg_tail<<<bicg_blocks(a.g), 256, 0, s>>>(a); }
+template <typename T>
+static void bicg_update(hipStream_t s, bool p, double *out, const double *r, const double *v, const double *sc,
+                        const Grid &g, T *f, T *e, T *far) {
+    if (p) k_bicg_update<true><<<tiles(g.nx, g.ny), 256, 0, s>>>(out, r, v, sc, g, f, e, far);
+    else k_bicg_update<false><<<tiles(g.nx, g.ny), 256, 0, s>>>(out, r, v, sc, g, f, e, far);
+}
+void launch_bicg_update(hipStream_t s, bool p, double *out, const double *r, const double *v, const double *sc,
+                        const Grid &g, double *e, double *far) {
+    bicg_update<double>(s, p, out, r, v, sc, g, nullptr, e, far);
+}
+void launch_bicg_update(hipStream_t s, bool p, double *out, const double *r, const double *v, const double *sc,
+                        const Grid &g, float *f, float *e, float *far) {
+    bicg_update<float>(s, p, out, r, v, sc, g, f, e, far);
 }
 void launch_seq_mean(hipStream_t s, double *out, const double *fine, const double *J, const Grid &g, double dxprod) {
     k_seq_mean<<<1, 256, 0, s>>>(out, fine, J, g, dxprod);

@@ -305,7 +305,7 @@ void KrylovMG::build(hipStream_t s, const DevGeo &top, const Bc &user_bc, const 
     if (impl->fgmres) ensure_fgmres(top.g);
     impl->sums.alloc(2);
     impl->scal.alloc(SC_COUNT);
-    impl->partial.alloc((size_t)reduce_blocks(top.g) + 8);
+    impl->partial.alloc(2 * (size_t)reduce_blocks(top.g) + 8);  // two products' partials, the blocks' count
     hip_check(hipHostMalloc((void **)&impl->host, SC_COUNT * sizeof(double)), "hipHostMalloc");
     impl->use_graph = o.use_graph != 0;
     built = true;
@@ -387,7 +387,8 @@ static void vcycle_t(hipStream_t s, KrylovMG::Impl &K, size_t d, T *e, const T *
 // out; in mixed precision the cycle runs on FP32 copies.  With y-lines the
 // input is transposed into the hierarchy's finest level and the result
 // transposed back (the valid cells of e; its ghosts are not read).
-static void precondition(hipStream_t s, KrylovMG::Impl &K, double *e, const double *f) {
+// started: the launch that wrote f has begun the cycle (x-lines only).
+static void precondition(hipStream_t s, KrylovMG::Impl &K, double *e, const double *f, bool started = false) {
     KLevel &l = K.L[0];
     const Grid &tg = K.top_g;
     if (K.tr) {
@@ -405,11 +406,11 @@ static void precondition(hipStream_t s, KrylovMG::Impl &K, double *e, const doub
         return;
     }
     if (!K.mixed) {
-        launch_begin(s, e, l.far.p, l.g);
+        if (!started) launch_begin(s, e, l.far.p, l.g);
         for (int c = 0; c < K.ncyc; ++c) vcycle_t(s, K, 0, e, f);
         return;
     }
-    launch_begin32(s, l.r32.p, l.e32.p, l.far32.p, f, l.g);
+    if (!started) launch_begin32(s, l.r32.p, l.e32.p, l.far32.p, f, l.g);
     for (int c = 0; c < K.ncyc; ++c) vcycle_t(s, K, 0, l.e32.p, (const float *)l.r32.p);
     launch_convert(s, e, l.e32.p, l.g, 0);
 }
@@ -582,31 +583,34 @@ int KrylovMG::solve(Workspace &W, hipStream_t s, const DevGeo &top, const Bc &us
     const Grid &g = top.g;
     const double vol = g.dx * g.dy;
     double *sc = K.scal.p;
-    double *partial = K.partial.p;
+    const size_t nb = (size_t)reduce_blocks(g);
+    const BicgSums sums{K.partial.p, reinterpret_cast<unsigned *>(K.partial.p + 2 * nb), sc};
     // the solution the BiCGStab runs update: phi itself, or (double-double)
     // the correction x of the current run, folded into phi + lo at each check
     double *xs = K.dd ? K.x.p : phi;
     auto true_residual = [&]() { return residual_norm(W, s, top, user_bc, homog, phi, rhs, nullptr); };
+    // p or s, and (x-lines) the start of the cycle that preconditions it into dst
+    const bool started = !K.tr;
+    auto update = [&](bool p, double *out, double *dst) {
+        KLevel &l = K.L[0];
+        if (K.mixed && started) launch_bicg_update(s, p, out, K.r.p, K.v.p, sc, g, l.r32.p, l.e32.p, l.far32.p);
+        else launch_bicg_update(s, p, out, K.r.p, K.v.p, sc, g, started ? dst : nullptr, started ? l.far.p : nullptr);
+    };
     // One BiCGStab iteration with every scalar on the device (right
-    // preconditioning, M = one V-cycle).  Ends with ||r||^2 * vol in sc[SC_RN].
+    // preconditioning, M = one V-cycle), from sc[SC_RHO] and sc[SC_BETA] of
+    // the last one's end or of the run's start.  Ends with ||r||^2 * vol in
+    // sc[SC_RN].
     auto body = [&]() {
-        launch_reduce(s, sc + SC_RHO_NEW, partial, K.rhat.p, K.r.p, nullptr, vol, g, 0);
-        launch_bicg_scalars(s, sc, 0);
-        launch_bicg_update(s, K.p.p, K.r.p, K.v.p, sc, g, 0);
-        precondition(s, K, K.phat.p, K.p.p);
+        update(true, K.p.p, K.phat.p);
+        precondition(s, K, K.phat.p, K.p.p, started);
         apply_h(s, K, top, user_bc, K.phat.p, K.v.p);
-        launch_reduce(s, sc + SC_RV, partial, K.rhat.p, K.v.p, nullptr, vol, g, 0);
-        launch_bicg_scalars(s, sc, 1);
-        launch_bicg_update(s, K.s.p, K.r.p, K.v.p, sc, g, 1);
-        launch_bicg_update(s, xs, K.phat.p, nullptr, sc, g, 2);
-        precondition(s, K, K.shat.p, K.s.p);
+        launch_bicg_alpha(s, sums, K.rhat.p, K.v.p, vol, g);
+        update(false, K.s.p, K.shat.p);
+        precondition(s, K, K.shat.p, K.s.p, started);
         apply_h(s, K, top, user_bc, K.shat.p, K.t.p);
-        launch_reduce(s, sc + SC_TS, partial, K.t.p, K.s.p, nullptr, vol, g, 0);
-        launch_reduce(s, sc + SC_TT, partial, K.t.p, K.t.p, nullptr, vol, g, 0);
-        launch_bicg_scalars(s, sc, 2);
-        launch_bicg_update(s, xs, K.shat.p, nullptr, sc, g, 3);
-        launch_bicg_update(s, K.r.p, K.s.p, K.t.p, sc, g, 4);
-        launch_reduce(s, sc + SC_RN, partial, K.r.p, K.r.p, nullptr, vol, g, 0);
+        launch_bicg_omega(s, sums, K.t.p, K.s.p, vol, g);
+        launch_bicg_tail(s, BicgTail{xs, K.r.p, K.phat.p, K.shat.p, K.s.p, K.t.p, K.rhat.p, sums.partial, sums.count,
+                                     sc, vol, g});
     };
     if (K.fgmres) return solve_fgmres(s, top, user_bc, phi, tol, maxiters, zerophi, relres, iters, true_residual);
     if (K.use_graph && !K.graph) {
@@ -659,7 +663,7 @@ int KrylovMG::solve(Workspace &W, hipStream_t s, const DevGeo &top, const Bc &us
                 hip_check(hipMemcpyAsync(K.rhat.p, K.r.p, K.r.n * sizeof(double), hipMemcpyDeviceToDevice, s), "copy");
                 launch_setval(s, K.p.p, 0.0, g, 0);
                 launch_setval(s, K.v.p, 0.0, g, 0);
-                launch_bicg_scalars(s, sc, 3);
+                launch_bicg_restart(s, sums, K.rhat.p, K.r.p, vol, g);
                 restart = false;
             }
             if (K.graph) hip_check(hipGraphLaunch(K.graph, s), "graph launch");

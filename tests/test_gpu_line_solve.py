@@ -99,3 +99,20 @@ def test_operator_and_restriction_tiles(nx, ny, types, method):
     _, oc = b.solve(1e-12, 100)
     assert oc[0] == mg.CONVERGED
     np.testing.assert_allclose(b.get_phi(0), exact, rtol=0, atol=1e-10 * np.max(np.abs(exact)))
+
+
+@pytest.mark.parametrize("nx,ny", [(4, 5), (255, 4), (256, 5), (257, 4), (511, 4), (513, 5)])
+@pytest.mark.parametrize("method", [mg.METHOD_KRYLOV_MG, mg.METHOD_KRYLOV_MG32])
+def test_iteration_passes_at_row_ends(nx, ny, method):
+    """The iteration's last pass takes two cells a thread 256 apart and sums
+    beside its updates; a launch's last workgroup adds the others' sums.  Two
+    solves in a row start from the count the first left."""
+    import scipy.sparse.linalg as spl
+    from cases import probed_matrix
+    geo, bc, _, rhs = setup(nx, ny, 0.08, 3.0, (1, 1, 0, 0), seed=nx)
+    exact = spl.spsolve(probed_matrix(geo, bc).tocsc(), rhs.ravel()).reshape(geo.ny, geo.nx)
+    s = mg.Solver(geo, bc, method=method)
+    for _ in range(2):
+        s.set_rhs(rhs)
+        assert s.solve(1e-12, 100)[2] == mg.CONVERGED
+        np.testing.assert_allclose(s.get_phi()[1:-1, 1:-1], exact, rtol=0, atol=1e-10 * np.max(np.abs(exact)))
