@@ -597,7 +597,13 @@ BatchKMG::XlPhase BatchKMG::stage_phase(TableSet &ts, int d, int set, int colour
     std::vector<XlTask> tasks;
     std::vector<XlBlock> blocks;
     for (const auto &kv : rows.tasks) {
-        const int C = kv.first.first, threads = kv.first.second, per = xline_block_rows(threads);
+        const int C = kv.first.first, threads = kv.first.second;
+        if (!xline_batch_class(C, threads)) {
+            g_last_error = "batch: no line kernel with chunks of " + std::to_string(C) + " cells and " +
+                           std::to_string(threads) + " threads";
+            throw Failure(MGP_ERR_ARG);
+        }
+        const int per = xline_block_rows(threads);
         const int first = (int)tasks.size(), n = (int)kv.second.size();
         ph.cls.push_back(XlClass{C, threads, first, n, rows.lds.at(kv.first)});
         tasks.insert(tasks.end(), kv.second.begin(), kv.second.end());
@@ -640,7 +646,9 @@ void BatchKMG::upload(TableSet &ts) {
 // largest class, which costs the short rows occupancy where there are many.
 // Solves, mixed never / up to 1024 / always: 24 problems of 33..400 cells in
 // FP64 47 / 41 / 41 ms (forked streams 53..114), 38 of 64..990 in FP64 153 / 123
-// / 132, 256 of 32..1024 in FP32 263 / 218 / 245.
+// / 132, 256 of 32..1024 in FP32 263 / 218 / 245.  Eight problems with rows of
+// 2056..4111 cells (one workgroup a CU by its LDS) beside 16 shorter ones, never
+// / up to 1024: 117 / 96 ms in FP64, 89 / 72 with FP32 cycles.
 constexpr int XL_MIXED_MAX_BLOCKS = 1024;
 
 void BatchKMG::launch_phase(const XlPhase &ph, int sel, int k) {

@@ -227,6 +227,8 @@ int xline_batch_chunk(int nx, int threads, size_t elem);
 size_t xline_lds_bytes(int nx, size_t elem);
 // the same for chunk length C and `threads` threads per row
 size_t xline_lds_bytes_for(int nx, int C, size_t elem, int threads);
+// Whether the batched line kernels have rows of chunk length C and `threads` threads.
+bool xline_batch_class(int C, int threads);
 // Rows of `threads` threads that a workgroup of the mixed batched launch holds,
 // and its LDS for rows of chunk length C.
 int xline_block_rows(int threads);

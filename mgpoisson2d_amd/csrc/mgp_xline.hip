@@ -883,6 +883,11 @@ __device__ __forceinline__ void xline_block(const XlBlock &b, const XlTask *task
     xline_task<C, NT, NT == XL_THREADS, T>(tasks[b.first + sub], levs, active, sel, k, tid, lds + sub * row_lds_elems(C, NT));
 }
 
+// The classes of the batched line kernels.
+#define MGP_XL_CLASSES(X)                                                                        \
+    X(2, XL_SHORT) X(4, XL_SHORT) X(8, XL_SHORT) X(2, XL_MID) X(4, XL_MID) X(8, XL_MID)          \
+    X(2, XL_THREADS) X(4, XL_THREADS) X(8, XL_THREADS) X(16, XL_THREADS)
+
 template <typename T>
 __global__ void __launch_bounds__(XL_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
 k_xline_mixed(const XlBlock *blocks, const XlTask *tasks, const BLev *levs, const int *active, int sel, int k) {
@@ -890,16 +895,10 @@ k_xline_mixed(const XlBlock *blocks, const XlTask *tasks, const BLev *levs, cons
     T *lds = reinterpret_cast<T *>(lds_bytes);
     const XlBlock b = blocks[launch_slot()];
     switch (b.cls) {
-        case xl_class(2, XL_SHORT): xline_block<2, XL_SHORT, T>(b, tasks, levs, active, sel, k, lds); break;
-        case xl_class(4, XL_SHORT): xline_block<4, XL_SHORT, T>(b, tasks, levs, active, sel, k, lds); break;
-        case xl_class(8, XL_SHORT): xline_block<8, XL_SHORT, T>(b, tasks, levs, active, sel, k, lds); break;
-        case xl_class(2, XL_MID): xline_block<2, XL_MID, T>(b, tasks, levs, active, sel, k, lds); break;
-        case xl_class(4, XL_MID): xline_block<4, XL_MID, T>(b, tasks, levs, active, sel, k, lds); break;
-        case xl_class(8, XL_MID): xline_block<8, XL_MID, T>(b, tasks, levs, active, sel, k, lds); break;
-        case xl_class(2, XL_THREADS): xline_block<2, XL_THREADS, T>(b, tasks, levs, active, sel, k, lds); break;
-        case xl_class(4, XL_THREADS): xline_block<4, XL_THREADS, T>(b, tasks, levs, active, sel, k, lds); break;
-        case xl_class(8, XL_THREADS): xline_block<8, XL_THREADS, T>(b, tasks, levs, active, sel, k, lds); break;
-        default: xline_block<16, XL_THREADS, T>(b, tasks, levs, active, sel, k, lds); break;
+#define MGP_XL_CASE(C, NT) \
+    case xl_class(C, NT): xline_block<C, NT, T>(b, tasks, levs, active, sel, k, lds); break;
+        MGP_XL_CLASSES(MGP_XL_CASE)
+#undef MGP_XL_CASE
     }
 }
 
@@ -965,6 +964,16 @@ size_t xline_lds_bytes_for(int nx, int C, size_t elem, int threads) {
     // chunk staging (4 arrays), or one chunk array plus the interface rows and unknowns
     const size_t tr = 4 * nt * (C + 1), iface = nt * (C + 1) + (threads > 64 ? 8 * (size_t)threads : 0);
     return (tr > iface ? tr : iface) * elem;
+}
+
+bool xline_batch_class(int C, int threads) {
+    switch (xl_class(C, threads)) {
+#define MGP_XL_CASE(c, nt) case xl_class(c, nt):
+        MGP_XL_CLASSES(MGP_XL_CASE)
+#undef MGP_XL_CASE
+        return true;
+    default: return false;
+    }
 }
 
 int xline_block_rows(int threads) { return XL_THREADS / threads; }

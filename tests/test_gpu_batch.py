@@ -191,3 +191,29 @@ def test_rebuilt_tables_keep_the_bits(method):
         assert (int(it1[0]), int(oc1[0])) == (int(iters[k]), int(outc[k]))
         np.testing.assert_array_equal(alone[0], phis[k])
         assert relres_oracle(*probs[k], phis[k]) <= 1.5e-10
+
+
+# rows of each 256-thread class, one off its edges: (8, 256) up to 2055 cells and (16, 256) up to 4111, beside shorter ones
+LONG = [
+    (64, 64, 0.10, 4.0, (1, 1, 0, 0)),
+    (200, 16, 0.10, 3.0, (1, 1, 0, 0)),
+    (576, 32, 0.05, 1.0, (1, 1, 0, 0)),
+    (1100, 10, 0.05, 1.0, (1, 1, 0, 0)),
+    (2055, 8, 0.05, 1.0, (1, 1, 1, 1)),
+    (2056, 9, 0.05, 1.0, (1, 1, 0, 0)),
+    (4111, 12, 0.05, 1.0, (1, 1, 0, 0)),
+]
+
+
+@pytest.mark.parametrize("method", [mg.METHOD_KRYLOV_MG, mg.METHOD_KRYLOV_MG32])
+def test_long_rows_beside_short_ones(method):
+    """One launch takes rows of every class; alone, a problem's rows take the
+    launch of their class: the same bits either way."""
+    probs = problems(LONG, seed0=90)
+    phis, iters, outc, _ = run_batch(probs, method=method)
+    assert np.all(outc == mg.CONVERGED), (iters, outc)
+    for k, (geo, bc, rhs) in enumerate(probs):
+        assert relres_oracle(geo, bc, rhs, phis[k]) <= 1.5e-10
+        alone, it1, _, _ = run_batch([probs[k]], method=method)
+        assert int(it1[0]) == int(iters[k])
+        np.testing.assert_array_equal(alone[0], phis[k])
