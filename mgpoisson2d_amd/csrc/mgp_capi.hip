@@ -78,14 +78,25 @@ void down_phi(hipStream_t s, double *h, const DevBuf &d, const Grid &g) { downlo
 void up_cc(hipStream_t s, DevBuf &d, const Grid &g, const double *h) { upload_block(s, d.p, g, h, 0, 0, g.nx, g.ny); }
 void down_cc(hipStream_t s, double *h, const DevBuf &d, const Grid &g) { download_block(s, h, d.p, g, 0, 0, g.nx, g.ny); }
 
+// Device bytes of the face data of NONUNIFORM sides.
+size_t face_data_bytes(const mgp_bc *bc, int nx, int ny) {
+    size_t b = 0;
+    for (int k = 0; bc && k < 4; ++k)
+        if (bc->mode[k] == MODE_NONUNIFORM) b += DevArena::rounded((size_t)(k < 2 ? ny : nx) * sizeof(double));
+    return b;
+}
+
 struct Call {
     hipStream_t s;
     std::unique_ptr<DevArena> arena;  // the metrics and the call's fields
     DevGeo geo;
     DevBc bc;
-    Call(const mgp_geo *g, const mgp_bc *b) : s(thread_stream()) {
+    // fields: level arrays that the call takes beside the metrics; table: elements
+    // of a table it takes; scalars and partial sums of reductions: 16 KiB
+    Call(const mgp_geo *g, const mgp_bc *b, int fields, size_t table = 0) : s(thread_stream()) {
         check_geo(g);
-        arena = std::make_unique<DevArena>(10 * (level_elems(g->nx, g->ny) * sizeof(double) + 256));
+        arena = std::make_unique<DevArena>((5 + fields) * DevArena::rounded(level_elems(g->nx, g->ny) * sizeof(double)) +
+                                           DevArena::rounded(table * sizeof(double)) + face_data_bytes(b, g->nx, g->ny) + 16384);
         geo.upload(s, *g);
         if (b) {
             check_bc(b);
@@ -153,7 +164,7 @@ int mgp_device_count(void) {
 
 int mgp_fill_ghosts(const mgp_geo *geo, const mgp_bc *bc, int homog, int do_neum, double *phi) {
     return guarded([&] {
-        Call c(geo, bc);
+        Call c(geo, bc, 1);
         DevBuf f = c.field();
         up_phi(c.s, f, c.geo.g, phi);
         launch_fill_ghosts(c.s, f.p, c.geo.g, c.geo.view(), c.bc.bc, homog, do_neum);
@@ -165,7 +176,7 @@ int mgp_fill_ghosts(const mgp_geo *geo, const mgp_bc *bc, int homog, int do_neum
 int mgp_compute_laplacian(const mgp_geo *geo, const mgp_bc *bc, int homog, int jscale, double *phi, double *lap) {
     return guarded([&] {
         no_lah(bc);
-        Call c(geo, bc);
+        Call c(geo, bc, 2);
         DevBuf f = c.field(), out = c.field();
         up_phi(c.s, f, c.geo.g, phi);
         launch_fill_ghosts(c.s, f.p, c.geo.g, c.geo.view(), c.bc.bc, homog, 0);
@@ -180,7 +191,7 @@ int mgp_compute_residual(const mgp_geo *geo, const mgp_bc *bc, int homog, const 
                          double *res) {
     return guarded([&] {
         no_lah(bc);
-        Call c(geo, bc);
+        Call c(geo, bc, 3);
         DevBuf f = c.field(), r = c.field(), out = c.field();
         up_phi(c.s, f, c.geo.g, phi);
         up_cc(c.s, r, c.geo.g, rhs);
@@ -195,7 +206,7 @@ int mgp_compute_residual(const mgp_geo *geo, const mgp_bc *bc, int homog, const 
 int mgp_compute_invdiags(const mgp_geo *geo, const mgp_bc *bc, int homog, double *invd) {
     return guarded([&] {
         no_lah(bc);
-        Call c(geo, bc);
+        Call c(geo, bc, 1);
         DevBuf out = c.field();
         launch_invdiags(c.s, out.p, c.geo.g, c.geo.view(), c.bc.bc, homog);
         down_cc(c.s, invd, out, c.geo.g);
@@ -212,7 +223,7 @@ int mgp_relax_gs(const mgp_geo *geo, const mgp_bc *bc, int homog, const double *
             g_last_error = "relax_gs ordering must be LEX or MC";
             throw Failure(MGP_ERR_ARG);
         }
-        Call c(geo, bc);
+        Call c(geo, bc, 3);
         if (ordering == MGP_ORDER_MC)
             for (int k = 0; k < 4; ++k)
                 if (bc->type[k] == BC_PERIODIC) {
@@ -240,7 +251,8 @@ int mgp_relax_gs(const mgp_geo *geo, const mgp_bc *bc, int homog, const double *
 int mgp_xline_relax(const mgp_geo *geo, const mgp_bc *bc, const double *rhs, double *phi, int sweeps) {
     return guarded([&] {
         if (sweeps <= 0) return;
-        Call c(geo, bc);
+        check_geo(geo);
+        Call c(geo, bc, 2, ring_table_elems(make_grid(geo->nx, geo->ny, geo->dx, geo->dy)));
         const Grid &g = c.geo.g;
         for (int k = 0; k < 4; ++k)
             if (bc->type[k] != BC_DIRI && bc->type[k] != BC_NEUM) {
@@ -266,7 +278,7 @@ int mgp_xline_relax(const mgp_geo *geo, const mgp_bc *bc, const double *rhs, dou
 
 int mgp_dc_compute_laplacian(const mgp_geo *geo, const mgp_bc *bc, int homog, double *phi, double *lap) {
     return guarded([&] {
-        Call c(geo, bc);
+        Call c(geo, bc, 2);
         DevBuf f = c.field(), out = c.field();
         up_phi(c.s, f, c.geo.g, phi);
         launch_fill_ghosts(c.s, f.p, c.geo.g, c.geo.view(), c.bc.bc, homog, 1);
@@ -279,7 +291,7 @@ int mgp_dc_compute_laplacian(const mgp_geo *geo, const mgp_bc *bc, int homog, do
 
 int mgp_dc_compute_invdiags(const mgp_geo *geo, double *invd) {
     return guarded([&] {
-        Call c(geo, nullptr);
+        Call c(geo, nullptr, 1);
         DevBuf out = c.field();
         launch_dc_invdiags(c.s, out.p, c.geo.g, c.geo.view());
         down_cc(c.s, invd, out, c.geo.g);
@@ -295,7 +307,7 @@ int mgp_dc_relax_gs(const mgp_geo *geo, const mgp_bc *bc, int homog, const doubl
             g_last_error = "DC relax_gs ordering must be LEX or RB";
             throw Failure(MGP_ERR_ARG);
         }
-        Call c(geo, bc);
+        Call c(geo, bc, ordering == MGP_ORDER_RB ? 5 : 4);
         DevBuf f = c.field(), r = c.field(), iv = c.field(), mod = c.field(), tmp;
         up_phi(c.s, f, c.geo.g, phi);
         up_cc(c.s, r, c.geo.g, rhs);
@@ -426,7 +438,7 @@ int mgp_compute_grad(const mgp_geo *geo, const mgp_bc *bc, int homog, double *ph
             g_last_error = "compute_grad: null array";
             throw Failure(MGP_ERR_ARG);
         }
-        Call c(geo, bc);
+        Call c(geo, bc, 3);
         const Grid &g = c.geo.g;
         DevBuf f = c.field(), xf = c.field(), yf = c.field();
         up_phi(c.s, f, g, phi);
@@ -546,7 +558,7 @@ int mgp_compute_residual_dd(const mgp_geo *geo, const mgp_bc *bc, const double *
                 g_last_error = "compute_residual_dd: Dirichlet or Neumann sides (homogeneous, not LAH)";
                 throw Failure(MGP_ERR_UNSUPPORTED);
             }
-        Call c(geo, bc);
+        Call c(geo, bc, 4);
         const Grid &g = c.geo.g;
         DevBuf hi = c.field(), lo = c.field(), f = c.field(), r = c.field();
         up_phi(c.s, hi, g, phi_hi);
@@ -741,7 +753,7 @@ int mgp_relax_jacobi(const mgp_geo *geo, const mgp_bc *bc, int homog, const doub
             g_last_error = "relax_jacobi: maxiters < 0";
             throw Failure(MGP_ERR_ARG);
         }
-        Call c(geo, bc);
+        Call c(geo, bc, 4);
         single_ordering(bc, ordering);
         const Grid &g = c.geo.g;
         DevBuf f = c.field(), r = c.field(), iv = c.field();
@@ -768,7 +780,7 @@ int mgp_solve_bicgstab(const mgp_geo *geo, const mgp_bc *bc, int homog, const do
             g_last_error = "solve_bicgstab: negative iteration limits";
             throw Failure(MGP_ERR_ARG);
         }
-        Call c(geo, bc);
+        Call c(geo, bc, 10);
         single_ordering(bc, ordering);
         const Grid &g = c.geo.g;
         DevBuf f = c.field(), r = c.field(), iv = c.field();
@@ -790,7 +802,7 @@ int mgp_solve_bicgstab2(int kind, const mgp_geo *geo, const mgp_bc *bc, int homo
                         int maxiters, int maxrestarts, int zerophi, const double *rhs, double *phi, int ordering) {
     return guarded([&] {
         if (kind == 0) no_lah(bc);
-        Call c(geo, bc);
+        Call c(geo, bc, kind == 0 && ordering == MGP_ORDER_MC ? 11 : 13);
         const Grid &g = c.geo.g;
         if (kind == 0 && ordering == MGP_ORDER_MC) {
             single_ordering(bc, ordering);
@@ -860,6 +872,22 @@ void mgp_solver_default_opts(mgp_solver_opts *o) {
 extern "C++" {
 namespace {
 
+// The device bytes of a solver's arrays (0: build() refuses the method, the
+// sides or the size).
+size_t solver_bytes(int nx, int ny, double dx, double dy, const mgp_bc &h, const mgp_solver_opts &o) {
+    size_t b = 0;
+    if (o.method == MGP_METHOD_KRYLOV_MG || o.method == MGP_METHOD_KRYLOV_MG32) {
+        Bc bc{};
+        for (int k = 0; k < 4; ++k) bc.type[k] = h.type[k];
+        b = KrylovMG::bytes(nx, ny, bc, o);
+    } else if (o.method == MGP_METHOD_VCYCLE || o.method == MGP_METHOD_FMG || o.method == MGP_METHOD_DC_VCYCLE) {
+        b = RefHierarchy::bytes(nx, ny, dx, dy, o.maxdepth);
+    }
+    if (b == 0) return 0;
+    // metrics, phi and rhs beside the hierarchy
+    return b + 7 * DevArena::rounded(level_elems(nx, ny) * sizeof(double)) + face_data_bytes(&h, nx, ny);
+}
+
 // Shared body of the two create calls: make_geo(stream) fills s->geo.
 template <class MakeGeo>
 int create_solver(mgp_solver **out, int nx, int ny, double dx, double dy, const mgp_bc *bc,
@@ -883,9 +911,7 @@ int create_solver(mgp_solver **out, int nx, int ny, double dx, double dy, const 
             throw Failure(MGP_ERR_ARG);
         }
         hip_check(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking), "hipStreamCreate");
-        const bool krylov = o.method == MGP_METHOD_KRYLOV_MG || o.method == MGP_METHOD_KRYLOV_MG32;
-        const DevArena arena(7 * (level_elems(nx, ny) * sizeof(double) + 256) + 64 * (size_t)(nx + ny) +
-                             (krylov ? KrylovMG::bytes(nx, ny, o) : RefHierarchy::bytes(nx, ny, dx, dy, o.maxdepth)));
+        const DevArena arena(solver_bytes(nx, ny, dx, dy, *bc, o));
         make_geo(s->stream, s->geo);
         s->ubc.upload(s->stream, *bc, nx, ny);
         const size_t n = level_elems(nx, ny);

@@ -51,6 +51,8 @@ class DevArena {
     DevArena &operator=(const DevArena &) = delete;
     // `bytes` of the current block (null: none, or no room), and the block
     static void *take(size_t bytes, std::shared_ptr<DevBlock> &owner);
+    // what an array of `bytes` takes of a block
+    static size_t rounded(size_t bytes) { return (bytes + 255) / 256 * 256; }
 
   private:
     std::shared_ptr<DevBlock> block, outer;

@@ -54,20 +54,22 @@ void dev_free(void *p) { (void)hipFree(p); }
 static thread_local std::shared_ptr<DevBlock> t_block;
 
 DevArena::DevArena(size_t bytes) : outer(t_block) {
-    try {
-        block = std::make_shared<DevBlock>();
-        block->p = static_cast<char *>(dev_alloc_zero(bytes));
-        block->bytes = bytes;
-    } catch (const Failure &) {
-        (void)hipGetLastError();
-        block.reset();
+    if (bytes) {
+        try {
+            block = std::make_shared<DevBlock>();
+            block->p = static_cast<char *>(dev_alloc_zero(bytes));
+            block->bytes = bytes;
+        } catch (const Failure &) {
+            (void)hipGetLastError();
+            block.reset();
+        }
     }
     t_block = block;
 }
 DevArena::~DevArena() { t_block = outer; }
 
 void *DevArena::take(size_t bytes, std::shared_ptr<DevBlock> &owner) {
-    const size_t b = (bytes + 255) / 256 * 256;
+    const size_t b = rounded(bytes);
     if (!t_block || b > t_block->bytes - t_block->used) return nullptr;
     void *p = t_block->p + t_block->used;
     t_block->used += b;
@@ -407,9 +409,9 @@ void RefHierarchy::build(hipStream_t s, const DevGeo &top, const Bc &user_bc, in
 size_t RefHierarchy::bytes(int nx, int ny, double dx, double dy, int maxdepth_user) {
     std::vector<int> rx, ry;
     const int depth = reference_schedule(nx, ny, dx, dy, maxdepth_user, rx, ry);
-    size_t b = 4096;
+    size_t b = DevArena::rounded(8 * sizeof(double));
     for (int d = 0;; ++d) {
-        const size_t n = level_elems(nx, ny) * sizeof(double) + 256;
+        const size_t n = DevArena::rounded(level_elems(nx, ny) * sizeof(double));
         b += 10 * n;
         if (d == depth) return b + 9 * n;
         nx /= rx[d];

@@ -22,8 +22,9 @@ struct KrylovMG {
     // fourth-order operator (o.order == 4) needs it for its face-averaged metrics.
     void build(hipStream_t s, const DevGeo &top, const Bc &user_bc, const mgp_solver_opts &o,
                const mgp_mapping *map = nullptr);
-    // About the device bytes build() allocates, an FGMRES basis aside.
-    static size_t bytes(int nx, int ny, const mgp_solver_opts &o);
+    // The device bytes build() allocates, an FGMRES basis aside (0: sides or a
+    // size it refuses).
+    static size_t bytes(int nx, int ny, const Bc &bc, const mgp_solver_opts &o);
     // Low part of the double-double solution (MGP_REFINE_DD; null otherwise).
     double *phi_lo() const;
     // rhs -= J sum(rhs) / sum(J) over the valid cells (the compatibility

@@ -138,19 +138,46 @@ void KrylovMG::ensure_fgmres(const Grid &g) {
     hip_check(hipHostMalloc((void **)&K.ghost, (size_t)(4 * m + 6) * sizeof(double)), "hipHostMalloc");
 }
 
-size_t KrylovMG::bytes(int nx, int ny, const mgp_solver_opts &o) {
-    const bool mixed = o.method == MGP_METHOD_KRYLOV_MG32;
-    const size_t n0 = level_elems(nx, ny) * sizeof(double) + 256;
-    size_t b = 65536 + 9 * n0;                                           // Krylov vectors
-    if (o.refine == MGP_REFINE_DD) b += 3 * n0;
-    if (o.order == 4) b += 8 * n0;
-    for (int lev = 0; ny >= MIN_COARSE_NY; ++lev) {
-        const size_t n = level_elems(nx, ny) * sizeof(double) + 256;
-        const size_t small = (size_t)ring_table_elems(make_grid(nx, ny, 1.0, 1.0)) * 12 + (size_t)level_pitch(nx) * 16 + 1024;
-        b += 5 * n + small + (!mixed || lev == 0 ? 3 * n : 0) + (mixed ? 3 * n + 1024 : 0);
-        if (o.maxdepth >= 0 && lev >= o.maxdepth) break;
-        int off = 0;
-        ny = semicoarsen_step(ny, MIN_COARSE_NY, true, true, off);
+// AUTO: x-lines where the cycle's element type solves the rows whole, else
+// y-lines where it solves the columns whole, else rows in segments.
+static bool y_lines(int nx, int ny, const mgp_solver_opts &o) {
+    const size_t celem = o.method == MGP_METHOD_KRYLOV_MG32 ? sizeof(float) : sizeof(double);
+    return o.lines == MGP_LINES_Y || (o.lines == MGP_LINES_AUTO && !xline_whole(nx, celem) && xline_whole(ny, celem));
+}
+
+// Rows of the hierarchy's levels, the finest first, each with KLevel::off.
+struct LevelRows {
+    int ny, off;
+};
+static std::vector<LevelRows> level_rows(int ny, bool neum_lo, bool neum_hi, int maxdepth) {
+    std::vector<LevelRows> rows;
+    const int maxlev = maxdepth < 0 ? 64 : maxdepth + 1;
+    while (true) {
+        rows.push_back(LevelRows{ny, 0});
+        if ((int)rows.size() >= maxlev) return rows;
+        const int nyc = semicoarsen_step(ny, MIN_COARSE_NY, neum_lo, neum_hi, rows.back().off);
+        if (nyc == 0) return rows;
+        ny = nyc;
+    }
+}
+
+size_t KrylovMG::bytes(int nx, int ny, const Bc &bc, const mgp_solver_opts &o) {
+    const bool mixed = o.method == MGP_METHOD_KRYLOV_MG32, tr = y_lines(nx, ny, o);
+    const auto arr = [](size_t n, size_t elem) { return DevArena::rounded(n * elem); };
+    const size_t d = sizeof(double), f = sizeof(float);
+    for (int k = 0; k < 4; ++k)
+        if (bc.type[k] != BC_DIRI && bc.type[k] != BC_NEUM) return 0;
+    if (nx < 4 || ny < 4 || xline_segments(tr ? ny : nx, mixed ? f : d) == 0) return 0;
+    size_t b = (size_t)(9 + (o.refine == MGP_REFINE_DD ? 3 : 0) + (o.order == 4 ? 8 : 0)) * arr(level_elems(nx, ny), d);
+    b += arr(2, d) + arr(SC_COUNT, d) + arr(2 * (size_t)reduce_blocks(make_grid(nx, ny, 1.0, 1.0)) + 8, d);
+    const Bc bc0 = tr ? transposed_bc(bc) : bc;
+    if (tr) std::swap(nx, ny);
+    bool finest = true;
+    for (const LevelRows &l : level_rows(ny, bc0.type[YLO] == BC_NEUM, bc0.type[YHI] == BC_NEUM, o.maxdepth)) {
+        const size_t n = level_elems(nx, l.ny), K = (size_t)ring_table_elems(make_grid(nx, l.ny, 1.0, 1.0));
+        b += (5 + (!mixed || finest ? 3 : 0)) * arr(n, d) + arr(K, d) + arr((size_t)2 * level_pitch(nx), mixed ? f : d);
+        if (mixed) b += 6 * arr(n, f) + arr(K, f);
+        finest = false;
     }
     return b;
 }
@@ -173,11 +200,8 @@ void KrylovMG::build(hipStream_t s, const DevGeo &top, const Bc &user_bc, const 
                        "BICGSTAB or FGMRES, restart 0..200";
         throw Failure(MGP_ERR_ARG);
     }
-    // AUTO: x-lines where the cycle's element type solves the rows whole,
-    // else y-lines where it solves the columns whole, else rows in segments
     const size_t celem = o.method == MGP_METHOD_KRYLOV_MG32 ? sizeof(float) : sizeof(double);
-    const bool tr = o.lines == MGP_LINES_Y ||
-                    (o.lines == MGP_LINES_AUTO && !xline_whole(top.g.nx, celem) && xline_whole(top.g.ny, celem));
+    const bool tr = y_lines(top.g.nx, top.g.ny, o);
     if (xline_segments(tr ? top.g.ny : top.g.nx, celem) == 0) {
         g_last_error = "KRYLOV_MG: no line solve for this size (lines of at most 4111 cells, 8207 in the FP32 "
                        "cycle, or cut into at most 64 equal segments of that length; with y-lines, columns)";
@@ -222,13 +246,12 @@ void KrylovMG::build(hipStream_t s, const DevGeo &top, const Bc &user_bc, const 
     // the hierarchy's finest grid and BCs: the caller's, or the transposed ones
     const Grid g0 = tr ? make_grid(top.g.ny, top.g.nx, top.g.dy, top.g.dx) : top.g;
     const Bc bc0 = tr ? transposed_bc(user_bc) : user_bc;
-    int ny = g0.ny;
     double dy = g0.dy;
-    const int maxlev = o.maxdepth < 0 ? 64 : o.maxdepth + 1;
-    while (true) {
+    for (const LevelRows &rows : level_rows(g0.ny, bc0.type[YLO] == BC_NEUM, bc0.type[YHI] == BC_NEUM, o.maxdepth)) {
         L.emplace_back();
         KLevel &l = L.back();
-        l.g = make_grid(g0.nx, ny, g0.dx, dy);
+        l.g = make_grid(g0.nx, rows.ny, g0.dx, dy);
+        l.off = rows.off;
         const size_t n = level_elems(l.g.nx, l.g.ny);
         for (DevBuf *b : {&l.J, &l.Jxx, &l.Jxy, &l.Jyx, &l.Jyy}) b->alloc(n);
         // FP64 level fields: the FP64 cycle, and on the finest level the
@@ -282,10 +305,6 @@ void KrylovMG::build(hipStream_t s, const DevGeo &top, const Bc &user_bc, const 
             l.r32.alloc(n);
             l.geo32 = GeoF{nullptr, l.Jxx32.p, l.Jxy32.p, l.Jyx32.p, l.Jyy32.p};
         }
-        if ((int)L.size() >= maxlev) break;
-        const int nyc = semicoarsen_step(ny, MIN_COARSE_NY, bc0.type[YLO] == BC_NEUM, bc0.type[YHI] == BC_NEUM, l.off);
-        if (nyc == 0) break;
-        ny = nyc;
         dy *= 2.0;
     }
     const size_t n0 = level_elems(top.g.nx, top.g.ny);
@@ -302,10 +321,10 @@ void KrylovMG::build(hipStream_t s, const DevGeo &top, const Bc &user_bc, const 
         DevBuf *m = impl->m4;
         launch_metric4(s, *map, top.g, Geo4W{m[0].p, m[1].p, m[2].p, m[3].p, m[4].p, m[5].p, m[6].p, m[7].p});
     }
-    if (impl->fgmres) ensure_fgmres(top.g);
     impl->sums.alloc(2);
     impl->scal.alloc(SC_COUNT);
     impl->partial.alloc(2 * (size_t)reduce_blocks(top.g) + 8);  // two products' partials, the blocks' count
+    if (impl->fgmres) ensure_fgmres(top.g);  // past the arrays that bytes() counts
     hip_check(hipHostMalloc((void **)&impl->host, SC_COUNT * sizeof(double)), "hipHostMalloc");
     impl->use_graph = o.use_graph != 0;
     built = true;
