@@ -55,12 +55,15 @@ static thread_local std::shared_ptr<DevBlock> t_block;
 
 DevArena::DevArena(size_t bytes) : outer(t_block) {
     if (bytes) {
+        const std::string error = g_last_error;
+        block = std::make_shared<DevBlock>();
         try {
-            block = std::make_shared<DevBlock>();
             block->p = static_cast<char *>(dev_alloc_zero(bytes));
             block->bytes = bytes;
-        } catch (const Failure &) {
+        } catch (const Failure &f) {
+            if (f.status != MGP_ERR_NOMEM) throw;
             (void)hipGetLastError();
+            g_last_error = error;
             block.reset();
         }
     }
