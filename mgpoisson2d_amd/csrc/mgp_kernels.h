@@ -51,6 +51,9 @@ bool dc_rb_relax(hipStream_t s, double *phi, double *tmp, double *mod, const dou
 // tile shape k - 1 of dc_rb_tile_shapes().  Returns the previous setting.
 int dc_rb_tile_choice(int choice);
 int dc_rb_tile_shapes();
+// The shape of a level whose shapes are not timed: below 256^2 cells, and any
+// level while its stream is being captured (the fewest window cells there).
+int dc_rb_tile_untimed(int nx, int ny, int S);
 // One tile launch of S sweeps with the modified rhs formed in the kernel,
 // phi -> out (measurement); returns the tile shape used.
 int dc_rb_tile_once(hipStream_t s, const double *phi, double *out, const double *rhs, const double *invd,

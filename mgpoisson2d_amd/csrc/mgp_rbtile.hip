@@ -279,6 +279,7 @@ std::map<std::tuple<int, int, int, int>, int> rb_picked;
 // Small levels do not fill the CUs: a launch takes as long as one window, and
 // that grows with the rows each wave holds (a level of 64^2: 21 us with 8 rows
 // a wave, 8 to 10 us with 4).
+constexpr long long RB_TIMED_CELLS = 256LL * 256;
 constexpr int RB_SMALL = 4;  // {16, 8}: two rows a wave
 
 // The shape for this level, sweeps per load and form: timed once per
@@ -298,8 +299,8 @@ int rb_pick(hipStream_t s, int S, bool fuse, const double *in, double *out, cons
     }
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     hip_check(hipStreamIsCapturing(s, &cs), "hipStreamIsCapturing");
-    if ((long long)g.nx * g.ny < 256LL * 256 || cs != hipStreamCaptureStatusNone) {
-        const int k = RB_SMALL;
+    if ((long long)g.nx * g.ny < RB_TIMED_CELLS || cs != hipStreamCaptureStatusNone) {
+        const int k = dc_rb_tile_untimed(g.nx, g.ny, S);
         if (cs == hipStreamCaptureStatusNone) {
             std::lock_guard<std::mutex> lk(rb_mu);
             rb_picked.emplace(key, k);
@@ -343,6 +344,19 @@ int dc_rb_tile_choice(int choice) {
 }
 
 int dc_rb_tile_shapes() { return RB_NSHAPES; }
+
+int dc_rb_tile_untimed(int nx, int ny, int S) {
+    if ((long long)nx * ny < RB_TIMED_CELLS) return RB_SMALL;
+    const Grid g = make_grid(nx, ny, 1.0, 1.0);
+    int best = 0;
+    long long bestc = -1;
+    for (int k = 0; k < RB_NSHAPES; ++k) {
+        int ntx;
+        const long long c = (long long)rb_tiles(g, k, S, ntx) * RB_WW * RB_SHAPES[k].H;
+        if (bestc < 0 || c < bestc) best = k, bestc = c;
+    }
+    return best;
+}
 
 int dc_rb_tile_once(hipStream_t s, const double *phi, double *out, const double *rhs, const double *invd,
                     const Grid &g, const Geo &geo, const Bc &bc, double omega, int S) {
