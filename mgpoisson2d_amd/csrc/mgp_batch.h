@@ -137,8 +137,9 @@ class BatchKMG {
     static size_t problem_bytes(const Problem &q, const mgp_solver_opts &o);
     // Measurement hook: mean ms of `reps` back-to-back launch sets of the
     // finest-level line relaxation of the even interior rows of every problem
-    // (as in a solve), timed with HIP events on the batch's stream; *bytes the algorithmic bytes of one
-    // set (each array element it needs once, the element size of the cycle).
+    // of more than one level (launched as in a solve), timed with HIP events on
+    // the batch's stream; *bytes the algorithmic bytes of one set (each array
+    // element it needs once, the element size of the cycle).
     // Between solves only: it relaxes the resident finest-level corrections.
     double time_fine_xline(int reps, double *bytes);
 
@@ -235,6 +236,8 @@ class BatchKMG {
     XlPhase stage_phase(TableSet &ts, int d, int set, int colour, const XlRows &rows);
     void upload(TableSet &ts);
     void launch_phase(const XlPhase &ph, int sel, int k);
+    void add_interior_even(XlRows &rows, int p, int C, int NT) const;
+    double time_rows(const XlRows &rows, int reps);
     void build_tables(TableSet &ts, const std::vector<int> &which);
     void release(TableSet &ts);       // the graph and the tables' contents (waits for the stream)
     void free_buffers(TableSet &ts);  // and the buffers

@@ -901,15 +901,10 @@ std::vector<int> BatchKMG::finish_step() {
 }
 
 double BatchKMG::time_fine_xline(int reps, double *bytes) {
-    if (T != &full) {
-        release(part);
-        T = &full;
-    }
     const int n = count();
-    // the even rows of level 0 (colour 0 of the first zebra phase; the bytes
-    // count its interior rows)
     const double es = mixed ? 4.0 : 8.0;
     double b = 0.0;
+    XlRows rows;
     for (int p = 0; p < n; ++p) {
         if (nlev[p] < 2) continue;  // a single-level problem's rows are in the bottom set
         const Grid &g = P[p].g;
@@ -917,28 +912,50 @@ double BatchKMG::time_fine_xline(int reps, double *bytes) {
         // e on rows 1 .. 2R+1 and written on R rows; f, Jxx, Jxy on R rows;
         // Jyx, Jyy on 2R face rows; 9 table entries for the 2R ring cells
         b += g.nx * es * ((2.0 * R + 1.0) + R + R + R + 2.0 * R + 2.0 * R + R) + R * 2.0 * 9.0 * es;
+        add_interior_even(rows, p, Cp[p], NTp[p]);
     }
     *bytes = b;
     std::vector<int> all(n, 1);
     upload_flags(active, all);
-    auto launch_set = [&]() {
-        for (const XlPhase &x : T->xl)
-            if (x.d == 0 && x.set == SET_MID && x.colour == 0) launch_phase(x, 0, -1);
-    };
-    hipEvent_t a = nullptr, e = nullptr;
-    hip_check(hipEventCreate(&a), "event");
-    hip_check(hipEventCreate(&e), "event");
-    launch_set();  // warm
-    hip_check(hipEventRecord(a, s), "event");
-    for (int k = 0; k < reps; ++k) launch_set();
-    hip_check(hipEventRecord(e, s), "event");
-    hip_check(hipEventSynchronize(e), "event");
-    float ms = 0.0f;
-    hip_check(hipEventElapsedTime(&ms, a, e), "event");
-    (void)hipEventDestroy(a);
-    (void)hipEventDestroy(e);
+    const double ms = time_rows(rows, reps);
     upload_flags(active, act_);
     hip_check(hipStreamSynchronize(s), "sync");
+    return ms;
+}
+
+// The even interior rows of problem p's finest level, in shape (C, NT).
+void BatchKMG::add_interior_even(XlRows &rows, int p, int C, int NT) const {
+    const Grid &g = P[p].g;
+    const size_t lds = xline_lds_bytes_for(g.nx, C, mixed ? sizeof(float) : sizeof(double), NT);
+    for (int j = 2; j < g.ny - 1; j += 2) rows.add(C, NT, lds, XlTask{P[p].lev0, j, 0, 0});
+}
+
+// Mean ms of `reps` launch sets of the rows, launched as inside a solve.
+double BatchKMG::time_rows(const XlRows &rows, int reps) {
+    TableSet ts;
+    hipEvent_t a = nullptr, e = nullptr;
+    float ms = 0.0f;
+    auto release_all = [&] {
+        free_buffers(ts);
+        if (a) (void)hipEventDestroy(a);
+        if (e) (void)hipEventDestroy(e);
+    };
+    try {
+        ts.xl.push_back(stage_phase(ts, 0, SET_MID, 0, rows));
+        upload(ts);
+        hip_check(hipEventCreate(&a), "event");
+        hip_check(hipEventCreate(&e), "event");
+        launch_phase(ts.xl[0], 0, -1);  // warm
+        hip_check(hipEventRecord(a, s), "event");
+        for (int r = 0; r < reps; ++r) launch_phase(ts.xl[0], 0, -1);
+        hip_check(hipEventRecord(e, s), "event");
+        hip_check(hipEventSynchronize(e), "event");
+        hip_check(hipEventElapsedTime(&ms, a, e), "event");
+    } catch (...) {
+        release_all();
+        throw;
+    }
+    release_all();
     return ms / reps;
 }
 
@@ -996,44 +1013,16 @@ int BatchKMG::set_tuning(const std::vector<TuneEntry> &t) {
 }
 
 // Mean ms of `reps` launch sets of the finest-level even-row line relaxation
-// of every problem with shapes (C[p], NT[p]), launched as inside a solve.  Sets the level table's
+// of every problem with shapes (C[p], NT[p]).  Sets the level table's
 // finest-level chunk counts to those shapes (apply_shapes restores them).
 double BatchKMG::time_shapes(const std::vector<int> &C, const std::vector<int> &NT, int reps) {
-    const int n = count();
-    const size_t elem = mixed ? sizeof(float) : sizeof(double);
     XlRows rows;
-    for (int p = 0; p < n; ++p) {
-        const int nx = P[p].g.nx, ny = P[p].g.ny, lev = P[p].lev0;
-        L[lev].nt = nx / C[p];
-        for (int j = 2; j < ny - 1; j += 2)
-            rows.add(C[p], NT[p], xline_lds_bytes_for(nx, C[p], elem, NT[p]), XlTask{lev, j, 0, 0});
+    for (int p = 0; p < count(); ++p) {
+        L[P[p].lev0].nt = P[p].g.nx / C[p];
+        add_interior_even(rows, p, C[p], NT[p]);
     }
     hip_check(hipMemcpyAsync(dL, L.data(), L.size() * sizeof(BLev), hipMemcpyHostToDevice, s), "level table");
-    TableSet ts;
-    ts.xl.push_back(stage_phase(ts, 0, SET_MID, 0, rows));
-    upload(ts);
-    auto launch_set = [&]() { launch_phase(ts.xl[0], 0, -1); };
-    hipEvent_t a = nullptr, e = nullptr;
-    float ms = 0.0f;
-    try {
-        hip_check(hipEventCreate(&a), "event");
-        hip_check(hipEventCreate(&e), "event");
-        launch_set();  // warm
-        hip_check(hipEventRecord(a, s), "event");
-        for (int r = 0; r < reps; ++r) launch_set();
-        hip_check(hipEventRecord(e, s), "event");
-        hip_check(hipEventSynchronize(e), "event");
-        hip_check(hipEventElapsedTime(&ms, a, e), "event");
-    } catch (...) {
-        free_buffers(ts);
-        if (a) (void)hipEventDestroy(a);
-        if (e) (void)hipEventDestroy(e);
-        throw;
-    }
-    free_buffers(ts);
-    (void)hipEventDestroy(a);
-    (void)hipEventDestroy(e);
-    return ms / reps;
+    return time_rows(rows, reps);
 }
 
 // Coordinate search over row-length bands (rows of up to 128, 256, 512, 1024
