@@ -54,16 +54,14 @@ def test_ordered_mean(nx, ny):
     np.testing.assert_array_equal(got[1:-1, 1:-1], want[1:-1, 1:-1])
 
 
-@pytest.mark.parametrize("n", [32, 64, 96, 160])
+# lexicographic sweeps are one workgroup: the small sizes only
+@pytest.mark.parametrize("n,order", [(32, rc.LEX), (64, rc.LEX), (32, rc.RB), (64, rc.RB), (96, rc.RB), (160, rc.RB)])
 @pytest.mark.parametrize("types", [(1, 1, 0, 0), (1, 1, 1, 1), (0, 1, 1, 0), (0, 0, 0, 0), (2, 2, 1, 1)])
-@pytest.mark.parametrize("order", [rc.LEX, rc.RB])
 @pytest.mark.parametrize("numcycles,up", [(1, 2), (2, 1), (1, 0)])
 def test_dc_cycle_transfers(n, types, order, numcycles, up):
     """The DC cycle's fused transfers (Neumann and Dirichlet sides, smoothing
     after the correction) and the separate ones (a periodic side, or none):
     two cycles against the oracle, bit for bit where no parallel sum enters."""
-    if order == rc.LEX and n > 64:
-        pytest.skip("lexicographic sweeps are one workgroup")
     geo, bc, phi, rhs = setup(n, n, 0.02, 0.3, types, seed=n)
     o = rc.oracle()
     args = dict(numcycles=numcycles, zerophi=True)
