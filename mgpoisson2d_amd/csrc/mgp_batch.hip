@@ -48,10 +48,11 @@ __device__ __forceinline__ void tile_cells(const BTile &t, const Grid &g, F &&f)
 }
 
 // v[out] = (v[rhs] -) A v[in], A the reference operator with the problem's
-// homogeneous BCs (ghosts synthesised from the valid cells).  Bound by memory
-// (48 bytes a cell).  Four rows a thread: 81 us over the batch of 256 problems
-// and 11.7 over 24 odd ones, 146 and 26 with the rows' cells loaded each by
-// itself and the ring's stencil among them.
+// homogeneous BCs (ghosts synthesised from the valid cells).  Bound by memory:
+// 48 bytes a cell, 270 us for the 20.6 M cells of 256 problems (3.7 TB/s).  Four
+// rows a thread; the mean of a launch over a whole solve, finished problems
+// masked, is 81 us for those 256 and 11.7 for 24 odd ones, 146 and 26 with the
+// rows' cells loaded each by itself and the ring's stencil among them.
 __global__ void __launch_bounds__(256) k_b_apply(const BTile *tiles, const BProb *P, const int *mask, int out, int in,
                                                  int rhs) {
     const BTile t = tiles[blockIdx.x];
@@ -239,8 +240,9 @@ __global__ void __launch_bounds__(256) k_b_end32(const BTile *tiles, const BProb
 
 // Row blocks of a problem's reductions: about 2048 cells each, 8 per thread,
 // which is one round of k_b_reduce_partial's loads (rows b, b + nb, ..): with
-// 8192 cells, four rounds one after the other, a pass took 29 us over 24 odd
-// problems and 47 over 256, now 11 and 30.
+// 8192 cells, four rounds one after the other, the mean pass of a whole solve
+// (finished problems masked) took 29 us for 24 odd problems and 47 for 256, now
+// 11 and 30; one over all 256 (two vectors, 330 MB) takes 58.
 int reduce_rows(int nx, int ny) { return std::max(1, std::min(ny, (nx * ny + 2047) / 2048)); }
 
 size_t round256(size_t b) { return (b + 255) / 256 * 256; }

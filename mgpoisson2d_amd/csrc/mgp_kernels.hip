@@ -1285,8 +1285,11 @@ __device__ __forceinline__ void bicg_scalars(double *sc, int op) {
 // is) into sc[slot0] and sc[slot1] and computes the scalars that follow.
 // count is 0 before and after.  No block waits for another.  The partial sums
 // pass from block to block by agent-scope atomics, each performed before the
-// count goes up: a release and acquire instead write back and drop the L2 in
-// every block, 12 to 20 us a pass with 512 to 1024 blocks.
+// count goes up: its exchange has returned (the asm below uses the value, which
+// makes the compiler wait for it, s_waitcnt vmcnt(0), before the count's
+// atomic).  A release of workgroup scope there adds no instruction; one of agent
+// scope, with an acquire, writes back and drops the L2 in every block, 12 to 20
+// us a pass with 512 to 1024 blocks.
 template <int N>
 __device__ __forceinline__ void bicg_finish(double *ss, double *cc, double *partial, unsigned *count, double *sc,
                                             const double (&sum)[N], int slot0, int slot1, int op) {

@@ -340,9 +340,20 @@ void KrylovMG::build(hipStream_t s, const DevGeo &top, const Bc &user_bc, const 
 //
 // Relaxing rows 0 and ny-1 after their neighbours, on the values of both, puts
 // two row solves one after the other into the odd-row launch, and a coarse
-// level's launch takes as long as its longest workgroup.  Solves took as many
-// V-cycles either way (64^2 32 against 40, 512^2 60 against 58, 2048^2 62
-// against 58); 64^2 10.56 -> 6.95 ms, 512^2 43.4 -> 37.5, 2048^2 116.0 -> 104.0.
+// level's launch takes as long as its longest workgroup: 64^2 10.56 -> 6.95 ms,
+// 512^2 43.4 -> 37.5, 2048^2 116.0 -> 104.0 with the rows beside the others.
+// It is another smoother, and V-cycle counts move both ways.  Rows after -> rows
+// beside, flexible GMRES to one tolerance: 64^2 at beta 5 29 -> 24, 333 x 257 28
+// -> 23, 1024 x 768 36 -> 37, 512^2 at beta 5 54 -> 62, 2048^2 at beta 4 49 ->
+// 55 and at beta 5 92 -> 107, 8192 x 2048 at beta 8 405 -> 463 with FP32 cycles
+// and 711 -> 619 with FP64 ones; 1024 mixed problems 21.7 on average either way,
+// the worst 84 -> 98 (FP32) and 94 -> 94.  Large strongly stretched grids pay up
+// to 16 %, and the 8192 x 2048 solve with FP32 cycles is slower for it (2.20 ->
+// 2.35 s); the others measured are faster or even.  Every level has its share:
+// for 2048^2 at beta 5 and 8192 x 2048 FP32, the old order on the levels of more
+// than 512 rows alone leaves 107 and 461 V-cycles, on those of up to 15 rows 103
+// and 459, up to 127 98 and 425, up to 255 96 and 411, and there 64^2 is back at
+// 29 and takes 1.7 times as long (the boundary rows in a launch of their own).
 template <typename T, typename G>
 static void zebra(hipStream_t s, const Grid &g, const G &geo, const T *K, T *e, const T *f, T *far) {
     const int ny = g.ny;

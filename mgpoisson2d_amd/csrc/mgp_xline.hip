@@ -12,7 +12,7 @@
 // extrapolations and the Dirichlet ghost rule, use an explicit coefficient
 // table probed once per level with unit impulses (k_ring_coef).
 //
-// One workgroup (64 to 512 threads) per row:
+// One workgroup (64 to 1024 threads) per row:
 //  1. coalesced pass: each thread evaluates d = f - L e and the row
 //     coefficients for cells i = tid + NT u (groups of loads issued up front);
 //  2. the values go through LDS into contiguous chunks of C or C+1 cells
@@ -54,7 +54,7 @@ constexpr int XL_WIDE = 512;
 // The single-problem solver's launches of few rows (up to two per CU: every
 // coarse level) take as long as one row solve, so they use more threads per
 // row than the fine levels' launches, whose many rows fill the CUs: rows of
-// 129 .. 512 cells 256 threads instead of one wave (512^2 FP64 35.5 -> 28.8 ms;
+// 129 .. 512 cells 256 threads instead of one wave (512^2 FP64 37.5 -> 31.1 ms;
 // at 128 cells and below one wave is as fast or faster), FP32 rows of 1025 ..
 // 2048 cells 512 threads (1500 x 800: 18.7 -> 16.9 ms; FP64 rows of that length
 // and rows of 513 .. 1024 cells were slower by 7 and 12 %).
@@ -228,18 +228,6 @@ __device__ __forceinline__ RowCtx<T> row_ctx(const Grid &g, int nt, int C) {
     return r;
 }
 
-// Coalesced pass over row j: for cells i = tid + 256 u, the residual
-// d = f - L e and the row coefficients a, b, c, written into the chunk layout
-// (Ld, La, Lb, Lc).  Interior cells use the metric stencil, ring cells the
-// table.  Lanes past the row end evaluate the last cell and store into the
-// chunk layout's last slot, which no chunk uses (the last chunk has C cells):
-// the loop stays branch-free.
-//
-// RG cells' loads are issued together before their stencils are evaluated,
-// so RG memory round trips overlap instead of following one another (one
-// cell at a time, a coarse-level row pass took 5.4 us of a 10.6 us row
-// solve).  The batched kernels take the RG of batch_rg: no more than fits
-// their VGPR budget, since they rely on many workgroups per CU.
 // Buffer-addressed reads of a field of a level: one 32-bit byte offset per
 // cell in a vector register, the row offsets (multiples of the pitch) in
 // scalar registers and the column neighbours in the instruction's immediate
@@ -260,6 +248,18 @@ struct Buf {
     }
 };
 
+// Coalesced pass over row j: for cells i = tid + NT u, the residual
+// d = f - L e and the row coefficients a, b, c, written into the chunk layout
+// (Ld, La, Lb, Lc).  Interior cells use the metric stencil, ring cells the
+// table.  Lanes past the row end evaluate the last cell and store into the
+// chunk layout's last slot, which no chunk uses (the last chunk has C cells):
+// the loop stays branch-free.
+//
+// RG cells' loads are issued together before their stencils are evaluated,
+// so RG memory round trips overlap instead of following one another (one
+// cell at a time, a coarse-level row pass took 5.4 us of a 10.6 us row
+// solve).  The batched kernels take the RG of batch_rg: no more than fits
+// their VGPR budget, since they rely on many workgroups per CU.
 template <int C, int NT, bool SEG = false, int RG = 1, typename T, typename GM>
 __device__ __forceinline__ void row_pass(const RowCtx<T> &X, const T *e_, const T *f_, const T *K_, const Grid &g,
                                          const GM &geo_, int j, const T *far, int tid, T *Ld, T *La, T *Lb, T *Lc,
@@ -705,11 +705,14 @@ __global__ void __launch_bounds__(XL_THREADS) k_xline_long(T *__restrict__ e, co
 // 64 x 4 R N coarse cells from (i0, J0) by a workgroup of 256 threads: a wave
 // takes N times R coarse rows of the interior columns, 2 R fine rows at a
 // stretch (lap_rows), then the coarse cells of one side of the ring.  Bound by
-// memory on the fine levels.  One level a launch, R = 1: 11.9 us over the nine
-// levels of 2048 x 2048 cells (16.1 with the ring's cells among the others; R =
-// 2 the same, and 5.6 against 4.8 on the levels of 512 x 512).  Batched, R = 2
-// and N = 2: 7.4 us (13.3) over 24 odd FP64 problems, 19.1 (25.5) over 256 FP32
-// ones; R = 1 takes 7.8 and 19.9, R = 4 7.3 and 18.8 with 190 registers.
+// memory on the fine levels: 56 bytes a fine cell, 40 us on the finest level of
+// 2048 x 2048 (235 MB).  Of one level a launch, R = 1, the mean over that
+// grid's nine levels is 11.9 us (16.1 with the ring's cells among the others; R
+// = 2 the same, and 5.6 against 4.8 on the levels of 512 x 512).  Batched, R = 2
+// and N = 2, means over the levels and a whole solve with its finished problems
+// masked: 7.4 us (13.3) for 24 odd FP64 problems, 19.1 (25.5) for 256 FP32 ones;
+// R = 1 takes 7.8 and 19.9, R = 4 7.3 and 18.8 with 190 registers.  The finest
+// level of all 256 takes 126 us.
 template <int R, int N, typename T, typename G>
 __device__ __forceinline__ void restrict_tile(T *rc, T *ec, T *farc, const T *e, const T *f, const T *K,
                                               const Grid &gf, const Grid &gc, const G &geo, int off, int i0, int J0) {
