@@ -397,11 +397,11 @@ int mgp_batch_solve(mgp_batch *b, double tol, int maxiters, int zerophi, int *it
 /* V-cycle applications of the longest-running problem in the last solve. */
 int mgp_batch_last_cycles(const mgp_batch *b);
 /* Measurement hook (between solves): times `reps` back-to-back launch sets of the finest-level
- * line relaxation of the even interior rows of every problem (kernel 0; launched as inside a
- * solve) with HIP events on the batch's stream.  *avg_ms is the
- * mean per set, *bytes the algorithmic bytes of one set (each array element it needs once, at
- * the element size of the cycle: 8 bytes, or 4 with KRYLOV_MG32).  Changes the resident
- * finest-level corrections, nothing else. */
+ * line relaxation of the even interior rows of every problem of more than one level (kernel 0;
+ * launched as inside a solve) with HIP events on the batch's stream.  *avg_ms is the mean per set,
+ * *bytes the algorithmic bytes of one set (each array element it needs once, at the element size
+ * of the cycle: 8 bytes, or 4 with KRYLOV_MG32).  Changes the resident finest-level corrections,
+ * nothing else. */
 int mgp_batch_time_kernel(mgp_batch *b, int kernel, int reps, double *avg_ms, double *bytes);
 /* Autotuner of the batched line solve (no counterpart in the reference).  The shape of a row's
  * line solve -- threads per row (64, 128 or 256) and with it the chunk length -- is chosen per key
