@@ -263,14 +263,13 @@ BatchKMG::Table BatchKMG::stage(TableSet &ts, const void *host, size_t bytes, in
     const size_t off = round256(ts.used);
     if (off + bytes > ts.hcap) {
         const size_t cap = std::max(off + bytes, 2 * ts.hcap);
-        unsigned char *h = nullptr;
-        if (hipHostMalloc((void **)&h, cap, hipHostMallocDefault) != hipSuccess || !h) {
-            (void)hipGetLastError();
+        unsigned char *h = static_cast<unsigned char *>(host_alloc(cap));
+        if (!h) {
             g_last_error = "batch: pinned staging of " + std::to_string(cap) + " bytes for the launch tables";
             throw Failure(MGP_ERR_NOMEM);
         }
         if (ts.used) memcpy(h, ts.host, ts.used);
-        if (ts.host) (void)hipHostFree(ts.host);
+        host_free(ts.host);
         ts.host = h;
         ts.hcap = cap;
     }
@@ -501,7 +500,7 @@ BatchKMG::BatchKMG(hipStream_t s_, const std::vector<Problem> &probs, const mgp_
     hip_check(hipMemcpyAsync(dL, L.data(), L.size() * sizeof(BLev), hipMemcpyHostToDevice, s), "level table");
     active = static_cast<int *>(dev_alloc_zero(n * sizeof(int)));
     mask = static_cast<int *>(dev_alloc_zero(n * sizeof(int)));
-    hip_check(hipHostMalloc((void **)&host_sc, (size_t)n * SC_COUNT * sizeof(double)), "hipHostMalloc");
+    host_sc = host_doubles((size_t)n * SC_COUNT);
     use_graph = o.use_graph != 0;
     act_.assign(n, 0);
     it_.assign(n, 0);
@@ -567,6 +566,7 @@ void BatchKMG::build_tables(TableSet &ts, const std::vector<int> &which) {
         TableSet *const saved = T;
         T = &ts;
         hipGraph_t g = nullptr;
+        const CaptureLock alone;
         hip_check(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "capture");
         try {
             body();
@@ -680,7 +680,7 @@ void BatchKMG::release(TableSet &ts) {
 void BatchKMG::free_buffers(TableSet &ts) {
     release(ts);
     if (ts.dev) dev_free(ts.dev);
-    if (ts.host) (void)hipHostFree(ts.host);
+    host_free(ts.host);
     ts.dev = nullptr;
     ts.host = nullptr;
     ts.dcap = ts.hcap = 0;
@@ -695,7 +695,7 @@ BatchKMG::~BatchKMG() {
     if (mask) dev_free(mask);
     if (arena) dev_free(arena);
     if (scal) dev_free(scal);
-    if (host_sc) (void)hipHostFree(host_sc);
+    host_free(host_sc);
 }
 
 void BatchKMG::zebra(int d, int set, int sel, int k) {

@@ -1496,7 +1496,10 @@ int mgp_server_result(mgp_server *v, long long ticket, double *phi, int *iters, 
 }
 
 int mgp_device_synchronize(void) {
-    return guarded([&] { hip_check(hipDeviceSynchronize(), "hipDeviceSynchronize"); });
+    return guarded([&] {
+        const NoCapture guard;
+        hip_check(hipDeviceSynchronize(), "hipDeviceSynchronize");
+    });
 }
 
 int mgp_vcycle(int kind, const mgp_geo *geo, const mgp_bc *bc, int homog, double tol, int maxiters, int maxdepth,

@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 
 #include <memory>
+#include <mutex>
+#include <shared_mutex>
 #include <string>
 #include <utility>
 #include <vector>
@@ -23,10 +25,28 @@ struct Failure {
 
 void hip_check(hipError_t e, const char *what);
 
+// While one thread captures a stream the runtime refuses other threads' fills
+// of new memory, device-wide waits and queries of events on that stream, and
+// such a call makes the capture fail.  Distinct solvers may be used from
+// distinct threads, so a capture holds this lock alone (CaptureLock), and the
+// library's allocations, staged host copies and device-wide waits share it
+// (NoCapture).  Launches and waits on a thread's own stream need neither.
+std::shared_mutex &capture_mutex();
+struct CaptureLock {
+    std::unique_lock<std::shared_mutex> lock{capture_mutex()};
+};
+struct NoCapture {
+    std::shared_lock<std::shared_mutex> lock{capture_mutex()};
+};
+
 // Zero-filled device allocation of `bytes` (throws MGP_ERR_NOMEM); dev_free
 // releases it.
 void *dev_alloc_zero(size_t bytes);
 void dev_free(void *p);
+// Pinned host memory (null: none to be had).
+void *host_alloc(size_t bytes);
+double *host_doubles(size_t n);  // throws where there is none
+void host_free(void *p);
 
 // One zero-filled device allocation that several arrays share; freed with the
 // last of them.

@@ -31,10 +31,16 @@ void hip_check(hipError_t e, const char *what) {
     }
 }
 
+std::shared_mutex &capture_mutex() {
+    static std::shared_mutex m;
+    return m;
+}
+
 // --------------------------------------------------------------------------
 // Device buffers
 // --------------------------------------------------------------------------
 void *dev_alloc_zero(size_t bytes) {
+    const NoCapture guard;
     void *p = nullptr;
     if (hipMalloc(&p, bytes) != hipSuccess) {
         g_last_error = "hipMalloc failed";
@@ -49,7 +55,32 @@ void *dev_alloc_zero(size_t bytes) {
     }
     return p;
 }
-void dev_free(void *p) { (void)hipFree(p); }
+void dev_free(void *p) {
+    const NoCapture guard;
+    (void)hipFree(p);
+}
+void *host_alloc(size_t bytes) {
+    const NoCapture guard;
+    void *p = nullptr;
+    if (hipHostMalloc(&p, bytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return p;
+}
+double *host_doubles(size_t n) {
+    double *p = static_cast<double *>(host_alloc(n * sizeof(double)));
+    if (!p) {
+        g_last_error = "hipHostMalloc failed";
+        throw Failure(MGP_ERR_HIP);
+    }
+    return p;
+}
+void host_free(void *p) {
+    if (!p) return;
+    const NoCapture guard;
+    (void)hipHostFree(p);
+}
 
 static thread_local std::shared_ptr<DevBlock> t_block;
 
@@ -162,6 +193,7 @@ void *stage_buffer(Staging &st, size_t bytes, hipStream_t s) {
 }  // namespace
 
 void upload_block(hipStream_t s, double *dev, const Grid &g, const double *host, int i0, int j0, int w, int h) {
+    const NoCapture guard;
     const size_t row = (size_t)w * sizeof(double), bytes = row * (size_t)h;
     double *d = dev + ix(g.pitch, i0, j0);
     const size_t dpitch = (size_t)g.pitch * sizeof(double);
@@ -197,6 +229,7 @@ void upload_block(hipStream_t s, double *dev, const Grid &g, const double *host,
     }
 }
 void download_block(hipStream_t s, double *host, const double *dev, const Grid &g, int i0, int j0, int w, int h) {
+    const NoCapture guard;
     const size_t row = (size_t)w * sizeof(double), bytes = row * (size_t)h;
     const double *d = dev + ix(g.pitch, i0, j0);
     const size_t dpitch = (size_t)g.pitch * sizeof(double);
@@ -334,7 +367,7 @@ double Workspace::reduce(hipStream_t s, const double *a, const double *b, const 
                          const Grid &g, int kind, int p) {
     const size_t need = (size_t)reduce_blocks(g) + 8;
     if (partial.n < need) partial.alloc(need);
-    if (!host_scalar) hip_check(hipHostMalloc((void **)&host_scalar, 8 * sizeof(double)), "hipHostMalloc");
+    if (!host_scalar) host_scalar = host_doubles(8);
     // result in partial.p[0], per-block partial sums from partial.p[8] on
     launch_reduce(s, partial.p, partial.p + 8, a, b, J, vol, g, kind, p);
     hip_check(hipMemcpyAsync(host_scalar, partial.p, sizeof(double), hipMemcpyDeviceToHost, s), "scalar");
@@ -342,7 +375,7 @@ double Workspace::reduce(hipStream_t s, const double *a, const double *b, const 
     return host_scalar[0];
 }
 Workspace::~Workspace() {
-    if (host_scalar) (void)hipHostFree(host_scalar);
+    host_free(host_scalar);
 }
 
 double pnorm2(Workspace &W, hipStream_t s, const double *a, const Grid &g) {

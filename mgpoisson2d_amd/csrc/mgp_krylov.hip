@@ -99,8 +99,8 @@ struct KrylovMG::Impl {
     hipGraphExec_t graph = nullptr;
     ~Impl() {
         if (graph) (void)hipGraphExecDestroy(graph);
-        if (host) (void)hipHostFree(host);
-        if (ghost) (void)hipHostFree(ghost);
+        host_free(host);
+        host_free(ghost);
     }
 };
 
@@ -135,7 +135,7 @@ void KrylovMG::ensure_fgmres(const Grid &g) {
     K.gh.alloc((size_t)3 * (m + 2));
     K.gpart.alloc((size_t)mdot_blocks(g) * (m + 1));
     K.gy.alloc((size_t)m);
-    hip_check(hipHostMalloc((void **)&K.ghost, (size_t)(4 * m + 6) * sizeof(double)), "hipHostMalloc");
+    K.ghost = host_doubles((size_t)(4 * m + 6));
 }
 
 // AUTO: x-lines where the cycle's element type solves the rows whole, else
@@ -325,7 +325,7 @@ void KrylovMG::build(hipStream_t s, const DevGeo &top, const Bc &user_bc, const 
     impl->scal.alloc(SC_COUNT);
     impl->partial.alloc(2 * (size_t)reduce_blocks(top.g) + 8);  // two products' partials, the blocks' count
     if (impl->fgmres) ensure_fgmres(top.g);  // past the arrays that bytes() counts
-    hip_check(hipHostMalloc((void **)&impl->host, SC_COUNT * sizeof(double)), "hipHostMalloc");
+    impl->host = host_doubles(SC_COUNT);
     impl->use_graph = o.use_graph != 0;
     built = true;
 }
@@ -645,6 +645,7 @@ int KrylovMG::solve(Workspace &W, hipStream_t s, const DevGeo &top, const Bc &us
     if (K.fgmres) return solve_fgmres(s, top, user_bc, phi, tol, maxiters, zerophi, relres, iters, true_residual);
     if (K.use_graph && !K.graph) {
         hipGraph_t graph = nullptr;
+        const CaptureLock alone;
         hip_check(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "capture");
         try {
             body();
